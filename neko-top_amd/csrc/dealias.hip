@@ -17,19 +17,23 @@
 // d_b f, w3 the GL tensor weights and c_b[a] the GL metric: the GLL cofactors
 // interpolated to GL, as init_dealias builds coef_GL (:155-163).
 //
-// One workgroup per element does everything on chip: the GLL fields are
-// staged in LDS, interpolated to GL by three tensor passes, combined point
-// by point in registers (PPT points per thread), and mapped back by three
-// transposed passes straight into f.  The reference's device branch makes
-// ~20 round trips through n_GL-sized HBM arrays per call; here HBM sees the
-// GLL inputs, the GL metric and f once.  The work is FP64 tensor
-// contractions of length lx and lxd, so the kernel is bounded by FP64 issue,
-// not HBM (about 1.6 MFLOP per element for the adjoint at lx = 8).
+// One workgroup per element does everything on chip: the GLL rows are read
+// straight into registers, interpolated to GL by three in-place tensor
+// passes, combined point by point, and mapped back by three transposed
+// passes straight into f.  The reference's device branch makes ~20 round
+// trips through n_GL-sized HBM arrays per call; here HBM sees the GLL inputs,
+// the GL metric and f once (174 KB per element for the adjoint at lx = 8,
+// 0.8 ms at 32^3; its 1.5 MFLOP take 0.6 ms at the FP64 rate).
+//
+// Measured at 32^3 p=7, before (two LDS reads per FMA) and now (one line per
+// thread, see dealias_k): forward 4.03 -> 1.24 ms, linearised 7.24 -> 2.24,
+// adjoint 6.98 -> 1.76; 13x11x9 p=5 forward 47.8 -> 23.2 us.
 #include <cmath>
 #include <vector>
 
 #include "internal.h"
 #include "nekoamd.h"
+#include "uniform.h"
 
 namespace nekoamd {
 namespace {
@@ -45,7 +49,8 @@ struct DealiasState {
   int lx = 0, lxd = 0, nelv = 0;
   int64_t n = 0, ngl = 0;
   double* cof = nullptr;   // [9][ngl], row m = 3b + a holds c_b[a]
-  double* mats = nullptr;  // J [lxd*lx] | Dg [lxd*lxd] | wg [lxd]
+  // J [lxd*lx] | Dg [lxd*lxd] | wg [lxd] | J^T [lx*lxd] | Dg^T [lxd*lxd]
+  double* mats = nullptr;
 };
 
 // LDS of one element: the 1-D matrices, the two interpolation temporaries
@@ -106,229 +111,422 @@ __device__ __forceinline__ void interp_up(DlShared<LX, LXD, NB>& sh,
   __syncthreads();
 }
 
-// Stage the element's GLL values of src and interpolate them to dst.
-template <int LX, int LXD, int NB>
-__device__ __forceinline__ void load_up(DlShared<LX, LXD, NB>& sh,
-                                        const double* __restrict__ src,
-                                        int64_t eb, double* dst) {
-  constexpr int NT = dl_threads<LXD>();
-  for (int p = threadIdx.x; p < LX * LX * LX; p += NT)
-    sh.t2[p] = __builtin_nontemporal_load(src + eb + p);
-  __syncthreads();
-  interp_up(sh, dst);
-}
+// ---- the operators -------------------------------------------------------
 
-// f[eb + .] = beta f - (J x J x J)^T src, src a GL field in LDS.  The caller
-// synchronised after writing src; returns synchronised.
-template <int LX, int LXD, int NB>
-__device__ __forceinline__ void down_store(DlShared<LX, LXD, NB>& sh,
-                                           const double* src,
-                                           double* __restrict__ f, int64_t eb,
-                                           double beta) {
-  constexpr int NT = dl_threads<LXD>();
-  for (int p = threadIdx.x; p < LXD * LXD * LX; p += NT) {
-    const int qr = p % (LXD * LXD), k = p / (LXD * LXD);
-    double s = 0.0;
-#pragma unroll
-    for (int l = 0; l < LXD; ++l)
-      s += sh.J[l * LX + k] * src[qr + LXD * LXD * l];
-    sh.t2[p] = s;
-  }
-  __syncthreads();
-  for (int p = threadIdx.x; p < LXD * LX * LX; p += NT) {
-    const int q = p % LXD, j = (p / LXD) % LX, k = p / (LXD * LX);
-    double s = 0.0;
-#pragma unroll
-    for (int l = 0; l < LXD; ++l)
-      s += sh.J[l * LX + j] * sh.t2[q + LXD * (l + LXD * k)];
-    sh.t1[p] = s;
-  }
-  __syncthreads();
-  for (int p = threadIdx.x; p < LX * LX * LX; p += NT) {
-    const int i = p % LX, jk = p / LX;
-    double s = 0.0;
-#pragma unroll
-    for (int l = 0; l < LXD; ++l) s += sh.J[l * LX + i] * sh.t1[l + LXD * jk];
-    const int64_t g = eb + p;
-    f[g] = (beta == 0.0 ? 0.0 : beta * f[g]) - s;
-  }
-  __syncthreads();
-}
+// LDS layout of a GL-sized field: row stride RS and plane stride PS in
+// doubles.  An even lxd gets one double of padding per row, so that the 64
+// lanes of a wave that read along r (stride RS) fall on distinct banks (at
+// lxd = 12 a stride of 12 doubles would use a quarter of them).
+template <int LX, int LXD>
+struct Dl {
+  static constexpr int NL = LXD * LXD;        // lines of one direction
+  static constexpr int NO = 3 * NL;           // working threads
+  static constexpr int NT = (NO + 63) / 64 * 64;
+  static constexpr int PPT = LXD / 3;         // points per thread
+  static constexpr int NP = LX * LX * LX, NPG = NL * LXD;
+  static constexpr int RS = LXD % 2 ? LXD : LXD + 1;
+  static constexpr int PS = RS * LXD;
+  static constexpr int BUF = PS * LXD;
+  static_assert(LXD == 3 * LX / 2 && LXD % 3 == 0, "points per thread");
+  static_assert(6 * LX * LX <= NT, "one thread per GLL row of six fields");
+};
 
-// r/s/t derivatives of the GL field f at (i, j, k).
-template <int LXD>
-__device__ __forceinline__ void gl_grad(const double* Dg, const double* f,
-                                        int i, int j, int k, double& r,
-                                        double& s, double& t) {
-  constexpr int NS = LXD * LXD;
-  r = 0.0;
-  s = 0.0;
-  t = 0.0;
-  // unrolled by 2 only: full unrolling lets the scheduler hoist the LDS
-  // reads of all points at once and spill
-#pragma unroll 2
-  for (int m = 0; m < LXD; ++m) {
-    r += Dg[i * LXD + m] * f[k * NS + j * LXD + m];
-    s += Dg[j * LXD + m] * f[k * NS + m * LXD + i];
-    t += Dg[k * LXD + m] * f[m * NS + j * LXD + i];
+// Offsets of the 1-D operators in `mats`.
+template <int LX, int LXD>
+struct DlMats {
+  static constexpr int J = 0, Dg = LXD * LX, w = Dg + LXD * LXD, JT = w + LXD,
+                       DgT = JT + LX * LXD, size = DgT + LXD * LXD;
+};
+
+// out[q] = sum_l M[q NI + l] in[l], l in order.  M is one of the 1-D
+// operators, the same for every lane, so its rows come by scalar loads and
+// enter the FMAs as scalar operands.  A row is requested once the first
+// product of the row before it is formed: two rows are in flight at most.
+template <int NI, int NQ>
+__device__ __forceinline__ void dl_apply(const double* __restrict__ M,
+                                         const double (&in)[NI],
+                                         double (&out)[NQ]) {
+  double row[NI], next[NI];
+  {
+    const auto m = uniform_row(M, in[0]);
+#pragma unroll
+    for (int l = 0; l < NI; ++l) row[l] = m[l];
+  }
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    double s = row[0] * in[0];
+    if (q + 1 < NQ) {
+      const auto m = uniform_row(M + (q + 1) * NI, s);
+#pragma unroll
+      for (int l = 0; l < NI; ++l) next[l] = m[l];
+    }
+#pragma unroll
+    for (int l = 1; l < NI; ++l) s += row[l] * in[l];
+    out[q] = s;
+    if (q + 1 < NQ) {
+#pragma unroll
+      for (int l = 0; l < NI; ++l) row[l] = next[l];
+    }
   }
 }
 
-template <int MODE>
-constexpr int dl_nbuf() {
-  return MODE == kFwd ? 3 : MODE == kLin ? 6 : 4;
+// One line of a tensor pass in place: NI values at p[l str] become NQ values
+// at p[q str].
+template <int NI, int NQ>
+__device__ __forceinline__ void dl_line(const double* __restrict__ M, double* p,
+                                        int str) {
+  double in[NI], out[NQ];
+#pragma unroll
+  for (int l = 0; l < NI; ++l) in[l] = p[l * str];
+  dl_apply<NI, NQ>(M, in, out);
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) p[q * str] = out[q];
 }
+
+// Line t of the 3 NL lines of a GL field (NL along r, then s, then t):
+// its first value's offset and its stride.
+template <int LX, int LXD>
+__device__ __forceinline__ void dl_dir_line(int t, int& base, int& str) {
+  using S = Dl<LX, LXD>;
+  const int b = t / S::NL, l = t % S::NL, lo = l % LXD, hi = l / LXD;
+  base = b == 0 ? S::RS * lo + S::PS * hi : b == 1 ? lo + S::PS * hi : lo + S::RS * hi;
+  str = b == 0 ? 1 : b == 1 ? S::RS : S::PS;
+}
+
+// Three fields (J x J x J)-interpolated into bf: thread t in [t0, t0 + 3 lx^2)
+// holds GLL row t - t0 in g.  Returns synchronised.
+template <int LX, int LXD>
+__device__ __forceinline__ void dl_up(double* bf,
+                                      const double* __restrict__ mats,
+                                      const double (&g)[LX], int t0) {
+  using S = Dl<LX, LXD>;
+  const double* J = mats + DlMats<LX, LXD>::J;
+  const int t = threadIdx.x, tr = t - t0;
+  if (tr >= 0 && tr < 3 * LX * LX) {
+    const int f = tr / (LX * LX), l = tr % (LX * LX);
+    double* p = bf + f * S::BUF + S::RS * (l % LX) + S::PS * (l / LX);
+    double out[LXD];
+    dl_apply<LX, LXD>(J, g, out);
+#pragma unroll
+    for (int q = 0; q < LXD; ++q) p[q] = out[q];
+  }
+  __syncthreads();
+  if (t < 3 * LXD * LX) {
+    const int f = t / (LXD * LX), l = t % (LXD * LX);
+    dl_line<LX, LXD>(J, bf + f * S::BUF + l % LXD + S::PS * (l / LXD), S::RS);
+  }
+  __syncthreads();
+  if (t < S::NO) {
+    const int f = t / S::NL, l = t % S::NL;
+    dl_line<LX, LXD>(J, bf + f * S::BUF + l % LXD + S::RS * (l / LXD), S::PS);
+  }
+  __syncthreads();
+}
+
+template <int LX>
+__device__ __forceinline__ void dl_row(double (&g)[LX],
+                                       const double* __restrict__ a0,
+                                       const double* __restrict__ a1,
+                                       const double* __restrict__ a2,
+                                       int64_t eb, int r) {
+  const int f = r / (LX * LX);
+  const double* a = (f == 0 ? a0 : f == 1 ? a1 : a2) + eb + (int64_t)LX * (r % (LX * LX));
+#pragma unroll
+  for (int l = 0; l < LX; ++l) g[l] = a[l];
+}
+
+constexpr int kDlFields = 5;  // GL-sized LDS fields: b[3] and x[2]
 
 // a*: forward u,v,w; linearised u'; adjoint the adjoint velocity.
 // b*: the base flow U (linearised and adjoint).
+//
+// Every tensor pass is a set of lines: a thread reads the line's values once
+// from LDS, forms all of the line's outputs with the 1-D operator in scalar
+// registers and writes them back, so a pass costs one LDS read and one write
+// per value (the first form of this kernel read two LDS values per FMA and
+// was bound by them).  The three directions of a gradient are 3 lxd^2 lines
+// of one pass (432 threads at lxd = 12); between passes the same threads own
+// lxd / 3 points each, whose pointwise factors stay in registers:
+//
+//   forward  O_c = sum_b C_b d_b t_c,       C_b = w3 sum_a c_b[a] t_a
+//   linear   O_c = sum_b C'_b d_b U_c + C_b d_b u'_c
+//   adjoint  O_c = w3 sum_b c_b[c] E_b + sum_b D_b^T (a_c C_b),
+//            E_b = sum_d a_d d_b U_d,       C_b = w3 sum_d c_b[d] U_d
+//
+// (contravariant components: the metric is read once per point, and
+// opgrad_c(U_d) is never formed).  Five GL fields of LDS (75 KB at lxd = 12)
+// leave room for two elements per CU; interpolation and map-back run in
+// place in them.  The linearised operator needs both sets' C_b and is held
+// to 128 registers so that two workgroups fit (2.24 ms with 16 spilled
+// registers against 2.82 ms without the cap at 32^3 p=7).
 template <int LX, int LXD, int MODE>
-__global__ void __launch_bounds__(dl_threads<LXD>())
+__global__ void __launch_bounds__((Dl<LX, LXD>::NT), (MODE == kLin ? 4 : 1))
     dealias_k(double* __restrict__ fx, double* __restrict__ fy,
               double* __restrict__ fz, const double* __restrict__ a0,
               const double* __restrict__ a1, const double* __restrict__ a2,
               const double* __restrict__ b0, const double* __restrict__ b1,
               const double* __restrict__ b2, const double* __restrict__ cof,
               const double* __restrict__ mats, int64_t ngl, double beta) {
-  constexpr int NT = dl_threads<LXD>();
-  constexpr int NP = LX * LX * LX, NPG = LXD * LXD * LXD;
-  constexpr int PPT = (NPG + NT - 1) / NT;
-  constexpr int NB = dl_nbuf<MODE>();
-  __shared__ DlShared<LX, LXD, NB> sh;
-  const int e = blockIdx.x;
-  const int64_t eb = (int64_t)e * NP, gb = (int64_t)e * NPG;
-  double* const f[3] = {fx, fy, fz};
-  load_mats(sh, mats);
+  using S = Dl<LX, LXD>;
+  using M = DlMats<LX, LXD>;
+  constexpr int PPT = S::PPT, NO = S::NO, R3 = 3 * LX * LX;
+  __shared__ double sh[kDlFields][S::BUF];
+  double (*const B)[S::BUF] = sh;
+  double (*const X)[S::BUF] = sh + 3;
+  const int t = threadIdx.x;
+  const bool on = t < NO;
+  const int64_t eb = (int64_t)blockIdx.x * S::NP, gb = (int64_t)blockIdx.x * S::NPG;
 
+  // GLL rows of the fields, all requested before the first pass
+  double g[LX];
   if constexpr (MODE == kFwd) {
-    load_up(sh, a0, eb, sh.buf[0]);
-    load_up(sh, a1, eb, sh.buf[1]);
-    load_up(sh, a2, eb, sh.buf[2]);
+    if (t < R3) dl_row<LX>(g, a0, a1, a2, eb, t);
   } else {
-    load_up(sh, b0, eb, sh.buf[0]);
-    load_up(sh, b1, eb, sh.buf[1]);
-    load_up(sh, b2, eb, sh.buf[2]);
-  }
-  if constexpr (MODE == kLin) {
-    load_up(sh, a0, eb, sh.buf[3]);
-    load_up(sh, a1, eb, sh.buf[4]);
-    load_up(sh, a2, eb, sh.buf[5]);
-  }
-  double A[3][PPT];  // adjoint: the adjoint velocity at the thread's points
-  if constexpr (MODE == kAdj) {
-    const double* src[3] = {a0, a1, a2};
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      load_up(sh, src[d], eb, sh.buf[3]);
-#pragma unroll
-      for (int q = 0; q < PPT; ++q) {
-        const int p = threadIdx.x + q * NT;
-        A[d][q] = p < NPG ? sh.buf[3][p] : 0.0;
-      }
-    }
+    if (t < R3)
+      dl_row<LX>(g, a0, a1, a2, eb, t);
+    else if (t < 2 * R3)
+      dl_row<LX>(g, b0, b1, b2, eb, t - R3);
   }
 
-  double O[3][PPT];              // the per-component GL integrand
-  double UC[3][PPT], W3[PPT];    // adjoint: U . c_b and w3
+  // the thread's points p = t + q NO: (i, j) the same for all of them,
+  // k = t / NL + 3 q
+  const int ij = t % S::NL, i = ij % LXD, j = ij / LXD, k0 = t / S::NL;
+  const int at0 = i + S::RS * j + S::PS * k0;  // + 3 PS q
+  const double* w = mats + M::w;
+  const double wij = on ? w[i] * w[j] : 0.0;
+  int lb = 0, ls = 0;
+  if (on) dl_dir_line<LX, LXD>(t, lb, ls);
+  const int db = on ? t / S::NL : 0;  // the line's direction
+
+  double O[3][PPT];
 #pragma unroll
-  for (int q = 0; q < PPT; ++q) {
-    const int p = threadIdx.x + q * NT;
-    if (p >= NPG) {
+  for (int c = 0; c < 3; ++c)
 #pragma unroll
-      for (int c = 0; c < 3; ++c) O[c][q] = UC[c][q] = 0.0;
-      W3[q] = 0.0;
-      continue;
-    }
-    const int i = p % LXD, j = (p / LXD) % LXD, k = p / (LXD * LXD);
-    const double w3 = sh.w[i] * sh.w[j] * sh.w[k];
-    double c[9];
+    for (int q = 0; q < PPT; ++q) O[c][q] = 0.0;
+
+  // C_b at point q from three fields' values there
+  auto metric = [&](int q, double (&c9)[9]) {
+    const int64_t p = gb + t + q * NO;
 #pragma unroll
     for (int m = 0; m < 9; ++m)
-      c[m] = __builtin_nontemporal_load(cof + m * ngl + gb + p);
-    // opgrad of the GL field g at this point
-    auto opg = [&](const double* g, double o[3]) {
-      double r, s, t;
-      gl_grad<LXD>(sh.Dg, g, i, j, k, r, s, t);
+      c9[m] = __builtin_nontemporal_load(cof + m * ngl + p);
+  };
+  // O_c += sum_b C_b d_b (field c of B); B is consumed
+  auto convect = [&](const double (&Cb)[3][PPT]) {
 #pragma unroll
-      for (int a = 0; a < 3; ++a)
-        o[a] = w3 * (c[a] * r + c[3 + a] * s + c[6 + a] * t);
-    };
-    if constexpr (MODE == kFwd) {
-      const double tv[3] = {sh.buf[0][p], sh.buf[1][p], sh.buf[2][p]};
+    for (int c = 0; c < 3; ++c) {
+      double in[LXD], out[LXD];
+      if (on) {
 #pragma unroll
-      for (int cc = 0; cc < 3; ++cc) {
-        double o[3];
-        opg(sh.buf[cc], o);
-        O[cc][q] = o[0] * tv[0] + o[1] * tv[1] + o[2] * tv[2];
+        for (int l = 0; l < LXD; ++l) in[l] = B[c][lb + l * ls];
+        dl_apply<LXD, LXD>(mats + M::Dg, in, out);
       }
-    } else if constexpr (MODE == kLin) {
-      const double ub[3] = {sh.buf[0][p], sh.buf[1][p], sh.buf[2][p]};
-      const double up[3] = {sh.buf[3][p], sh.buf[4][p], sh.buf[5][p]};
+      __syncthreads();  // rows of field c and the sums of field c - 1 read
+      if (on) {
+        double* o = db == 0 ? X[0] : db == 1 ? X[1] : B[c];
 #pragma unroll
-      for (int cc = 0; cc < 3; ++cc) {
-        double o[3], o2[3];
-        opg(sh.buf[cc], o);
-        opg(sh.buf[3 + cc], o2);
-        O[cc][q] = (o[0] * up[0] + o[1] * up[1] + o[2] * up[2]) +
-                   (o2[0] * ub[0] + o2[1] * ub[1] + o2[2] * ub[2]);
+        for (int l = 0; l < LXD; ++l) o[lb + l * ls] = out[l];
       }
+      __syncthreads();
+      if (on) {
+#pragma unroll
+        for (int q = 0; q < PPT; ++q) {
+          const int at = at0 + 3 * S::PS * q;
+          O[c][q] += Cb[0][q] * X[0][at] + Cb[1][q] * X[1][at] + Cb[2][q] * B[c][at];
+        }
+      }
+    }
+  };
+
+  dl_up<LX, LXD>(sh[0], mats, g, 0);
+  if constexpr (MODE == kFwd) {
+    double C[3][PPT];
+    if (on) {
+#pragma unroll
+      for (int q = 0; q < PPT; ++q) {
+        const int at = at0 + 3 * S::PS * q;
+        const double w3 = wij * w[k0 + 3 * q];
+        double c9[9];
+        metric(q, c9);
+#pragma unroll
+        for (int b = 0; b < 3; ++b)
+          C[b][q] = w3 * (c9[3 * b] * B[0][at] + c9[3 * b + 1] * B[1][at] +
+                          c9[3 * b + 2] * B[2][at]);
+      }
+    }
+    convect(C);
+  } else {
+    // the first set's values at the thread's points: u' or the adjoint a
+    double A[3][PPT];
+    if (on) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int q = 0; q < PPT; ++q) A[d][q] = B[d][at0 + 3 * S::PS * q];
+    }
+    __syncthreads();
+    dl_up<LX, LXD>(sh[0], mats, g, R3);
+    if constexpr (MODE == kLin) {
+      double C[3][PPT], Cp[3][PPT];
+      if (on) {
+#pragma unroll
+        for (int q = 0; q < PPT; ++q) {
+          const int at = at0 + 3 * S::PS * q;
+          const double w3 = wij * w[k0 + 3 * q];
+          double c9[9];
+          metric(q, c9);
+#pragma unroll
+          for (int b = 0; b < 3; ++b) {
+            C[b][q] = w3 * (c9[3 * b] * B[0][at] + c9[3 * b + 1] * B[1][at] +
+                            c9[3 * b + 2] * B[2][at]);
+            Cp[b][q] = w3 * (c9[3 * b] * A[0][q] + c9[3 * b + 1] * A[1][q] +
+                             c9[3 * b + 2] * A[2][q]);
+          }
+        }
+      }
+      convect(Cp);
+      // u' again for its own gradients
+      if (t < R3) dl_row<LX>(g, a0, a1, a2, eb, t);
+      __syncthreads();
+      dl_up<LX, LXD>(sh[0], mats, g, 0);
+      convect(C);
     } else {
-      const double ub[3] = {sh.buf[0][p], sh.buf[1][p], sh.buf[2][p]};
-      double o[3][3];  // o[d][c] = opgrad_c(U_d)
+      // E_b along the thread's line, the adjoint velocity through X
+      double E[LXD];
 #pragma unroll
-      for (int d = 0; d < 3; ++d) opg(sh.buf[d], o[d]);
+      for (int l = 0; l < LXD; ++l) E[l] = 0.0;
+      if (on) {
 #pragma unroll
-      for (int cc = 0; cc < 3; ++cc)
-        O[cc][q] = A[0][q] * o[0][cc] + A[1][q] * o[1][cc] + A[2][q] * o[2][cc];
+        for (int q = 0; q < PPT; ++q) {
+          X[0][at0 + 3 * S::PS * q] = A[0][q];
+          X[1][at0 + 3 * S::PS * q] = A[1][q];
+        }
+      }
+      __syncthreads();
 #pragma unroll
-      for (int b = 0; b < 3; ++b)
-        UC[b][q] = ub[0] * c[3 * b] + ub[1] * c[3 * b + 1] + ub[2] * c[3 * b + 2];
-      W3[q] = w3;
+      for (int d = 0; d < 3; ++d) {
+        if (d == 2) {
+          __syncthreads();
+          if (on) {
+#pragma unroll
+            for (int q = 0; q < PPT; ++q) X[0][at0 + 3 * S::PS * q] = A[2][q];
+          }
+          __syncthreads();
+        }
+        if (on) {
+          double in[LXD], out[LXD];
+#pragma unroll
+          for (int l = 0; l < LXD; ++l) in[l] = B[d][lb + l * ls];
+          dl_apply<LXD, LXD>(mats + M::Dg, in, out);
+          const double* a = X[d == 1 ? 1 : 0] + lb;
+#pragma unroll
+          for (int l = 0; l < LXD; ++l) E[l] += a[l * ls] * out[l];
+        }
+      }
+      __syncthreads();
+      // U at the thread's points, E_b in its place
+      double U[3][PPT];
+      if (on) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+          for (int q = 0; q < PPT; ++q) U[d][q] = B[d][at0 + 3 * S::PS * q];
+      }
+      __syncthreads();
+      if (on) {
+        double* o = B[db] + lb;
+#pragma unroll
+        for (int l = 0; l < LXD; ++l) o[l * ls] = E[l];
+      }
+      __syncthreads();
+      if (on) {
+#pragma unroll
+        for (int q = 0; q < PPT; ++q) {
+          const int at = at0 + 3 * S::PS * q;
+          const double w3 = wij * w[k0 + 3 * q];
+          double c9[9];
+          metric(q, c9);
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+            O[c][q] = w3 * (c9[c] * B[0][at] + c9[3 + c] * B[1][at] + c9[6 + c] * B[2][at]);
+#pragma unroll
+          for (int b = 0; b < 3; ++b)
+            B[b][at] = w3 * (c9[3 * b] * U[0][q] + c9[3 * b + 1] * U[1][q] +
+                             c9[3 * b + 2] * U[2][q]);
+          X[0][at] = A[0][q];
+          X[1][at] = A[1][q];
+        }
+      }
+      __syncthreads();
+      // C_b along the thread's line; then the weak term of each component
+      double C[LXD];
+      if (on) {
+#pragma unroll
+        for (int l = 0; l < LXD; ++l) C[l] = B[db][lb + l * ls];
+      }
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        if (on) {
+          const double* a = X[c == 1 ? 1 : 0] + lb;
+          double in[LXD], out[LXD];
+#pragma unroll
+          for (int l = 0; l < LXD; ++l) in[l] = a[l * ls] * C[l];
+          dl_apply<LXD, LXD>(mats + M::DgT, in, out);
+          double* o = B[db] + lb;
+#pragma unroll
+          for (int l = 0; l < LXD; ++l) o[l * ls] = out[l];
+        }
+        __syncthreads();
+        if (on) {
+#pragma unroll
+          for (int q = 0; q < PPT; ++q) {
+            const int at = at0 + 3 * S::PS * q;
+            O[c][q] += B[0][at] + B[1][at] + B[2][at];
+            if (c == 0) X[0][at] = A[2][q];
+          }
+        }
+        __syncthreads();
+      }
     }
   }
-  __syncthreads();  // the GL input fields are consumed
 
+  // f = beta f - (J x J x J)^T O
+  __syncthreads();
+  if (on) {
 #pragma unroll
-  for (int cc = 0; cc < 3; ++cc) {
-    if constexpr (MODE == kAdj) {
-      // weak term: F_b = w3 a_c (U . c_b), then G = O_c + sum_b D_b^T F_b
+    for (int c = 0; c < 3; ++c)
 #pragma unroll
-      for (int q = 0; q < PPT; ++q) {
-        const int p = threadIdx.x + q * NT;
-        if (p < NPG) {
-          const double wa = W3[q] * A[cc][q];
-          sh.buf[0][p] = wa * UC[0][q];
-          sh.buf[1][p] = wa * UC[1][q];
-          sh.buf[2][p] = wa * UC[2][q];
-        }
-      }
-      __syncthreads();
+      for (int q = 0; q < PPT; ++q) B[c][at0 + 3 * S::PS * q] = O[c][q];
+  }
+  const int fc = t / (LX * LX), fl = t % (LX * LX);
+  double* f = (fc == 0 ? fx : fc == 1 ? fy : fz) + eb + (int64_t)LX * fl;
+  double old[LX];
 #pragma unroll
-      for (int q = 0; q < PPT; ++q) {
-        const int p = threadIdx.x + q * NT;
-        if (p < NPG) {
-          const int i = p % LXD, j = (p / LXD) % LXD, k = p / (LXD * LXD);
-          constexpr int NS = LXD * LXD;
-          double s = 0.0;
+  for (int l = 0; l < LX; ++l) old[l] = 0.0;
+  if (t < R3 && beta != 0.0) {
 #pragma unroll
-          for (int m = 0; m < LXD; ++m) {
-            s += sh.Dg[m * LXD + i] * sh.buf[0][k * NS + j * LXD + m];
-            s += sh.Dg[m * LXD + j] * sh.buf[1][k * NS + m * LXD + i];
-            s += sh.Dg[m * LXD + k] * sh.buf[2][m * NS + j * LXD + i];
-          }
-          sh.buf[3][p] = O[cc][q] + s;
-        }
-      }
-      __syncthreads();
-      down_store(sh, sh.buf[3], f[cc], eb, beta);
-    } else {
+    for (int l = 0; l < LX; ++l) old[l] = f[l];
+  }
+  __syncthreads();
+  const double* JT = mats + M::JT;
+  if (on) {
+    const int c = t / S::NL, l = t % S::NL;
+    dl_line<LXD, LX>(JT, B[c] + l % LXD + S::RS * (l / LXD), S::PS);
+  }
+  __syncthreads();
+  if (t < 3 * LXD * LX) {
+    const int c = t / (LXD * LX), l = t % (LXD * LX);
+    dl_line<LXD, LX>(JT, B[c] + l % LXD + S::PS * (l / LXD), S::RS);
+  }
+  __syncthreads();
+  if (t < R3) {
+    const double* p = B[fc] + S::RS * (fl % LX) + S::PS * (fl / LX);
+    double in[LXD], out[LX];
 #pragma unroll
-      for (int q = 0; q < PPT; ++q) {
-        const int p = threadIdx.x + q * NT;
-        if (p < NPG) sh.buf[0][p] = O[cc][q];
-      }
-      __syncthreads();
-      down_store(sh, sh.buf[0], f[cc], eb, beta);
-    }
+    for (int l = 0; l < LXD; ++l) in[l] = p[l];
+    dl_apply<LXD, LX>(JT, in, out);
+#pragma unroll
+    for (int l = 0; l < LX; ++l) f[l] = (beta == 0.0 ? 0.0 : beta * old[l]) - out[l];
   }
 }
 
@@ -426,7 +624,7 @@ int dealias_run(const DealiasState* s, int mode, double* fx, double* fy,
                 double* fz, const double* a0, const double* a1,
                 const double* a2, const double* b0, const double* b1,
                 const double* b2, double beta) {
-  const dim3 grid(s->nelv), block(dl_threads<LXD>());
+  const dim3 grid(s->nelv), block(Dl<LX, LXD>::NT);
   switch (mode) {
     case kFwd:
       hipLaunchKernelGGL((dealias_k<LX, LXD, kFwd>), grid, block, 0, stream(),
@@ -512,7 +710,7 @@ int nekoamd_dealias_create(void** st, const void* x, const void* y,
   }
   gauss_legendre(LD, zg, wg);
   // J[q*L + i] = l_i(zg_q); Dg[i*LD + j] = l'_j(zg_i) on the GL nodes
-  std::vector<double> mats(LD * L + LD * LD + LD);
+  std::vector<double> mats(2 * (LD * L + LD * LD) + LD);
   for (int q = 0; q < LD; ++q)
     for (int i = 0; i < L; ++i) {
       double v = 1.0;
@@ -535,6 +733,12 @@ int nekoamd_dealias_create(void** st, const void* x, const void* y,
     Dg[i * LD + i] = d;
   }
   for (int i = 0; i < LD; ++i) mats[LD * L + LD * LD + i] = wg[i];
+  double* JT = Dg + LD * LD + LD;
+  double* DgT = JT + L * LD;
+  for (int q = 0; q < LD; ++q)
+    for (int i = 0; i < L; ++i) JT[i * LD + q] = mats[q * L + i];
+  for (int i = 0; i < LD; ++i)
+    for (int q = 0; q < LD; ++q) DgT[i * LD + q] = Dg[q * LD + i];
   hipError_t e = hipMalloc(&s->mats, sizeof(double) * mats.size());
   if (e == hipSuccess && s->ngl > 0)
     e = hipMalloc(&s->cof, sizeof(double) * 9 * (size_t)s->ngl);

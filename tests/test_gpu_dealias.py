@@ -105,3 +105,39 @@ def test_device_duality(pair):
     scale = sum(np.abs(a[k]) @ np.abs(Lh[k]) for k in range(3))
     print(f"lx={c.lx}: duality {lhs:.14e} vs {rhs:.14e}")
     assert abs(lhs - rhs) < 1e-13 * scale
+
+
+@pytest.mark.parametrize("mode", ["forward", "linear", "adjoint"])
+def test_fields_at_odd_offsets(pair, mode):
+    """Fields that start 8 bytes past a 16-byte boundary, and a scaled
+    forcing (beta = -0.5): the aligned call's values bit for bit, and nothing
+    written outside f."""
+    import ctypes as C
+
+    from nekoamd import device as dev
+    from nekoamd._lib import check, lib, ptr, rd
+    g, c, d, o = pair
+    n = c.n
+    host = [np.concatenate([[np.nan], a, [np.nan]]) for a in _fields(c, 12, 9)]
+    off = [dev.DeviceArray.from_host(a) for a in host]
+    f, a, b = ([C.c_void_p(x.ptr + 8) for x in off[3 * k:3 * k + 3]] for k in range(3))
+    fa, aa, ba = ([g.field(x[1:n + 1]) for x in host[3 * k:3 * k + 3]] for k in range(3))
+    h = C.c_void_p(d.h)
+    L = lib()
+    for F, A, Bf in ((f, a, b), (list(map(ptr, fa)), list(map(ptr, aa)), list(map(ptr, ba)))):
+        if mode == "forward":
+            check(L.nekoamd_dealias_advection(h, *F, *A, rd(-0.5)), mode)
+        elif mode == "linear":
+            check(L.nekoamd_dealias_linear(h, *F, *A, *Bf), mode)
+        else:
+            check(L.nekoamd_dealias_adjoint(h, *F, *A, *Bf), mode)
+    if mode == "forward":
+        # beta f - t, t the term alone
+        t = oracle.dealias_advection(o, *(x[1:n + 1] for x in host[3:6]))
+        ref = [-0.5 * x[1:n + 1] + y for x, y in zip(host[:3], t)]
+        assert _err([x.get() for x in fa], ref) < 1e-12
+    for x, y, h0 in zip(off[:3], fa, host[:3]):
+        got = x.get()
+        assert np.isnan(got[0]) and np.isnan(got[-1])
+        assert np.array_equal(got[1:n + 1], y.get())
+        assert not np.array_equal(got[1:n + 1], h0[1:n + 1])
