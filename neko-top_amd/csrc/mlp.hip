@@ -14,11 +14,20 @@
 // The Galerkin scaling makes the guess safe: it never increases the A-norm
 // of the error, and gamma = 0 (no guess) when <q,Aq> <= 0.
 //
-// GEMMs: one 256-thread kernel, 128 x 128 x 32 tiles staged through LDS,
-// v_mfma_f32_32x32x16_bf16 (four waves, 64 x 64 each), FP32 accumulation.
-// Three operand layouts (NT forward, NN data gradient, TN weight gradient
-// with split-K) are converted to one K-contiguous LDS layout on load; the
-// bias, SiLU, SiLU' and BF16 rounding are fused into the epilogues.
+// GEMMs: 64 x 64 output tiles of a 256-thread workgroup, K in steps of 64
+// staged through two LDS buffers, v_mfma_f32_32x32x16_bf16 (four waves, one
+// 32 x 32 tile each), FP32 accumulation.  Operands that are contiguous along
+// the output dimension (both of the weight gradient's, the data gradient's
+// weights) are transposed in registers on their way to LDS.  Bias, SiLU,
+// SiLU', the loss and its gradient, the column sums of the bias gradients
+// and the BF16 rounding are in the epilogues; the three weight gradients
+// are one split-K launch.  A training gradient is seven launches and bound
+// by their latency (7 GFLOP at 4096 rows is 6 us of matrix peak): 80 us at
+// 4096 rows, 67 us at 256 and 177 us at 19200.  With 128 x 128 tiles
+// transposed into LDS value by value (two-byte stores, four-way and worse
+// bank conflicts), a launch per weight gradient, separate column-sum, loss
+// and unpadding passes and no loads in flight across a step it was 348, 231
+// and 652 us (23 launches).
 // BF16 is stored as uint16_t and rounded to nearest-even by bit arithmetic.
 #include <algorithm>
 #include <cmath>
@@ -36,7 +45,11 @@ constexpr int kNP = 512;    // GLL values per element (lx = 8)
 constexpr int kNIN = 518;   // inputs
 constexpr int kKIN = 544;   // inputs padded to the K tile
 constexpr int kHID = 256;
-constexpr int kBM = 128, kBN = 128, kBK = 32, kLdsK = kBK + 8;
+// GEMM tile; LDS rows of 72 halfwords (36 banks), so that the 16-byte
+// accesses of 8 consecutive lanes, in rows or in every other row, fall into
+// distinct banks.
+constexpr int kBT = 64, kBK = 64, kLdsK = kBK + 8;
+constexpr int kMaxSplit = 16;
 
 // padded parameter layout (FP32): W1[256][544] b1 W2[256][256] b2
 // W3[512][256] b3
@@ -70,153 +83,326 @@ __device__ __forceinline__ float dsilu(float z) {
   return s * (1.0f + z * (1.0f - s));
 }
 
-enum Layout { kNT = 0, kNN = 1, kTN = 2 };
-enum Epi { kFwdHidden = 0, kFwdOut = 1, kBwdData = 2, kWgrad = 3 };
+enum Epi { kFwdHidden, kFwdOut, kFwdLoss, kBwdData };
 
 struct EpiArgs {
-  const float* bias;  // FwdHidden / FwdOut
-  float* zf;          // FwdHidden: Z (may be null); BwdData: dZ fp32; Wgrad: partials
-  uint16_t* hb;       // FwdHidden: H; BwdData: dZ bf16
-  const float* z;     // BwdData: the forward pre-activation
+  const float* bias;  // forward
+  float* zf;          // FwdHidden: Z (may be null)
+  uint16_t* hb;       // FwdHidden: H; FwdLoss, BwdData: dZ
+  const float* z;     // BwdData: the forward pre-activation; FwdLoss: targets
   float* yf;          // FwdOut (float output)
   double* yd;         // FwdOut (double output, scaled by *yscale)
-  const double* yscale;
+  const double* yscale;  // FwdOut; FwdLoss: yscale[1] scales the targets
+                         // (null: unscaled)
+  float gscale;       // FwdLoss: 2 / (M 512)
+  float* colpart;     // FwdLoss, BwdData: [tile row][ldc] column sums of dZ
+  double* lpart;      // FwdLoss: one loss partial per workgroup
   int ldc;
 };
 
-// C[M,N] = sum_k opA[m,k] opB[n,k]:
-//   NT: A[m*lda+k], B[n*ldb+k];  NN: A[m*lda+k], B[k*ldb+n];
-//   TN: A[k*lda+m], B[k*ldb+n].
-// K (NT: also the contiguous dim), and the contiguous dims of NN / TN
-// operands, must be multiples of 8; other dims are guarded.  Split-K
-// (gridDim.z > 1, Wgrad only): block z covers k in [z*kz, (z+1)*kz).
-// BM x BN output tile per 256-thread workgroup, four waves in a 2 x 2
-// arrangement, each wave (BM/2) x (BN/2) as (BM/64) x (BN/64) MFMA tiles of
-// 32 x 32.  128 x 128 for the training GEMMs; 64 x 64 for the forward ones,
-// whose M = elements is tall and K <= 544 small: four times the workgroups
-// (8 waves per SIMD at 32^3) hide the global-load latency of each k-step
-// (inference at 32^3: 116 -> 77 us; prefetching the next k-tile into
-// registers on top of that measured no gain).
-template <int LAYOUT, int EPI, int BM = kBM, int BN = kBN>
-__global__ void __launch_bounds__(256)
-    gemm_bf16_k(int M, int N, int K, int kz, const uint16_t* __restrict__ A,
-                int lda, const uint16_t* __restrict__ B, int ldb, EpiArgs ep) {
-  static_assert(BM % 64 == 0 && BN % 64 == 0, "tile must be a multiple of 64");
-  constexpr int TI = BM / 64, TJ = BN / 64;
-  __shared__ __attribute__((aligned(16))) uint16_t As[BM * kLdsK];
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[BN * kLdsK];
+// One operand's 64 x 64 tile on its way to LDS: 16 BF16 values per thread.
+// KM false: the operand is P[row][ld] with k contiguous; a thread holds
+// two 8-value pieces of rows.  KM true: P[k][ld] with the output dimension
+// contiguous; a thread holds columns c0 + 2 (t % 32) and the next of the 8
+// rows of k group t / 32 (4-byte loads, 128 bytes of a row per half wave),
+// and the store turns them into two 8-value pieces along k.  Values past
+// `rows` or kend are zero; K ranges are multiples of 8.
+template <bool KM>
+struct Stage {
+  uint32_t v[8];
+  __device__ __forceinline__ void load(const uint16_t* __restrict__ P, int ld,
+                                       int c0, int rows, int k0, int kend) {
+    const int t = threadIdx.x;
+    if constexpr (KM) {
+      const int c = c0 + 2 * (t & 31), k = k0 + 8 * (t >> 5);
+      const bool in = c < rows && k < kend;
+      const uint16_t* q = P + (int64_t)k * ld + c;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        v[j] = in ? *(const uint32_t*)(q + (int64_t)j * ld) : 0u;
+    } else {
+#pragma unroll
+      for (int c2 = 0; c2 < 2; ++c2) {
+        const int c = t + c2 * 256, r = c0 + (c >> 3), k = k0 + (c & 7) * 8;
+        uint4 w = make_uint4(0, 0, 0, 0);
+        if (r < rows && k < kend) w = *(const uint4*)(P + (int64_t)r * ld + k);
+        v[4 * c2] = w.x;
+        v[4 * c2 + 1] = w.y;
+        v[4 * c2 + 2] = w.z;
+        v[4 * c2 + 3] = w.w;
+      }
+    }
+  }
+  __device__ __forceinline__ void store(uint16_t* lds) const {
+    const int t = threadIdx.x;
+    if constexpr (KM) {
+      uint32_t lo[4], hi[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        lo[j] = (v[2 * j] & 0xFFFFu) | (v[2 * j + 1] << 16);
+        hi[j] = (v[2 * j] >> 16) | (v[2 * j + 1] & 0xFFFF0000u);
+      }
+      uint16_t* d = lds + 2 * (t & 31) * kLdsK + 8 * (t >> 5);
+      *(uint4*)d = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+      *(uint4*)(d + kLdsK) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+    } else {
+#pragma unroll
+      for (int c2 = 0; c2 < 2; ++c2) {
+        const int c = t + c2 * 256;
+        *(uint4*)(lds + (c >> 3) * kLdsK + (c & 7) * 8) =
+            make_uint4(v[4 * c2], v[4 * c2 + 1], v[4 * c2 + 2], v[4 * c2 + 3]);
+      }
+    }
+  }
+};
+
+// acc = this wave's 32 x 32 part of sum_k A[m0+.][k] B[n0+.][k], k in
+// [kbeg, kend).  The next step's loads are in flight while a step is
+// multiplied, one barrier per step: the launches of a training batch have
+// one to four workgroups per CU, so nothing else hides the latency.
+constexpr int kTileLds = 4 * kBT * kLdsK;  // halfwords: two buffers of A and B
+template <bool AKM, bool BKM>
+__device__ __forceinline__ f32x16 tile_mma(const uint16_t* __restrict__ A,
+                                           int lda, int m0, int M,
+                                           const uint16_t* __restrict__ B,
+                                           int ldb, int n0, int N, int kbeg,
+                                           int kend, uint16_t* lds) {
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int wm = w >> 1, wn = w & 1;
-  const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-  const int kbeg = blockIdx.z * kz;
-  const int kend = min(K, kbeg + kz);
-
-  f32x16 acc[TI][TJ];
+  const int ra = ((w >> 1) * 32 + (lane & 31)) * kLdsK + (lane >> 5) * 8;
+  const int rb = ((w & 1) * 32 + (lane & 31)) * kLdsK + (lane >> 5) * 8;
+  f32x16 acc;
 #pragma unroll
-  for (int i = 0; i < TI; ++i)
-#pragma unroll
-    for (int j = 0; j < TJ; ++j)
-#pragma unroll
-      for (int a = 0; a < 16; ++a) acc[i][j][a] = 0.0f;
-
+  for (int a = 0; a < 16; ++a) acc[a] = 0.0f;
+  Stage<AKM> sa;
+  Stage<BKM> sb;
+  sa.load(A, lda, m0, M, kbeg, kend);
+  sb.load(B, ldb, n0, N, kbeg, kend);
+  int buf = 0;
   for (int k0 = kbeg; k0 < kend; k0 += kBK) {
-    // ---- stage A tile into As[m][k] ----
-#pragma unroll
-    for (int c2 = 0; c2 < BM / 64; ++c2) {
-      const int c = t + c2 * 256;
-      if (LAYOUT == kTN) {
-        const int kk = c / (BM / 8), mc = (c % (BM / 8)) * 8;
-        uint4 v = make_uint4(0, 0, 0, 0);
-        if (k0 + kk < kend && m0 + mc < M)
-          v = *(const uint4*)(A + (int64_t)(k0 + kk) * lda + m0 + mc);
-        const uint16_t* h = (const uint16_t*)&v;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) As[(mc + j) * kLdsK + kk] = h[j];
-      } else {
-        const int r = c >> 2, kc = (c & 3) * 8;
-        uint4 v = make_uint4(0, 0, 0, 0);
-        if (m0 + r < M && k0 + kc < kend)
-          v = *(const uint4*)(A + (int64_t)(m0 + r) * lda + k0 + kc);
-        *(uint4*)(As + r * kLdsK + kc) = v;
-      }
-    }
-    // ---- stage B tile into Bs[n][k] ----
-#pragma unroll
-    for (int c2 = 0; c2 < BN / 64; ++c2) {
-      const int c = t + c2 * 256;
-      if (LAYOUT == kNT) {
-        const int r = c >> 2, kc = (c & 3) * 8;
-        uint4 v = make_uint4(0, 0, 0, 0);
-        if (n0 + r < N && k0 + kc < kend)
-          v = *(const uint4*)(B + (int64_t)(n0 + r) * ldb + k0 + kc);
-        *(uint4*)(Bs + r * kLdsK + kc) = v;
-      } else {
-        const int kk = c / (BN / 8), nc = (c % (BN / 8)) * 8;
-        uint4 v = make_uint4(0, 0, 0, 0);
-        if (k0 + kk < kend && n0 + nc < N)
-          v = *(const uint4*)(B + (int64_t)(k0 + kk) * ldb + n0 + nc);
-        const uint16_t* h = (const uint16_t*)&v;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) Bs[(nc + j) * kLdsK + kk] = h[j];
-      }
-    }
+    uint16_t* la = lds + buf * 2 * kBT * kLdsK;
+    uint16_t* lb = la + kBT * kLdsK;
+    sa.store(la);
+    sb.store(lb);
+    // the buffer of the step before is written again only after this barrier
+    // of the next step, which every wave reaches when done reading it
     __syncthreads();
-    // ---- MFMA: each wave TI x TJ tiles of 32 x 32, two k-steps ----
+    if (k0 + kBK < kend) {
+      sa.load(A, lda, m0, M, k0 + kBK, kend);
+      sb.load(B, ldb, n0, N, k0 + kBK, kend);
+    }
 #pragma unroll
     for (int ks = 0; ks < kBK; ks += 16) {
-      const int kq = ks + (lane >> 5) * 8;
-      bf16x8 a[TI], b[TJ];
+      const bf16x8 a = __builtin_bit_cast(bf16x8, *(const uint4*)(la + ra + ks));
+      const bf16x8 b = __builtin_bit_cast(bf16x8, *(const uint4*)(lb + rb + ks));
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+    }
+    buf ^= 1;
+  }
+  return acc;
+}
+
+// Row of accumulator value a: D[row][col], col = lane % 32,
+// row = 8 (a / 4) + 4 (lane / 32) + a % 4.
+__device__ __forceinline__ int acc_row(int a, int lane) {
+  return 8 * (a >> 2) + 4 * (lane >> 5) + (a & 3);
+}
+
+// C[M,N] = sum_k A[m][k] B[n][k] (BKM: B[k][n]) with the epilogue EPI.
+// Tiles of 64 x 64 for all M: at 4096 rows the widest layer has 512
+// workgroups, at 32768 rows the narrow ones 2048.  The forward pass takes
+// 22, 24 and 79 us at 256, 4096 and 32768 rows (29, 32 and 79 us with a K
+// step of 32 and no loads in flight across it).
+template <bool BKM, int EPI>
+__global__ void __launch_bounds__(256)
+    gemm_bf16_k(int M, int N, int K, const uint16_t* __restrict__ A, int lda,
+                const uint16_t* __restrict__ B, int ldb, EpiArgs ep) {
+  __shared__ __attribute__((aligned(16))) uint16_t lds[kTileLds];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int m0 = blockIdx.x * kBT, n0 = blockIdx.y * kBT;
+  const int rw = m0 + (w >> 1) * 32, col = n0 + (w & 1) * 32 + (lane & 31);
+  f32x16 acc = tile_mma<false, BKM>(A, lda, m0, M, B, ldb, n0, N, 0, K, lds);
+  if constexpr (EPI == kFwdHidden || EPI == kFwdOut) {
+    if (col >= N) return;
+    const float bias = ep.bias[col];
 #pragma unroll
-      for (int i = 0; i < TI; ++i) {
-        const int row = wm * (BM / 2) + i * 32 + (lane & 31);
-        const uint4 v = *(const uint4*)(As + row * kLdsK + kq);
-        a[i] = __builtin_bit_cast(bf16x8, v);
+    for (int a = 0; a < 16; ++a) {
+      const int row = rw + acc_row(a, lane);
+      if (row >= M) continue;
+      const int64_t o = (int64_t)row * ep.ldc + col;
+      const float z = acc[a] + bias;
+      if constexpr (EPI == kFwdHidden) {
+        if (ep.zf) ep.zf[o] = z;
+        ep.hb[o] = f2bf(silu(z));
+      } else {
+        if (ep.yf) ep.yf[o] = z;
+        if (ep.yd) ep.yd[o] = (double)z * ep.yscale[0];
       }
+    }
+  } else {
+    // dZ: FwdLoss d(loss)/dY of Y = acc + bias against the targets, BwdData
+    // acc * silu'(Z); stored in BF16, its column sums over the tile's 64
+    // rows taken from the FP32 values.  N is a multiple of the tile here.
+    float z[16];
 #pragma unroll
-      for (int j = 0; j < TJ; ++j) {
-        const int col = wn * (BN / 2) + j * 32 + (lane & 31);
-        const uint4 v = *(const uint4*)(Bs + col * kLdsK + kq);
-        b[j] = __builtin_bit_cast(bf16x8, v);
+    for (int a = 0; a < 16; ++a) {
+      const int row = min(rw + acc_row(a, lane), M - 1);
+      z[a] = ep.z[(int64_t)row * ep.ldc + col];
+    }
+    const float bias = EPI == kFwdLoss ? ep.bias[col] : 0.0f;
+    const float inv =
+        EPI == kFwdLoss && ep.yscale != nullptr ? (float)ep.yscale[1] : 1.0f;
+    double loss = 0.0;
+    float cs = 0.0f;
+#pragma unroll
+    for (int a = 0; a < 16; ++a) {
+      const int row = rw + acc_row(a, lane);
+      if (row >= M) continue;
+      float dz;
+      if constexpr (EPI == kFwdLoss) {
+        const float d = acc[a] + bias - z[a] * inv;
+        loss += (double)d * (double)d;
+        dz = ep.gscale * d;
+      } else {
+        dz = acc[a] * dsilu(z[a]);
       }
-#pragma unroll
-      for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j],
-                                                              acc[i][j], 0, 0, 0);
+      ep.hb[(int64_t)row * ep.ldc + col] = f2bf(dz);
+      cs += dz;
+    }
+    __shared__ float scol[2][kBT];
+    __shared__ double sloss[4];
+    cs += __shfl_xor(cs, 32, 64);
+    if (lane < 32) scol[w >> 1][(w & 1) * 32 + lane] = cs;
+    if constexpr (EPI == kFwdLoss) {
+      loss = wave_sum(loss);
+      if (lane == 0) sloss[w] = loss;
     }
     __syncthreads();
+    if (threadIdx.x < kBT)
+      ep.colpart[(int64_t)blockIdx.x * ep.ldc + n0 + threadIdx.x] =
+          scol[0][threadIdx.x] + scol[1][threadIdx.x];
+    if (EPI == kFwdLoss && threadIdx.x == 0)
+      ep.lpart[blockIdx.y * gridDim.x + blockIdx.x] =
+          (sloss[0] + sloss[1]) + (sloss[2] + sloss[3]);
   }
+}
 
-  // ---- epilogue: D[row][col], col = lane % 32, row = 8(a/4) + 4(lane/32) + a%4
+// The three weight gradients dW_l = dZ_l^T H_{l-1}, split over the rows:
+// workgroup (tile, z) sums rows [z kz, (z+1) kz) of one 64 x 64 tile of one
+// layer into ws[z] (the padded parameter layout).  One launch for all three:
+// each alone has 16 to 36 tiles for 256 CUs.
+struct WgradArgs {
+  const uint16_t* dz[3];  // [M][rows[l]]
+  const uint16_t* h[3];   // [M][cols[l]]
+};
+constexpr int kWgTiles1 = (kHID / kBT) * ((kKIN + kBT - 1) / kBT);
+constexpr int kWgTiles2 = (kHID / kBT) * (kHID / kBT);
+constexpr int kWgTiles3 = (kNP / kBT) * (kHID / kBT);
+constexpr int kWgTiles = kWgTiles1 + kWgTiles2 + kWgTiles3;
+
+__global__ void __launch_bounds__(256)
+    mlp_wgrad_k(int M, int kz, WgradArgs v, float* __restrict__ ws) {
+  __shared__ __attribute__((aligned(16))) uint16_t lds[kTileLds];
+  int tile = blockIdx.x, l = 0;
+  int64_t off = kOffW1;
+  if (tile >= kWgTiles1 + kWgTiles2) {
+    tile -= kWgTiles1 + kWgTiles2;
+    l = 2;
+    off = kOffW3;
+  } else if (tile >= kWgTiles1) {
+    tile -= kWgTiles1;
+    l = 1;
+    off = kOffW2;
+  }
+  const int rows = l == 2 ? kNP : kHID, cols = l == 0 ? kKIN : kHID;
+  const int m0 = tile % (rows / kBT) * kBT, n0 = tile / (rows / kBT) * kBT;
+  const int kbeg = blockIdx.y * kz, kend = min(M, kbeg + kz);
+  const f32x16 acc = tile_mma<true, true>(v.dz[l], rows, m0, rows, v.h[l],
+                                          cols, n0, cols, kbeg, kend, lds);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int col = n0 + (w & 1) * 32 + (lane & 31);
+  if (col >= cols) return;
+  float* o = ws + (int64_t)blockIdx.y * kNParPad + off + col;
 #pragma unroll
-  for (int i = 0; i < TI; ++i)
+  for (int a = 0; a < 16; ++a)
+    o[(int64_t)(m0 + (w >> 1) * 32 + acc_row(a, lane)) * cols] = acc[a];
+}
+
+// The gradient from its partial sums: weights over the nz row splits of ws,
+// biases over the nt tile rows of cp ([nt][512] b3, then [nt][256] b2 and
+// b1), acc[0] = (accum ? acc[0] : 0) + the np loss partials, each in a fixed
+// order.  g: padded layout (the padding columns of W1 zero); out: unpadded
+// (may be null).
+constexpr int kFinW = (int)((kNParPad - (2 * kHID + kNP)) / 4 + 255) / 256;
+constexpr int kFinB = (2 * kHID + kNP) / 16;
+__global__ void __launch_bounds__(256)
+    mlp_grad_fin_k(const float* __restrict__ ws, int nz,
+                   const float* __restrict__ cp, int nt,
+                   const double* __restrict__ lpart, int np, int accum,
+                   double* __restrict__ acc, float* __restrict__ g,
+                   float* __restrict__ out) {
+  __shared__ float sc[256];
+  __shared__ double sh[256 / 64];
+  const int t = threadIdx.x, b = blockIdx.x;
+  constexpr int64_t kPad = (int64_t)kHID * (kKIN - kNIN);
+  if (b < kFinW) {
+    // the i-th group of 4 weights, b1 and b2 left out
+    int64_t i = 4 * ((int64_t)b * 256 + t);
+    if (i >= kOffB1) i += kHID;
+    if (i >= kOffB2) i += kHID;
+    if (i >= kOffB3) return;
+    float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll 4
+    for (int z = 0; z < nz; ++z) {
+      const float4 v = *(const float4*)(ws + (int64_t)z * kNParPad + i);
+      s.x += v.x;
+      s.y += v.y;
+      s.z += v.z;
+      s.w += v.w;
+    }
+    float q[4] = {s.x, s.y, s.z, s.w};
 #pragma unroll
-    for (int j = 0; j < TJ; ++j)
-#pragma unroll
-      for (int a = 0; a < 16; ++a) {
-        const int row = m0 + wm * (BM / 2) + i * 32 + 8 * (a >> 2) +
-                        4 * (lane >> 5) + (a & 3);
-        const int col = n0 + wn * (BN / 2) + j * 32 + (lane & 31);
-        if (row >= M || col >= N) continue;
-        const int64_t o = (int64_t)row * ep.ldc + col;
-        const float v = acc[i][j][a];
-        if constexpr (EPI == kFwdHidden) {
-          const float zz = v + ep.bias[col];
-          if (ep.zf) ep.zf[o] = zz;
-          ep.hb[o] = f2bf(silu(zz));
-        } else if constexpr (EPI == kFwdOut) {
-          const float y = v + ep.bias[col];
-          if (ep.yf) ep.yf[o] = y;
-          if (ep.yd) ep.yd[o] = (double)y * ep.yscale[0];
-        } else if constexpr (EPI == kBwdData) {
-          const float dz = v * dsilu(ep.z[o]);
-          ep.zf[o] = dz;
-          ep.hb[o] = f2bf(dz);
-        } else {
-          ep.zf[(int64_t)blockIdx.z * M * ep.ldc + o] = v;
-        }
+    for (int j = 0; j < 4; ++j) {
+      const int64_t p = i + j;
+      if (p < kOffB1) {
+        const int64_t r = p / kKIN, c = p % kKIN;
+        if (c >= kNIN) q[j] = 0.0f;
+        else if (out) out[r * kNIN + c] = q[j];
+      } else if (out) {
+        out[p - kPad] = q[j];
       }
+    }
+    *(float4*)(g + i) = make_float4(q[0], q[1], q[2], q[3]);
+  } else if (b < kFinW + kFinB) {
+    // 16 columns, 16 threads each over the tile rows
+    const int c0 = (b - kFinW) * 16, c = c0 + (t & 15), ch = t >> 4;
+    const float* p = cp + c;  // b3
+    int ld = kNP;
+    int64_t o = kOffB3 + c;
+    if (c0 >= kNP + kHID) {
+      p = cp + (int64_t)nt * (kNP + kHID) + (c - kNP - kHID);
+      ld = kHID;
+      o = kOffB1 + (c - kNP - kHID);
+    } else if (c0 >= kNP) {
+      p = cp + (int64_t)nt * kNP + (c - kNP);
+      ld = kHID;
+      o = kOffB2 + (c - kNP);
+    }
+    float s = 0.0f;
+#pragma unroll 4
+    for (int r = ch; r < nt; r += 16) s += p[(int64_t)r * ld];
+    sc[t] = s;
+    __syncthreads();
+    if (t < 16) {
+      float q = 0.0f;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) q += sc[k * 16 + t];
+      g[o] = q;
+      if (out) out[o - kPad] = q;
+    }
+  } else {
+    const double s = sum_partials<256>(lpart, np, sh);
+    if (t == 0) acc[0] = (accum ? acc[0] : 0.0) + s;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -295,72 +481,6 @@ __global__ void __launch_bounds__(256)
     T[i] = (float)(x[i] * inv);
 }
 
-// dY = 2 (Y - T inv_ysc) / (M 512) as FP32 and BF16; part[b] = partial of
-// (Y - T inv_ysc)^2.
-__global__ void __launch_bounds__(256)
-    mlp_dloss_k(int64_t n, const float* __restrict__ Y,
-                const float* __restrict__ T, const double* __restrict__ ysc,
-                float* __restrict__ dzf, uint16_t* __restrict__ dzb,
-                double* __restrict__ part) {
-  __shared__ double sh[256 / 64];
-  const float inv = (float)ysc[1];
-  const float g = 2.0f / (float)n;
-  double s = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * 256) {
-    const float d = Y[i] - T[i] * inv;
-    s += (double)d * (double)d;
-    const float dz = g * d;
-    dzf[i] = dz;
-    dzb[i] = f2bf(dz);
-  }
-  s = block_sum<256>(s, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
-}
-
-// Column sums db[c] = sum_r dz[r][c] in two fixed-order levels:
-// part[chunk][c] = sum of kColRows consecutive rows, then db[c] = sum of the
-// chunks.  kColRows rows per thread, unrolled so the loads overlap.
-constexpr int kColRows = 64;
-
-__global__ void __launch_bounds__(256)
-    mlp_colsum_part_k(int M, int N, const float* __restrict__ dz,
-                      float* __restrict__ part) {
-  const int c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= N) return;
-  const int r0 = blockIdx.y * kColRows;
-  const int r1 = min(M, r0 + kColRows);
-  float s = 0.0f;
-#pragma unroll 16
-  for (int r = r0; r < r1; ++r) s += dz[(int64_t)r * N + c];
-  part[(int64_t)blockIdx.y * N + c] = s;
-}
-
-__global__ void __launch_bounds__(256)
-    mlp_colsum_fin_k(int nchunk, int N, const float* __restrict__ part,
-                     float* __restrict__ db) {
-  const int c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= N) return;
-  float s = 0.0f;
-  for (int q = 0; q < nchunk; ++q) s += part[(int64_t)q * N + c];
-  db[c] = s;
-}
-
-// g[i] = sum_z ws[z][i] for the first ncols of every row of width ld.
-__global__ void __launch_bounds__(256)
-    mlp_splitk_sum_k(int64_t rows, int ld, int ncols, int nz,
-                     const float* __restrict__ ws, float* __restrict__ g) {
-  const int64_t n = rows * ld;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * 256) {
-    const int col = (int)(i % ld);
-    float s = 0.0f;
-    if (col < ncols)
-      for (int z = 0; z < nz; ++z) s += ws[(int64_t)z * n + i];
-    g[i] = s;
-  }
-}
-
 // Adam on the padded FP32 parameters; refreshes the BF16 weight copies.
 // Padding entries have zero gradient and stay zero.
 __global__ void __launch_bounds__(256)
@@ -393,20 +513,6 @@ __global__ void __launch_bounds__(256)
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * 256)
     b[i] = f2bf(a[i]);
-}
-
-// out (unpadded, 330,240) <- in (padded)
-__global__ void __launch_bounds__(256)
-    mlp_unpad_k(const float* __restrict__ in, float* __restrict__ out) {
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-       i < NEKOAMD_MLP_NPARAM; i += (int64_t)gridDim.x * 256) {
-    int64_t src;
-    if (i < (int64_t)kHID * kNIN)
-      src = (i / kNIN) * kKIN + (i % kNIN);
-    else
-      src = kOffB1 + (i - (int64_t)kHID * kNIN);
-    out[i] = in[src];
-  }
 }
 
 __global__ void __launch_bounds__(256)
@@ -482,15 +588,6 @@ __global__ void __launch_bounds__(kRedBlock)
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// acc[0] += sum of the np loss partials (one block, fixed order).
-__global__ void __launch_bounds__(kFinBlock)
-    mlp_loss_acc_k(const double* __restrict__ part, int np,
-                   double* __restrict__ acc) {
-  __shared__ double sh[kFinBlock / 64];
-  const double s = sum_partials<kFinBlock>(part, np, sh);
-  if (threadIdx.x == 0) acc[0] += s;
-}
-
 // ---------------------------------------------------------------------------
 struct MlpState {
   int nelv = 0, nx = 0, ny = 0, nz = 0;
@@ -506,9 +603,10 @@ struct MlpState {
   // per-batch work (rows = max(batch, nelv))
   int rows = 0;
   uint16_t *xb = nullptr, *h1 = nullptr, *h2 = nullptr, *dzb = nullptr;
-  float *z1 = nullptr, *z2 = nullptr, *y = nullptr, *dzf = nullptr;
-  float* ws = nullptr;  // split-K partials
-  int64_t ws_len = 0;
+  float *z1 = nullptr, *z2 = nullptr;
+  float* ws = nullptr;     // kMaxSplit padded parameter sets: split-K partials
+  float* cpart = nullptr;  // [tile row][512 + 256 + 256] column sums of dZ
+  double* lpart = nullptr; // [tile row][512 / 64] loss partials
   double* mean = nullptr;  // nelv
   double* sc = nullptr;    // scalars: [0..1] rms/inv of the input field,
                            // [2..3] target scale, [8..12] guess dots/gamma
@@ -522,60 +620,36 @@ struct MlpState {
 
 static MlpState* as_mlp(void* p) { return (MlpState*)p; }
 
-// K range per split (a multiple of the K tile) and the number of splits.
-static int split_kz(int K, int splits) {
-  if (splits <= 1) return K;
-  return ((K + splits - 1) / splits + kBK - 1) / kBK * kBK;
-}
-static int split_nz(int K, int splits) {
-  const int kz = split_kz(K, splits);
-  return kz > 0 ? (K + kz - 1) / kz : 1;
-}
-
-template <int LAYOUT, int EPI, int BM = kBM, int BN = kBN>
+template <bool BKM, int EPI>
 static int gemm(int M, int N, int K, const uint16_t* A, int lda,
-                const uint16_t* B, int ldb, const EpiArgs& ep, int splits = 1) {
-  if (M <= 0 || N <= 0) return kOk;
-  const int kz = split_kz(K, splits);
-  const int nz = split_nz(K, splits);
-  dim3 grid((M + BM - 1) / BM, (N + BN - 1) / BN, nz);
-  hipLaunchKernelGGL((gemm_bf16_k<LAYOUT, EPI, BM, BN>), grid, dim3(256), 0,
-                     stream(), M, N, K, kz, A, lda, B, ldb, ep);
+                const uint16_t* B, int ldb, const EpiArgs& ep) {
+  if (M <= 0) return kOk;
+  dim3 grid((M + kBT - 1) / kBT, (N + kBT - 1) / kBT);
+  hipLaunchKernelGGL((gemm_bf16_k<BKM, EPI>), grid, dim3(256), 0, stream(), M,
+                     N, K, A, lda, B, ldb, ep);
   NK_LAUNCHED();
   return kOk;
 }
 
-// db = column sums of dz[M][N]; uses the split-K workspace as scratch.
-static int colsum(MlpState* s, int M, int N, const float* dz, float* db) {
-  const int nchunk = (M + kColRows - 1) / kColRows;
-  hipLaunchKernelGGL(mlp_colsum_part_k, dim3((N + 255) / 256, nchunk),
-                     dim3(256), 0, stream(), M, N, dz, s->ws);
-  NK_LAUNCHED();
-  hipLaunchKernelGGL(mlp_colsum_fin_k, dim3((N + 255) / 256), dim3(256), 0,
-                     stream(), nchunk, N, s->ws, db);
-  NK_LAUNCHED();
-  return kOk;
-}
-
-static int nsplits(int K) {
-  int z = K / 512;
-  return z < 1 ? 1 : (z > 32 ? 32 : z);
-}
-
-// Forward over M rows of X into the state's work buffers.
-static int forward(MlpState* s, const uint16_t* X, int M, bool keep_z,
-                   float* yf, double* yd, const double* yscale) {
+// The two hidden layers over M rows of X into the state's work buffers.
+static int forward_hidden(MlpState* s, const uint16_t* X, int M, bool keep_z) {
   EpiArgs e{};
   e.bias = s->th + kOffB1;
   e.zf = keep_z ? s->z1 : nullptr;
   e.hb = s->h1;
   e.ldc = kHID;
-  int rc = gemm<kNT, kFwdHidden, 64, 64>(M, kHID, kKIN, X, kKIN, s->w1b, kKIN, e);
+  const int rc =
+      gemm<false, kFwdHidden>(M, kHID, kKIN, X, kKIN, s->w1b, kKIN, e);
   if (rc) return rc;
   e.bias = s->th + kOffB2;
   e.zf = keep_z ? s->z2 : nullptr;
   e.hb = s->h2;
-  rc = gemm<kNT, kFwdHidden, 64, 64>(M, kHID, kHID, s->h1, kHID, s->w2b, kHID, e);
+  return gemm<false, kFwdHidden>(M, kHID, kHID, s->h1, kHID, s->w2b, kHID, e);
+}
+
+static int forward(MlpState* s, const uint16_t* X, int M, float* yf,
+                   double* yd, const double* yscale) {
+  const int rc = forward_hidden(s, X, M, false);
   if (rc) return rc;
   EpiArgs o{};
   o.bias = s->th + kOffB3;
@@ -583,68 +657,54 @@ static int forward(MlpState* s, const uint16_t* X, int M, bool keep_z,
   o.yd = yd;
   o.yscale = yscale;
   o.ldc = kNP;
-  return gemm<kNT, kFwdOut, 64, 64>(M, kNP, kHID, s->h2, kHID, s->w3b, kHID, o);
+  return gemm<false, kFwdOut>(M, kNP, kHID, s->h2, kHID, s->w3b, kHID, o);
 }
 
-// Gradient of the batch (X, T) into s->g (padded layout); loss partials in
-// s->part[0..np).  inv_ysc: device scalar the targets are multiplied by.
+// Gradient of the batch (X, T) into s->g (padded layout) and out (unpadded,
+// may be null); the loss sum into acc (added to it when accum).  ysc[1]:
+// device scalar the targets are multiplied by (null: none).
 static int backward(MlpState* s, const uint16_t* X, const float* T, int M,
-                    const double* ysc, int* np_out) {
-  int rc = forward(s, X, M, true, s->y, nullptr, nullptr);
+                    const double* ysc, int accum, double* acc, float* out) {
+  int rc = forward_hidden(s, X, M, true);
   if (rc) return rc;
-  const int64_t ny = (int64_t)M * kNP;
-  const int gl = nk_grid(ny, 256, kRedGrid);
-  hipLaunchKernelGGL(mlp_dloss_k, dim3(gl), dim3(256), 0, stream(), ny, s->y,
-                     T, ysc, s->dzf, s->dzb, s->part);
-  NK_LAUNCHED();
-  *np_out = gl;
-  // layer 3
-  rc = colsum(s, M, kNP, s->dzf, s->g + kOffB3);
+  const int nt = (M + kBT - 1) / kBT;
+  uint16_t* dz3 = s->dzb;
+  uint16_t* dz2 = dz3 + (int64_t)M * kNP;
+  uint16_t* dz1 = dz2 + (int64_t)M * kHID;
+  EpiArgs e{};
+  e.bias = s->th + kOffB3;
+  e.z = T;
+  e.hb = dz3;
+  e.yscale = ysc;
+  e.gscale = 2.0f / (float)((int64_t)M * kNP);
+  e.colpart = s->cpart;
+  e.lpart = s->lpart;
+  e.ldc = kNP;
+  rc = gemm<false, kFwdLoss>(M, kNP, kHID, s->h2, kHID, s->w3b, kHID, e);
   if (rc) return rc;
-  const int sp = nsplits(M);
-  EpiArgs w{};
-  w.zf = s->ws;
-  w.ldc = kHID;
-  rc = gemm<kTN, kWgrad>(kNP, kHID, M, s->dzb, kNP, s->h2, kHID, w, sp);
-  if (rc) return rc;
-  const int nz = split_nz(M, sp);
-  hipLaunchKernelGGL(mlp_splitk_sum_k, dim3(nk_grid((int64_t)kNP * kHID, 256)),
-                     dim3(256), 0, stream(), (int64_t)kNP, kHID, kHID, nz,
-                     s->ws, s->g + kOffW3);
-  NK_LAUNCHED();
-  // dZ2 = (dZ3 W3) * silu'(Z2): dZ3 lives in dz*[0, M*512), dZ2 goes
-  // behind it; dZ1 then reuses the front of the buffers.
-  uint16_t* dz2b = s->dzb + ny;
-  float* dz2f = s->dzf + ny;
   EpiArgs d{};
   d.z = s->z2;
-  d.zf = dz2f;
-  d.hb = dz2b;
+  d.hb = dz2;
+  d.colpart = s->cpart + (int64_t)nt * kNP;
   d.ldc = kHID;
-  rc = gemm<kNN, kBwdData>(M, kHID, kNP, s->dzb, kNP, s->w3b, kHID, d);
+  rc = gemm<true, kBwdData>(M, kHID, kNP, dz3, kNP, s->w3b, kHID, d);
   if (rc) return rc;
-  rc = colsum(s, M, kHID, dz2f, s->g + kOffB2);
-  if (rc) return rc;
-  rc = gemm<kTN, kWgrad>(kHID, kHID, M, dz2b, kHID, s->h1, kHID, w, sp);
-  if (rc) return rc;
-  hipLaunchKernelGGL(mlp_splitk_sum_k, dim3(nk_grid((int64_t)kHID * kHID, 256)),
-                     dim3(256), 0, stream(), (int64_t)kHID, kHID, kHID, nz,
-                     s->ws, s->g + kOffW2);
-  NK_LAUNCHED();
-  // dZ1 = (dZ2 W2) * silu'(Z1) into the first part of the buffers
   d.z = s->z1;
-  d.zf = s->dzf;
-  d.hb = s->dzb;
-  rc = gemm<kNN, kBwdData>(M, kHID, kHID, dz2b, kHID, s->w2b, kHID, d);
+  d.hb = dz1;
+  d.colpart += (int64_t)nt * kHID;
+  rc = gemm<true, kBwdData>(M, kHID, kHID, dz2, kHID, s->w2b, kHID, d);
   if (rc) return rc;
-  rc = colsum(s, M, kHID, s->dzf, s->g + kOffB1);
-  if (rc) return rc;
-  w.ldc = kKIN;
-  rc = gemm<kTN, kWgrad>(kHID, kKIN, M, s->dzb, kHID, X, kKIN, w, sp);
-  if (rc) return rc;
-  hipLaunchKernelGGL(mlp_splitk_sum_k, dim3(nk_grid((int64_t)kHID * kKIN, 256)),
-                     dim3(256), 0, stream(), (int64_t)kHID, kKIN, kNIN, nz,
-                     s->ws, s->g + kOffW1);
+  // row splits: at least one K step each, and no more than the partials'
+  // buffer holds
+  const int per = (nt + kMaxSplit - 1) / kMaxSplit;
+  const int nz = (nt + per - 1) / per;
+  WgradArgs v{{dz1, dz2, dz3}, {X, s->h1, s->h2}};
+  hipLaunchKernelGGL(mlp_wgrad_k, dim3(kWgTiles, nz), dim3(256), 0, stream(),
+                     M, per * kBK, v, s->ws);
+  NK_LAUNCHED();
+  hipLaunchKernelGGL(mlp_grad_fin_k, dim3(kFinW + kFinB + 1), dim3(256), 0,
+                     stream(), s->ws, nz, s->cpart, nt, s->lpart,
+                     nt * (kNP / kBT), accum, acc, s->g, out);
   NK_LAUNCHED();
   return kOk;
 }
@@ -708,7 +768,7 @@ int mlp_direction(void* mlp, int64_t n, const double* r, double* q,
     return fail_arg("mlp_direction", "the network was made for another mesh");
   int rc = rms(s, r, s->sc);
   if (!rc) rc = make_features(s, r, s->sc, s->xb);
-  if (!rc) rc = forward(s, s->xb, s->nelv, false, nullptr, q, s->sc);
+  if (!rc) rc = forward(s, s->xb, s->nelv, nullptr, q, s->sc);
   if (!rc) rc = gs_launch<double>(gs, q, NEKOAMD_GS_ADD, nullptr);
   if (rc) return rc;
   hipLaunchKernelGGL(mlp_mulmask_k, dim3(nk_grid(s->n, 256)), dim3(256), 0,
@@ -742,8 +802,7 @@ int nekoamd_mlp_create(void** mlp, const int* nx, const int* ny, const int* nz,
   s->cap = *capacity;
   s->rows = s->nelv > *batch ? s->nelv : *batch;
   const int64_t R = s->rows;
-  s->ws_len = 32LL * kHID * kKIN;
-  if ((int64_t)kNP * kHID * 32 > s->ws_len) s->ws_len = (int64_t)kNP * kHID * 32;
+  const int64_t nt = (R + kBT - 1) / kBT;
   hipError_t e = hipSuccess;
   s->nbr = dalloc<int32_t>((int64_t)s->nelv * 6, e);
   s->th = dalloc<float>(kNParPad, e);
@@ -758,12 +817,12 @@ int nekoamd_mlp_create(void** mlp, const int* nx, const int* ny, const int* nz,
   s->xb = dalloc<uint16_t>(R * kKIN, e);
   s->h1 = dalloc<uint16_t>(R * kHID, e);
   s->h2 = dalloc<uint16_t>(R * kHID, e);
-  s->dzb = dalloc<uint16_t>(R * (kNP + kHID), e);
+  s->dzb = dalloc<uint16_t>(R * (kNP + 2 * kHID), e);
   s->z1 = dalloc<float>(R * kHID, e);
   s->z2 = dalloc<float>(R * kHID, e);
-  s->y = dalloc<float>(R * kNP, e);
-  s->dzf = dalloc<float>(R * (kNP + kHID), e);
-  s->ws = dalloc<float>(s->ws_len, e);
+  s->ws = dalloc<float>(kMaxSplit * kNParPad, e);
+  s->cpart = dalloc<float>(nt * (kNP + 2 * kHID), e);
+  s->lpart = dalloc<double>(nt * (kNP / kBT), e);
   s->mean = dalloc<double>(s->nelv, e);
   s->sc = dalloc<double>(16, e);
   s->part = dalloc<double>(3 * kRedGrid, e);
@@ -827,7 +886,7 @@ int nekoamd_mlp_free(void* mlp) {
   if (initialised()) NK_HIP(hipStreamSynchronize(stream()));
   void* dev[] = {s->nbr, s->th,  s->g,    s->m,    s->v,  s->w1b, s->w2b,
                  s->w3b, s->Xd,  s->Td,   s->xb,   s->h1, s->h2,  s->dzb,
-                 s->z1,  s->z2,  s->y,    s->dzf,  s->ws, s->mean, s->sc,
+                 s->z1,  s->z2,  s->cpart, s->lpart, s->ws, s->mean, s->sc,
                  s->part, s->q,  s->aq,   s->bsave};
   for (void* p : dev)
     if (p) NK_HIP(hipFree(p));
@@ -873,8 +932,7 @@ int nekoamd_mlp_forward(void* mlp, const void* X, const int* M, void* Y,
   MlpState* s = as_mlp(mlp);
   NK_REQUIRE(s && X && M && Y, "null argument");
   NK_REQUIRE(*M >= 0 && *M <= s->rows, "M exceeds the work buffers");
-  int rc = forward(s, (const uint16_t*)X, *M, false, (float*)Y, nullptr,
-                   nullptr);
+  int rc = forward(s, (const uint16_t*)X, *M, (float*)Y, nullptr, nullptr);
   if (rc) return rc;
   if (H1)
     NK_HIP(hipMemcpyAsync(H1, s->h1, (size_t)*M * kHID * 2,
@@ -892,24 +950,10 @@ int nekoamd_mlp_loss_grad(void* mlp, const void* X, const void* T,
   NK_REQUIRE(s && X && T && M && loss && g, "null argument");
   NK_REQUIRE(*M > 0 && *M <= s->rows && *M % 8 == 0,
              "M must be a positive multiple of 8 within the work buffers");
-  // targets unscaled: sc[2..3] = {1, 1}
-  s->host[0] = 1.0;
-  s->host[1] = 1.0;
-  NK_HIP(hipMemcpyAsync(s->sc + 2, s->host, 2 * sizeof(double),
-                        hipMemcpyHostToDevice, stream()));
-  NK_HIP(hipMemsetAsync(s->sc + 6, 0, sizeof(double), stream()));
-  int np = 0;
-  int rc = backward(s, (const uint16_t*)X, (const float*)T, *M, s->sc + 2,
-                    &np);
+  int rc = backward(s, (const uint16_t*)X, (const float*)T, *M, nullptr, 0,
+                    s->sc + 6, (float*)g);
+  if (!rc) rc = to_host(s->host + 2, s->sc + 6, sizeof(double));
   if (rc) return rc;
-  hipLaunchKernelGGL(mlp_loss_acc_k, dim3(1), dim3(kFinBlock), 0, stream(),
-                     s->part, np, s->sc + 6);
-  NK_LAUNCHED();
-  hipLaunchKernelGGL(mlp_unpad_k, dim3(nk_grid(NEKOAMD_MLP_NPARAM, 256)),
-                     dim3(256), 0, stream(), s->g, (float*)g);
-  NK_LAUNCHED();
-  NK_HIP(hipMemcpyAsync(s->host + 2, s->sc + 6, sizeof(double),
-                        hipMemcpyDeviceToHost, stream()));
   NK_HIP(hipStreamSynchronize(stream()));
   *loss = s->host[2] / ((double)*M * kNP);
   return kOk;
@@ -974,16 +1018,11 @@ int nekoamd_mlp_train(void* mlp, const int* epochs, const int* batch,
   for (int ep = 0; ep < *epochs; ++ep) {
     for (int64_t q = 0; q < nb; ++q) order[(size_t)q] = q;
     std::shuffle(order.begin(), order.end(), rng);
-    NK_HIP(hipMemsetAsync(acc, 0, sizeof(double), stream()));
     for (int64_t q = 0; q < nb; ++q) {
       const int64_t r0 = order[(size_t)q] * B;
-      int np = 0;
-      int rc = backward(s, s->Xd + r0 * kKIN, s->Td + r0 * kNP, B, s->sc + 2,
-                        &np);
+      const int rc = backward(s, s->Xd + r0 * kKIN, s->Td + r0 * kNP, B,
+                              s->sc + 2, q > 0, acc, nullptr);
       if (rc) return rc;
-      hipLaunchKernelGGL(mlp_loss_acc_k, dim3(1), dim3(kFinBlock), 0,
-                         stream(), s->part, np, acc);
-      NK_LAUNCHED();
       ++s->adam_t;
       const float c1 = 1.0f - powf(b1, (float)s->adam_t);
       const float c2 = 1.0f - powf(b2, (float)s->adam_t);
@@ -1034,7 +1073,7 @@ int nekoamd_mlp_pre(void* mlp, void* b, const void* mult, void* gs,
   if (!*apply) return kOk;
   int rc = rms(s, bd, s->sc);
   if (!rc) rc = make_features(s, bd, s->sc, s->xb);
-  if (!rc) rc = forward(s, s->xb, s->nelv, false, nullptr, s->q, s->sc);
+  if (!rc) rc = forward(s, s->xb, s->nelv, nullptr, s->q, s->sc);
   if (!rc) rc = gs_launch<double>(gs, s->q, NEKOAMD_GS_ADD, nullptr);
   if (rc) return rc;
   hipLaunchKernelGGL(mlp_mulmask_k, dim3(ge), dim3(256), 0, stream(), n, s->q,

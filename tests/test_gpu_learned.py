@@ -100,6 +100,26 @@ def test_gradients_match_oracle(L):
         assert rel < 2e-3 and cos > 0.99999, k
 
 
+@pytest.mark.parametrize("M", [8, 72, 1096])
+def test_gradients_at_tile_edges(L, M):
+    """Row counts below one 64-row tile, with a remainder, and with unequal
+    row splits (1096 rows: 18 tile rows in 9 splits, the last one short); the
+    bars are those of the oracle comparison above (BF16 rounding of the hidden
+    activations and of dZ, FP32 sums)."""
+    from nekoamd import device as dev
+    rng = np.random.default_rng(M)
+    net, p = _net(L, rng, batch=1120)
+    Xd, Xq = _features(L, rng, M)
+    T = (rng.standard_normal((M, omlp.NP)) * 0.5).astype(np.float32)
+    loss, g = net.loss_grad(Xd, dev.DeviceArray.from_host(T.ravel()), M)
+    lo, go = omlp.loss_grad(p, Xq, T.astype(np.float64))
+    gu = omlp.unpack(g.astype(np.float64))
+    assert abs(loss - lo) < 1e-4 * lo
+    for k, _ in omlp.SIZES:
+        a, b = gu[k].ravel(), go[k].ravel()
+        assert np.linalg.norm(a - b) < 2e-3 * np.linalg.norm(b), k
+
+
 def test_training_lowers_loss_and_guess_is_safe(L):
     """Pairs (b, x) with A x = b from the device's FP64 CG on a 4^3 box of
     order 7; after training, a guessed solve reaches the same solution as the
