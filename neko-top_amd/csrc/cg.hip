@@ -53,6 +53,7 @@
 #include "ax_core.h"
 #include <algorithm>
 
+#include "gridsum.h"
 #include "internal.h"
 #include "nekoamd.h"
 #include "reduce.h"
@@ -78,6 +79,7 @@ struct CgScal {
   // the iteration kernels return at once while halt is set: the solve is
   // done, or (mixed) a reliable update was requested and has not yet run
   int halt;
+  int stuck;  // cg_grid_k gave up a wait: the solve starts over
 };
 
 static_assert(sizeof(CgScal) % 4 == 0, "CgScal is copied in 4-byte words");
@@ -113,6 +115,12 @@ struct CgState {
   // built)
   float* geo32 = nullptr;
   const void* geo_key[9] = {};
+  // cg_grid_k: the words its workgroups exchange (per workgroup 2 of pap, 4
+  // of rtr and rtz; then 2 of w per point), the next unused tag, and whether
+  // a solve of this state got stuck in it
+  uint64_t* slots = nullptr;
+  uint32_t tag = 1;
+  bool grid_off = false;
 };
 
 // ---------------------------------------------------------------------------
@@ -299,6 +307,7 @@ __global__ void __launch_bounds__(kFinBlock)
     sc->nupdate = 0;
     sc->done = (rn == 0.0 || max_iter <= 0) ? 1 : 0;
     sc->halt = sc->done;
+    sc->stuck = 0;
   }
 }
 
@@ -778,6 +787,175 @@ __global__ void __launch_bounds__(kFinBlock)
 }
 
 // ---------------------------------------------------------------------------
+// The FP64 iteration of small meshes as one kernel: workgroup b keeps the
+// vectors and operator data of EPB elements in registers over all iterations
+// (x, r, p, d_m, mult, G, h1, h2 B: 28 to 34 VGPRs), and an iteration is two
+// exchanges over the grid (gridsum.h) -- the shared points' w and the element
+// sums of w.p, then the sums of r.r and r.z.  A shared point gathers its
+// copies' w itself, summed in the order of the gs map, so every copy gets
+// the same bits.  The arithmetic per point is that of the
+// kernel-by-kernel iteration; the sums are taken in another order.
+//
+// Bound by the two exchanges, about 2 us each (a store and a load past the
+// L2s); the five launches it replaces take 17 us however small the mesh is.
+// FP64 pressure solve, us per solve by launches -> here: 8x4x4 order 5
+// (336 iterations) 6170 -> 2380, 8x8x4 order 7 12550 -> 6290, 12x10x8 order
+// 3 6330 -> 3470, 10x8x6 order 5 10240 -> 5260.
+//
+// Up to kGridWg workgroups, one per CU.  Two per CU lose: the registers then
+// spill and a reader has twice the slots to wait for (10x8x6 order 7, 480
+// workgroups: 21100 us against 17700 by launches; 14x10x7 order 5, 490
+// workgroups of two elements: 16300 against 15300).
+constexpr int kGridWg = 256;    // most workgroups of cg_grid_k
+constexpr int kGridCap = 2048;  // iterations of one launch
+
+struct CgGrid {
+  double *x, *r, *p;
+  uint64_t* w;         // two words per point
+  const double *dm, *mult, *dx, *h1, *h2;
+  const double *g11, *g12, *g13, *g22, *g23, *g33, *bm;
+  const int2* ref;     // per point: offset into idx and multiplicity
+  const int32_t* idx;
+  CgScal* sc;
+  uint64_t* slots;
+  uint32_t tag;
+  int nelv;
+};
+
+template <int LX, int EPB, bool H2>
+__global__ void __launch_bounds__((LX * LX * LX * EPB + 63) / 64 * 64)
+    cg_grid_k(CgGrid a) {
+  constexpr int NS = LX * LX, NP = NS * LX, NB = NP * EPB;
+  constexpr int BS = (NB + 63) / 64 * 64, NW = BS / 64;
+  // the threads past NB compute on a slice of their own and count for nothing
+  constexpr int NL = NB == BS ? NB : NB + NP;
+  __shared__ double su[NL];
+  __shared__ double sr[NL];
+  __shared__ double ss[NL];
+  __shared__ double st[NL];
+  __shared__ double sD[NS];
+  __shared__ double s1[NW], s2[NW], s3[2 * NW], s4[2 * NW];
+  __shared__ int fail;
+  CgScal* sc = a.sc;
+  if (sc->halt) return;  // the same in every workgroup: set before the launch
+  const int tid = threadIdx.x, nwg = gridDim.x;
+  const int el = tid / NP, t = tid % NP, o = el * NP;
+  const int e = blockIdx.x * EPB + el;
+  const bool live = tid < NB && e < a.nelv;
+  const int64_t g = live ? (int64_t)e * NP + t : 0;
+  if (tid < NS) sD[tid] = a.dx[tid];
+  if (tid == 0) fail = 0;
+  int it = sc->iter;
+  const int max_iter = sc->max_iter;
+  const double norm_fac = sc->norm_fac, abstol = sc->abstol;
+  double rtz1 = sc->rtz1, rtz2 = sc->rtz2, beta = sc->beta;
+  double alpha = 0.0, pap[1] = {0.0}, rr[2] = {0.0, 0.0}, rn = 0.0;
+  AxPoint<double> op{};
+  double x = 0.0, r = 0.0, p = 0.0, dm = 0.0, mult = 0.0;
+  int m = 0, idx[8] = {};
+  if (live) {
+    op = ax_load<double, double, double, H2>(g, a.h1, a.h2, a.g11, a.g12,
+                                             a.g13, a.g22, a.g23, a.g33, a.bm);
+    x = a.x[g];
+    r = a.r[g];
+    if (it > 0) p = a.p[g];
+    dm = a.dm[g];
+    mult = a.mult[g];
+    const int2 rf = a.ref[g];
+    m = rf.y;
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (q < m) idx[q] = a.idx[rf.x + q];
+  }
+  uint64_t* slot_p = a.slots;
+  uint64_t* slot_r = a.slots + 2 * nwg;
+  bool stop = false, ok = true;
+  for (int q = 0; q < kGridCap && !stop; ++q) {
+    const uint32_t tag = a.tag + 2u * (uint32_t)q;
+    const double z = r * dm;
+    p = it == 0 ? z : z + beta * p;
+    su[o + t] = p;
+    __syncthreads();
+    const double w = ax_point<LX, double, H2>(p, op, su + o, sr + o, ss + o,
+                                              st + o, sD, t);
+    if (m > 0) grid_put(a.w + 2 * g, tag, w);
+    const double d = wave_total(live ? w * p : 0.0);
+    if ((tid & 63) == 0) s1[tid >> 6] = d;
+    __syncthreads();
+    if (tid == 0) {
+      double v[1] = {0.0};
+#pragma unroll
+      for (int k = 0; k < NW; ++k) v[0] += s1[k];
+      grid_publish<1>(slot_p, blockIdx.x, tag, v);
+    }
+    double ws = w;
+    if (m > 0) {
+      const uint64_t* src[8];
+      double v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) src[k] = a.w + 2 * (int64_t)idx[k];
+      grid_get<8>(src, m, tag, &fail, v);
+      ws = v[0];
+#pragma unroll
+      for (int k = 1; k < 8; ++k)
+        if (k < m) ws += v[k];
+    }
+    if (!(ok = grid_sum<1>(slot_p, nwg, tag, s2, &fail, pap))) break;
+    alpha = rtz1 / pap[0];
+    x += alpha * p;
+    r = dm == 0.0 ? 0.0 : r - alpha * ws;
+    const double rm = r * mult;
+    const double c0 = wave_total(rm * r), c1 = wave_total(rm * (r * dm));
+    if ((tid & 63) == 0) {
+      s3[tid >> 6] = c0;
+      s3[NW + (tid >> 6)] = c1;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      double v[2] = {0.0, 0.0};
+#pragma unroll
+      for (int k = 0; k < NW; ++k) {
+        v[0] += s3[k];
+        v[1] += s3[NW + k];
+      }
+      grid_publish<2>(slot_r, blockIdx.x, tag + 1u, v);
+    }
+    // every workgroup has read its copies' w before it publishes here, so
+    // the next iteration may overwrite them
+    if (!(ok = grid_sum<2>(slot_r, nwg, tag + 1u, s4, &fail, rr))) break;
+    ++it;
+    rn = sqrt(rr[0]) * norm_fac;
+    beta = rr[1] / rtz1;
+    rtz2 = rtz1;
+    rtz1 = rr[1];
+    // a non-finite residual ends the solve (reported as not converged)
+    stop = rn < abstol || it >= max_iter || !isfinite(rn);
+  }
+  if (live) {
+    a.x[g] = x;
+    a.r[g] = r;
+    a.p[g] = p;
+  }
+  if (!ok) {
+    if (tid == 0) dev_store(&sc->stuck, 1);
+    return;
+  }
+  // every workgroup read sc before it first published, so before this
+  if (blockIdx.x == 0 && tid == 0) {
+    sc->iter = it;
+    sc->pap = pap[0];
+    sc->alpha = alpha;
+    sc->beta = beta;
+    sc->rtr = rr[0];
+    sc->rnorm = rn;
+    sc->rtz1 = rtz1;
+    sc->rtz2 = rtz2;
+    sc->done = stop ? 1 : 0;
+    sc->halt = sc->done;
+  }
+}
+
+// ---------------------------------------------------------------------------
 template <typename T, typename TG>
 static int ax_cg_launch(int lx, int nelv, bool ifh2, T* p, double* x, T* w,
                         const T* r, const T* dm, const double* dx, const T* h1,
@@ -1130,6 +1308,107 @@ static int cg_drive(CgState* s, int max_iter, int batch, F&& queue_batch) {
   return status;
 }
 
+// Workgroups of cg_grid_k on this device at once (0: it does not fit).
+template <int LX, int EPB, bool H2>
+static int cg_grid_room(int nelv, int* wg) {
+  constexpr int BS = (LX * LX * LX * EPB + 63) / 64 * 64;
+  *wg = (nelv + EPB - 1) / EPB;
+  if (*wg > kGridWg) return 0;
+  int dev = 0, cus = 0, per = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
+                            dev) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(
+          &per, (const void*)cg_grid_k<LX, EPB, H2>, BS, 0) != hipSuccess)
+    return 0;
+  return cus * per;
+}
+
+// One launch of up to kGridCap iterations; *ran = false where the mesh does
+// not fit.
+template <int LX, int EPB, bool H2>
+static int cg_grid_launch(const CgGrid& a, bool* ran) {
+  int wg = 0;
+  *ran = cg_grid_room<LX, EPB, H2>(a.nelv, &wg) >= wg;
+  if (!*ran) return kOk;
+  hipLaunchKernelGGL((cg_grid_k<LX, EPB, H2>), dim3(wg),
+                     dim3((LX * LX * LX * EPB + 63) / 64 * 64), 0, stream(), a);
+  NK_LAUNCHED();
+  return kOk;
+}
+
+template <int LX, int ES, int EL>
+static int cg_grid_pick(const CgGrid& a, bool h2, bool* ran) {
+  if (a.nelv <= kGridWg * ES)
+    return h2 ? cg_grid_launch<LX, ES, true>(a, ran)
+              : cg_grid_launch<LX, ES, false>(a, ran);
+  return h2 ? cg_grid_launch<LX, EL, true>(a, ran)
+            : cg_grid_launch<LX, EL, false>(a, ran);
+}
+
+// The started FP64 solve of s by cg_grid_k; *ran = false if the mesh is not
+// one of its (more than kGridWg workgroups, lx outside 4..8, points shared
+// by more than 8 elements), or if it got stuck (another process holding the
+// device): the caller then starts the solve over with the launches.  The
+// smaller orders take the fewest elements that make 256 threads while that
+// fits, else as many as 512 threads hold.
+static int cg_grid(CgState* s, const CgOp& op, double* x, const double* mult,
+                   bool* ran) {
+  *ran = false;
+  if (s->grid_off || s->nelv == 0 || op.lx < 4 || op.lx > 8) return kOk;
+  if (s->nelv > kGridWg * (op.lx == 4 ? 8 : op.lx == 5 ? 4 : op.lx == 6 ? 2 : 1))
+    return kOk;
+  CgGrid a{};
+  bool ok = false;
+  int rc = gs_point_refs(op.gs, 8, &a.ref, &a.idx, &ok);
+  if (rc || !ok) return rc;
+  if (!s->slots) {
+    const size_t bytes = sizeof(uint64_t) * (6 * kGridWg + 2 * (size_t)s->n);
+    NK_HIP(hipMalloc((void**)&s->slots, bytes));
+    NK_HIP(hipMemsetAsync(s->slots, 0, bytes, stream()));
+  }
+  a.x = x;
+  a.r = s->r;
+  a.p = s->p;
+  a.w = s->slots + 6 * kGridWg;
+  a.dm = s->dm;
+  a.mult = mult;
+  a.dx = op.dx;
+  a.h1 = op.h1;
+  a.h2 = op.h2;
+  a.g11 = op.g11;
+  a.g12 = op.g12;
+  a.g13 = op.g13;
+  a.g22 = op.g22;
+  a.g23 = op.g23;
+  a.g33 = op.g33;
+  a.bm = op.B;
+  a.sc = s->sc;
+  a.slots = s->slots;
+  a.nelv = s->nelv;
+  for (;;) {
+    a.tag = s->tag;
+    s->tag += 2 * kGridCap;
+    switch (op.lx) {
+      case 4: rc = cg_grid_pick<4, 4, 8>(a, op.ifh2, ran); break;
+      case 5: rc = cg_grid_pick<5, 2, 4>(a, op.ifh2, ran); break;
+      case 6: rc = cg_grid_pick<6, 1, 2>(a, op.ifh2, ran); break;
+      case 7: rc = cg_grid_pick<7, 1, 1>(a, op.ifh2, ran); break;
+      default: rc = cg_grid_pick<8, 1, 1>(a, op.ifh2, ran);
+    }
+    if (rc || !*ran) return rc;
+    rc = to_host(&s->host[0], s->sc, sizeof(CgScal));
+    if (rc) return rc;
+    NK_HIP(hipStreamSynchronize(stream()));
+    if (s->host[0].stuck) {
+      s->grid_off = true;
+      *ran = false;
+      return kOk;
+    }
+    if (s->host[0].done) return kOk;
+  }
+}
+
 // cg_drive for the three states of a coupled solve: each status read copies
 // the three device structs; the solve ends when all three are done (a
 // converged component's kernels skip on its done flag meanwhile).
@@ -1338,7 +1617,7 @@ int nekoamd_cg_free(void* cg) {
   void* dev[] = {s->sc,    s->part_ax, s->part_pap, s->part,  s->r,
                  s->w,     s->p,       s->dm,       s->r32,   s->p32,
                  s->w32,   s->dm32,    s->mult32,   s->h1_32, s->h2_32,
-                 s->geo32, s->dx32};
+                 s->geo32, s->dx32,    s->slots};
   for (void* q : dev)
     if (q) NK_HIP(hipFree(q));
   if (s->host) NK_HIP(hipHostFree(s->host));
@@ -1410,14 +1689,28 @@ int nekoamd_cg_solve(void* cg, void* x, const void* f, const void* d,
       NK_LAUNCHED();
     }
     double* X = (double*)x;
-    hipLaunchKernelGGL(cg_start_k<double>, dim3(s->grid), dim3(kRedBlock), 0,
-                       stream(), n, X, s->r, F, s->dm, (const double*)mult,
-                       nullptr, s->part);
-    NK_LAUNCHED();
-    hipLaunchKernelGGL(cg_start_fin_k, dim3(1), dim3(kFinBlock), 0, stream(),
-                       s->sc, s->part, s->grid, *volume, *abstol, *max_iter,
-                       0);
-    NK_LAUNCHED();
+    const auto start = [&]() -> int {
+      hipLaunchKernelGGL(cg_start_k<double>, dim3(s->grid), dim3(kRedBlock), 0,
+                         stream(), n, X, s->r, F, s->dm, (const double*)mult,
+                         nullptr, s->part);
+      NK_LAUNCHED();
+      hipLaunchKernelGGL(cg_start_fin_k, dim3(1), dim3(kFinBlock), 0, stream(),
+                         s->sc, s->part, s->grid, *volume, *abstol, *max_iter,
+                         0);
+      NK_LAUNCHED();
+      return kOk;
+    };
+    if ((status = start())) return status;
+    const bool was_off = s->grid_off;
+    bool ran = false;
+    status = cg_grid(s, op, X, (const double*)mult, &ran);
+    if (status) return status;
+    if (ran) {
+      fill_monitor(s->host[0], mon);
+      s->last_iter = mon->iter;
+      return kOk;
+    }
+    if (s->grid_off != was_off && (status = start())) return status;
     status = cg_drive(s, *max_iter, batch, [&](int nb) {
       for (int q = 0; q < nb; ++q) {
         int rc = cg_iteration<double>(s, op, geo64(op), X, s->r, s->p, s->w, s->dm,

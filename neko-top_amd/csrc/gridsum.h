@@ -1,0 +1,147 @@
+// gridsum.h -- sums over all workgroups of a running kernel, for solvers
+// whose iterations are too short to be launches of their own.
+//
+// Every workgroup publishes its partial sums in a slot of its own and reads
+// all slots: a reduction and a grid barrier in one exchange, without an
+// atomic that the workgroups contend for.  A double travels as two 64-bit
+// words of 32 value bits and a 32-bit tag, each stored and loaded whole at
+// device scope, so a reader knows from the word itself whether it belongs to
+// this exchange; tags must not repeat while an older word can still be in a
+// slot (one counter per set of slots, advanced over launches).
+//
+// Other values cross the grid the same way (grid_put, grid_get): the reader
+// waits for the very words it needs, so nothing has to be ordered before a
+// publish.  A word may be overwritten once a later exchange has shown that
+// every workgroup is past reading it.
+//
+// All workgroups must be resident at once: the launcher bounds the grid by
+// the occupancy of an empty device.  A wait lasts at most kGridWait; a
+// workgroup that gives up leaves, and so the others do.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "reduce.h"
+
+namespace nekoamd {
+
+constexpr unsigned long long kGridWait = 100000000ull;  // 1 s at 100 MHz
+
+template <typename T>
+__device__ __forceinline__ T dev_load(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void dev_store(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ void grid_put(uint64_t* s, uint32_t tag, double v) {
+  const uint64_t hi = (uint64_t)tag << 32;
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  dev_store(s, (uint64_t)(hi | (b & 0xFFFFFFFFull)));
+  dev_store(s + 1, (uint64_t)(hi | (b >> 32)));
+}
+// The N values at s[j], waited for together (their loads in flight at once);
+// the first n of them count.  *fail = 1 if the wait was given up.
+template <int N>
+__device__ __forceinline__ void grid_get(const uint64_t* const (&s)[N], int n,
+                                         uint32_t tag, int* fail,
+                                         double (&out)[N]) {
+  const unsigned long long t0 = wall_clock64();
+  for (;;) {
+    uint64_t w[2 * N];
+    bool here = true;
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      if (j < n) {
+        w[2 * j] = dev_load(s[j]);
+        w[2 * j + 1] = dev_load(s[j] + 1);
+      }
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      if (j < n) {
+        here &= (uint32_t)(w[2 * j] >> 32) == tag &&
+                (uint32_t)(w[2 * j + 1] >> 32) == tag;
+        out[j] = __longlong_as_double(
+            (long long)((w[2 * j] & 0xFFFFFFFFull) | (w[2 * j + 1] << 32)));
+      }
+    if (here) return;
+    if (wall_clock64() - t0 > kGridWait) {
+      *fail = 1;
+      return;
+    }
+  }
+}
+
+// The wave's sum of v in every lane (all 64 active), by lane moves of the
+// vector unit: within a row of 16 by quad permutes and mirrors, then row 0
+// into 1 and 2 into 3, then 1 into 3; a fixed order, about a fifth of
+// wave_sum's latency, which counts where nothing else runs meanwhile.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double lane_moved(double v) {
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, (uint32_t)b, CTRL, ROWS, 0xf, false);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, (uint32_t)(b >> 32), CTRL, ROWS, 0xf, false);
+  return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+__device__ __forceinline__ double wave_total(double v) {
+  v += lane_moved<0xB1, 0xf>(v);   // quad_perm [1,0,3,2]
+  v += lane_moved<0x4E, 0xf>(v);   // quad_perm [2,3,0,1]
+  v += lane_moved<0x141, 0xf>(v);  // row_half_mirror
+  v += lane_moved<0x140, 0xf>(v);  // row_mirror
+  v += lane_moved<0x142, 0xa>(v);  // row_bcast15 into rows 1 and 3
+  v += lane_moved<0x143, 0xc>(v);  // row_bcast31 into rows 2 and 3
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)b, 63);
+  const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(b >> 32), 63);
+  return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+
+// One thread of a workgroup: its NV partial sums into slots[wg].
+template <int NV>
+__device__ __forceinline__ void grid_publish(uint64_t* slots, int wg,
+                                             uint32_t tag,
+                                             const double (&v)[NV]) {
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+    grid_put(slots + ((int64_t)wg * NV + j) * 2, tag, v[j]);
+}
+
+// Every thread of a workgroup: the sums over the nwg slots of this tag, the
+// same value in every thread of every workgroup (blockDim.x, a multiple of
+// 64, must be the same in all).  sh: NV doubles per wave of the workgroup;
+// *fail: a shared int that is 0, set if a wait was given up.  Returns false
+// (in every thread) in that case.  sh may be written again after the next
+// workgroup barrier.
+template <int NV>
+__device__ __forceinline__ bool grid_sum(const uint64_t* slots, int nwg,
+                                         uint32_t tag, double* sh, int* fail,
+                                         double (&out)[NV]) {
+  double v[NV];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) v[j] = 0.0;
+  for (int q = threadIdx.x; q < nwg; q += blockDim.x) {
+    const uint64_t* s[NV];
+    double p[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) s[j] = slots + ((int64_t)q * NV + j) * 2;
+    grid_get<NV>(s, NV, tag, fail, p);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) v[j] += p[j];
+  }
+  const int wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    v[j] = wave_total(v[j]);
+    if ((threadIdx.x & 63) == 0) sh[wv * NV + j] = v[j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NV; ++j) out[j] = 0.0;
+  for (int k = 0; k < nw; ++k)
+#pragma unroll
+    for (int j = 0; j < NV; ++j) out[j] += sh[k * NV + j];
+  return *fail == 0;
+}
+
+}  // namespace nekoamd

@@ -66,6 +66,7 @@ struct GsMap {
   double* avg_binv = nullptr;  // one per group, buckets in order
   int64_t goff[NEKOAMD_GS_MAX_MULT] = {};
   const void* avg_key[2] = {nullptr, nullptr};
+  int2* ref = nullptr;  // per point, see gs_point_refs
 };
 
 template <int OP, typename T>
@@ -491,6 +492,40 @@ template int gs_launch3<double>(void*, double* const*, int, const int* const*,
 template int gs_launch3<float>(void*, float* const*, int, const int* const*,
                                const bool*);
 
+// ref[l] = {off + t m, m} for the members l of tuple t of one bucket.
+__global__ void __launch_bounds__(256)
+    gs_ref_k(int64_t nocc, int m, int64_t off, const int32_t* __restrict__ idx,
+             int2* __restrict__ ref) {
+  for (int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x; k < nocc;
+       k += (int64_t)gridDim.x * 256)
+    ref[idx[off + k]] = make_int2((int)(off + k / m * m), m);
+}
+
+int gs_point_refs(void* gs, int maxm, const int2** ref, const int32_t** idx,
+                  bool* ok) {
+  GsMap* g = (GsMap*)gs;
+  if (!g) return fail_arg("gs_point_refs", "null gs handle");
+  *ok = g->n > 0 && g->dev_len <= INT32_MAX;
+  for (int b = 0; b < g->nb; ++b) *ok = *ok && g->m[b] <= maxm;
+  if (!*ok) return kOk;
+  if (!g->ref) {
+    int2* r = nullptr;
+    NK_HIP(hipMalloc((void**)&r, sizeof(int2) * g->n));
+    g->ref = r;
+    NK_HIP(hipMemsetAsync(r, 0, sizeof(int2) * g->n, stream()));
+    for (int b = 0; b < g->nb; ++b) {
+      const int64_t nocc = g->cnt[b] * g->m[b];
+      if (nocc == 0) continue;
+      hipLaunchKernelGGL(gs_ref_k, dim3(nk_grid(nocc, 256)), dim3(256), 0,
+                         stream(), nocc, g->m[b], g->dev_off[b], g->idx_d, r);
+      NK_LAUNCHED();
+    }
+  }
+  *ref = g->ref;
+  *idx = g->idx_d;
+  return kOk;
+}
+
 // Local points per group of the launch layout, and CUs per XCD on gfx950
 // (MI355X: 256 CUs in 8 XCDs).
 constexpr int64_t kBlkGroup = 8192;
@@ -600,6 +635,7 @@ static void free_map(GsMap* g) {
   if (g->avg_binv) (void)hipFree(g->avg_binv);
   if (g->avg_bb) (void)hipFree(g->avg_bb);
   if (g->avg_binvb) (void)hipFree(g->avg_binvb);
+  if (g->ref) (void)hipFree(g->ref);
   delete g;
 }
 

@@ -504,3 +504,62 @@ def test_cg_solve3_matches_separate_solves(cases, key, sem):
         assert rel_max(xg, sep[c]) < 1e-7
         assert rel_max(xg, x_ref) < 1e-6
         assert np.all(xg[mask] == 0.0)
+
+
+@pytest.mark.parametrize("box", [(1, 1, 1, 4), (7, 5, 3, 4), (13, 11, 9, 4), (3, 1, 1, 5),
+                                 (9, 8, 8, 5), (3, 3, 3, 6), (7, 7, 6, 6), (2, 2, 2, 7),
+                                 (8, 8, 4, 8), (2, 2, 2, 9)])
+@pytest.mark.parametrize("ifh2", [False, True])
+def test_cg_small_meshes(box, ifh2, sem):
+    """The FP64 PCG of meshes that fit one kernel: one element, element counts
+    that leave a workgroup part empty, more than 256 workgroups' worth of
+    elements at the smaller packing, 256 workgroups exactly, and an order
+    outside its range.  The same iterates as the oracle's: a fixed number of
+    iterations to the rounding of the sums, and a converged solve within an
+    iteration."""
+    nx, ny, nz, lx = box
+    g = sem.BoxCase(nx, ny, nz, lx, jitter=0.05, seed=1234)
+    o = oracle.build_case(nx, ny, nz, lx, jitter=0.05, seed=1234)
+    rng = np.random.default_rng(lx + nx)
+    faces = sem.VEL_DIRICHLET if ifh2 else sem.PRS_DIRICHLET
+    mask = oracle.face_mask(nx, ny, nz, lx, faces)
+    h1 = np.full(o.n, 0.01 if ifh2 else 1.0)
+    h2 = o.gs(rng.uniform(10.0, 500.0, o.n)) if ifh2 else None
+    f = o.gs(o.B * rng.uniform(-1, 1, o.n))
+    f[mask] = 0.0
+    h1d, h2d = g.field(h1), g.field(h2) if ifh2 else None
+    d = g.field()
+    g.jacobi(d, h1d, h2d, ifh2)
+    cg, x = sem.CG(g), g.field()
+    for abstol, max_iter in ((0.0, 4), (1e-9, 3000)):
+        ref, it, r0, r1 = o.cg(f, mask, h1, h2, ifh2, abstol=abstol, max_iter=max_iter)
+        mon = cg.solve(x, g.field(f), d, g.mask(faces), h1d, h2d, ifh2, abstol=abstol,
+                       max_iter=max_iter)
+        assert abs(mon.res_start - r0) <= 1e-12 * r0
+        if abstol == 0.0:
+            # four iterations: sums of up to 1e5 terms, each of eps relative
+            assert mon.iter == it == 4
+            assert abs(mon.res_final - r1) <= 1e-9 * r0
+            assert np.abs(x.get() - ref).max() <= 1e-9 * np.abs(ref).max()
+        else:
+            assert abs(mon.iter - it) <= 1 and mon.res_final < abstol and mon.done == 1
+            assert np.abs(x.get() - ref).max() <= 1e-5 * np.abs(ref).max()
+
+
+def test_cg_small_mesh_over_many_iterations(sem):
+    """More iterations than one launch takes: the solve goes on from the
+    stored state, and x stays at the converged solution."""
+    box = (8, 8, 4, 4)
+    g = sem.BoxCase(*box, jitter=0.05, seed=1234)
+    o = oracle.build_case(*box, jitter=0.05, seed=1234)
+    mask = oracle.face_mask(*box, sem.PRS_DIRICHLET)
+    f = o.gs(o.B * np.random.default_rng(3).uniform(-1, 1, o.n))
+    f[mask] = 0.0
+    h1, d = g.field(np.ones(g.n)), g.field()
+    g.jacobi(d, h1)
+    x = g.field()
+    mon = sem.CG(g).solve(x, g.field(f), d, g.mask(sem.PRS_DIRICHLET), h1, abstol=0.0,
+                          max_iter=2100)
+    ref = o.cg(f, mask, abstol=1e-12, max_iter=2000)[0]
+    assert mon.iter == 2100
+    assert np.abs(x.get() - ref).max() <= 1e-9 * np.abs(ref).max()
