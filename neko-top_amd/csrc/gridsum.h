@@ -35,6 +35,11 @@ __device__ __forceinline__ void dev_store(T* p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// The calling thread's earlier dev_stores have reached the device's memory.
+__device__ __forceinline__ void dev_stores_done() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 __device__ __forceinline__ void grid_put(uint64_t* s, uint32_t tag, double v) {
   const uint64_t hi = (uint64_t)tag << 32;
   const uint64_t b = (uint64_t)__double_as_longlong(v);

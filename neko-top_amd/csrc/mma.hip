@@ -9,11 +9,21 @@
 // zeta, the (m+1)x(m+1) Newton system) live on the host, which is where the
 // reference's MPI_Allreduce calls would hand them over anyway.
 //
-// Per Newton step the device makes four passes over the n variables:
-//   newton : delx, diagx and the reductions g_i, bb_i, AA_ik
-//   dir    : dx, dxsi, deta, the step-length bound and the line-search copy
-//   step   : x, xsi, eta at the trial step and the residual reductions
-//            (repeated while the backtracking line search halves the step)
+// Per Newton step the device makes two passes over the n variables:
+//   dir  : the search direction's step-length bound
+//   eval : the trial point at that step, its residual and the pieces of the
+//          Newton system there (repeated while the backtracking line search
+//          halves the step; the accepted trial's pieces are the next step's)
+// Both are bound by HBM: they read the 9 + 2 m vectors that define the
+// subproblem and the iterate, and recompute the direction from them instead
+// of storing it (delx, diagx, dx, dxsi, deta and the line search's copies
+// were 22 of the 47 vector streams of a step in three passes: newton, dir,
+// trial).  At n = 4.2 M, m = 1 dir takes 65 us and eval 84 us (5.7 TB/s)
+// where the three passes took 86, 96 and 118 us and each a finalise launch
+// and a copy; three updates 40.0 -> 20.4 ms, at n = 20000 (bound by the host
+// reads, one per trial) 62 -> 46 ms.  Successive passes run through the
+// variables in opposite directions, so a pass begins on what the one before
+// left in the 256 MB cache behind the L2s (23.9 ms all in one direction).
 // Reductions are deterministic (fixed trees); sums and maxima come back in one
 // read per pass.  The reference's default-real literals (0.01, 0.1, 0.9,
 // 1.01 in single precision) are kept.  m is a template parameter (1..4).
@@ -21,6 +31,7 @@
 #include <cstring>
 #include <vector>
 
+#include "gridsum.h"
 #include "internal.h"
 #include "nekoamd.h"
 #include "reduce.h"
@@ -33,16 +44,19 @@ namespace nekoamd {
 #define MMA_F1_01 ((double)1.01f)
 
 constexpr int kMmaMaxM = 4;
-constexpr int kMB = 256;        // threads per block of an n-pass
-constexpr int kMG = 1024;       // max blocks (partials per value)
+// Threads per block of an n-pass and most blocks (partials per value): 16
+// waves per CU, in few blocks, since each counts itself done at one address;
+// the last block has a thread for every partial.
+constexpr int kMB = 512;
+constexpr int kMG = 512;
 constexpr int kMaxVals = 2 + 2 * kMmaMaxM + kMmaMaxM * kMmaMaxM;
 
 struct MmaVec {
   int64_t n;
   double *x, *xsi, *eta, *low, *upp, *alpha, *beta, *xmin, *xmax, *p0j, *q0j;
   double *pij, *qij;  // [i*n + j]
-  double *xold1, *xold2, *dx, *dxsi, *deta, *xold, *xsiold, *etaold, *delx,
-      *diagx;
+  double *xold1, *xold2;
+  double *xt, *xsit, *etat;  // the trial point; swapped with x, xsi, eta
 };
 
 struct MmaState {
@@ -52,8 +66,12 @@ struct MmaState {
   std::vector<double> a, c, d, bi, y, lambda, s, mu;
   MmaVec v{};
   double* mem = nullptr;   // one device block for all vectors
-  double* part = nullptr;  // kMaxVals * kMG partials + kMaxVals results
-  double* hres = nullptr;  // pinned read-back
+  double* part = nullptr;  // kMaxVals * kMG partials
+  int* count = nullptr;    // workgroups of the running pass that are done
+  bool down = false;       // direction of the next pass over the variables
+  double* bound = nullptr; // the direction pass's result
+  // pinned: the last evaluation's results, then the direction pass's
+  double* hres = nullptr;
   int newton_iters = 0;    // diagnostics of the last update
 };
 
@@ -64,12 +82,27 @@ __device__ __forceinline__ double wave_max(double v) {
   return v;
 }
 
-// Reduce K per-thread values over the block; ismax bit v selects max for
-// value v, else sum.  Writes part[v*gridDim.x + blockIdx.x].
+// Where a pass's reductions go: block partials, the count of finished
+// blocks (0 between passes), and the pinned host memory of the results; dev
+// (may be null): the first result for the next pass.
+struct MmaOut {
+  double* part;
+  int* count;
+  double* host;
+  double* dev;
+};
+
+// Reduce K per-thread values over the grid; ismax bit v selects max for
+// value v, else sum.  Every block stores its partials past its L2 (device
+// scope) and waits for those stores before it counts itself done; the last
+// one to do so sums them all, in an order that does not depend on which
+// block that is, and writes the results to the host's memory.  (A fence in
+// their place writes back the whole L2 in every block: 75 us more a pass.)
 template <int K>
-__device__ __forceinline__ void block_out(double (&acc)[K], unsigned ismax,
-                                          double* __restrict__ part) {
+__device__ __forceinline__ void grid_out(double (&acc)[K], unsigned ismax,
+                                         const MmaOut& o) {
   __shared__ double sh[K][kMB / 64];
+  __shared__ int last;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
   for (int v = 0; v < K; ++v) {
@@ -82,30 +115,38 @@ __device__ __forceinline__ void block_out(double (&acc)[K], unsigned ismax,
     double r = sh[v][0];
     for (int q = 1; q < kMB / 64; ++q)
       r = (ismax >> v) & 1u ? fmax(r, sh[v][q]) : r + sh[v][q];
-    part[(int64_t)v * gridDim.x + blockIdx.x] = r;
+    dev_store(o.part + (int64_t)v * gridDim.x + blockIdx.x, r);
+    dev_stores_done();
   }
-}
-
-__global__ void __launch_bounds__(kFinBlock)
-    mma_fin_k(const double* __restrict__ part, int np, unsigned ismax,
-              double* __restrict__ out) {
-  __shared__ double sh[kFinBlock / 64];
-  const int v = blockIdx.x;
-  const bool mx = (ismax >> v) & 1u;
-  double r = 0.0;
-  for (int q = threadIdx.x; q < np; q += kFinBlock) {
-    const double p = part[(int64_t)v * np + q];
-    r = mx ? fmax(r, p) : r + p;
-  }
-  r = mx ? wave_max(r) : wave_sum(r);
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  if (lane == 0) sh[wv] = r;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double a = sh[0];
-    for (int q = 1; q < kFinBlock / 64; ++q) a = mx ? fmax(a, sh[q]) : a + sh[q];
-    out[v] = a;
+  if (threadIdx.x == 0)
+    last = __hip_atomic_fetch_add(o.count, 1, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT) ==
+           (int)gridDim.x - 1;
+  __syncthreads();
+  if (!last) return;
+  static_assert(kMG <= kMB, "one partial per thread");
+  const bool in = threadIdx.x < gridDim.x;
+  double p[K];
+#pragma unroll
+  for (int v = 0; v < K; ++v)
+    p[v] = in ? dev_load(o.part + (int64_t)v * gridDim.x + threadIdx.x) : 0.0;
+#pragma unroll
+  for (int v = 0; v < K; ++v) {
+    // maxima are of absolute values or at least 1
+    const double r = (ismax >> v) & 1u ? wave_max(p[v]) : wave_sum(p[v]);
+    if (lane == 0) sh[v][wv] = r;
   }
+  __syncthreads();
+  if (threadIdx.x < K) {
+    const int v = threadIdx.x;
+    double r = sh[v][0];
+    for (int q = 1; q < kMB / 64; ++q)
+      r = (ismax >> v) & 1u ? fmax(r, sh[v][q]) : r + sh[v][q];
+    o.host[v] = r;
+    if (v == 0 && o.dev != nullptr) *o.dev = r;
+  }
+  if (threadIdx.x == 0) dev_store(o.count, 0);
 }
 
 // ---- per-variable kernels --------------------------------------------------
@@ -114,7 +155,7 @@ __global__ void __launch_bounds__(kMB)
     gensub_k(MmaVec V, const double* __restrict__ xd,
              const double* __restrict__ df0dx, const double* __restrict__ dfdx,
              int early, double asyinit, double asyincr, double asydecr,
-             double* __restrict__ part) {
+             MmaOut out) {
   double acc[M];
 #pragma unroll
   for (int i = 0; i < M; ++i) acc[i] = 0.0;
@@ -164,7 +205,7 @@ __global__ void __launch_bounds__(kMB)
       acc[i] = acc[i] + p / (up - x) + q / (x - lo);
     }
   }
-  block_out<M>(acc, 0u, part);
+  grid_out<M>(acc, 0u, out);
 }
 
 template <int M>
@@ -182,120 +223,149 @@ struct Lam {
   double v[kMmaMaxM];
 };
 
-// Residual pieces at (x, xsi, eta); with STEP, first x = xold + steg dx etc.
-// Values: [sum of rex^2+rexsi^2+reeta^2, max |.|, g_0..g_{M-1}].
-template <int M, bool STEP>
-__global__ void __launch_bounds__(kMB)
-    resid_k(MmaVec V, Lam lam, double epsi, double steg,
-            double* __restrict__ part) {
-  double acc[2 + M];
+// The vectors a pass reads, for variable j.
+template <int M>
+struct MmaVar {
+  double x, xsi, eta, low, upp, alpha, beta, p0, q0, p[M], q[M];
+  __device__ __forceinline__ MmaVar(const MmaVec& V, int64_t j)
+      : x(V.x[j]), xsi(V.xsi[j]), eta(V.eta[j]), low(V.low[j]), upp(V.upp[j]),
+        alpha(V.alpha[j]), beta(V.beta[j]), p0(V.p0j[j]), q0(V.q0j[j]) {
 #pragma unroll
-  for (int q = 0; q < 2 + M; ++q) acc[q] = 0.0;
-  for (int64_t j = (int64_t)blockIdx.x * kMB + threadIdx.x; j < V.n;
-       j += (int64_t)gridDim.x * kMB) {
-    double x, xsi, eta;
-    if constexpr (STEP) {
-      x = V.xold[j] + steg * V.dx[j];
-      xsi = V.xsiold[j] + steg * V.dxsi[j];
-      eta = V.etaold[j] + steg * V.deta[j];
-      V.x[j] = x;
-      V.xsi[j] = xsi;
-      V.eta[j] = eta;
-    } else {
-      x = V.x[j];
-      xsi = V.xsi[j];
-      eta = V.eta[j];
+    for (int i = 0; i < M; ++i) {
+      p[i] = V.pij[(int64_t)i * V.n + j];
+      q[i] = V.qij[(int64_t)i * V.n + j];
     }
-    const double ux = V.upp[j] - x, xl = x - V.low[j];
+  }
+};
+
+// One variable's part of the Newton system at (x, xsi, eta): the distances
+// to the asymptotes and bounds and their reciprocals, the gradients GG_i of
+// the constraints, and delx and 1/diagx.
+template <int M>
+struct MmaNewton {
+  double xa, bx, iu, il, ia, ib, GG[M], delx, inv, dpsi;
+  __device__ __forceinline__ MmaNewton(const MmaVar<M>& v, double x, double xsi,
+                                       double eta, const Lam& lam, double epsi) {
+    const double ux = v.upp - x, xl = x - v.low;
+    xa = x - v.alpha;
+    bx = v.beta - x;
+    iu = 1.0 / ux;
+    il = 1.0 / xl;
+    ia = 1.0 / xa;
+    ib = 1.0 / bx;
+    const double iu2 = iu * iu, il2 = il * il;
     double pl = 0.0, ql = 0.0;
 #pragma unroll
     for (int i = 0; i < M; ++i) {
-      const double p = V.pij[(int64_t)i * V.n + j], q = V.qij[(int64_t)i * V.n + j];
-      pl += p * lam.v[i];
-      ql += q * lam.v[i];
-      acc[2 + i] = acc[2 + i] + p / ux + q / xl;
+      pl += v.p[i] * lam.v[i];
+      ql += v.q[i] * lam.v[i];
+      GG[i] = v.p[i] * iu2 - v.q[i] * il2;
     }
-    pl = V.p0j[j] + pl;
-    ql = V.q0j[j] + ql;
-    const double rex = (pl / (ux * ux) - ql / (xl * xl)) - xsi + eta;
-    const double rexsi = xsi * (x - V.alpha[j]) - epsi;
-    const double reeta = eta * (V.beta[j] - x) - epsi;
-    acc[0] += rex * rex + rexsi * rexsi + reeta * reeta;
-    acc[1] = fmax(acc[1], fmax(fabs(rex), fmax(fabs(rexsi), fabs(reeta))));
+    pl = v.p0 + pl;
+    ql = v.q0 + ql;
+    dpsi = pl * iu2 - ql * il2;
+    delx = dpsi - epsi * ia + epsi * ib;
+    inv = 1.0 / (2.0 * (pl * iu2 * iu + ql * il2 * il) + xsi * ia + eta * ib);
   }
-  block_out<2 + M>(acc, 2u, part);
+};
+
+// The search direction of one variable for the multipliers' dlam.
+template <int M>
+__device__ __forceinline__ void mma_dir(const MmaNewton<M>& w, double xsi,
+                                        double eta, const Lam& dlam,
+                                        double epsi, double& dx, double& dxsi,
+                                        double& deta) {
+  double gl = 0.0;
+#pragma unroll
+  for (int i = 0; i < M; ++i) gl += w.GG[i] * dlam.v[i];
+  dx = -(w.delx + gl) * w.inv;
+  dxsi = -xsi + (epsi - dx * xsi) * w.ia;
+  deta = -eta + (epsi + dx * eta) * w.ib;
 }
 
-// Newton system pieces.  Values: [g_i (M), bb_i (M), AA_ik (M*M)].
-template <int M>
-__global__ void __launch_bounds__(kMB)
-    newton_k(MmaVec V, Lam lam, double epsi, double* __restrict__ part) {
-  double acc[2 * M + M * M];
-#pragma unroll
-  for (int q = 0; q < 2 * M + M * M; ++q) acc[q] = 0.0;
-  for (int64_t j = (int64_t)blockIdx.x * kMB + threadIdx.x; j < V.n;
-       j += (int64_t)gridDim.x * kMB) {
-    const double x = V.x[j], ux = V.upp[j] - x, xl = x - V.low[j];
-    const double xa = x - V.alpha[j], bx = V.beta[j] - x;
-    double a = 0.0, pl = 0.0, ql = 0.0, GG[M];
-#pragma unroll
-    for (int i = 0; i < M; ++i) {
-      const double p = V.pij[(int64_t)i * V.n + j], q = V.qij[(int64_t)i * V.n + j];
-      a = a + p * lam.v[i] / (ux * ux) - q * lam.v[i] / (xl * xl);
-      pl += p * lam.v[i];
-      ql += q * lam.v[i];
-      GG[i] = p / (ux * ux) - q / (xl * xl);
-      acc[i] = acc[i] + p / ux + q / xl;
-    }
-    const double delx = a + V.p0j[j] / (ux * ux) - V.q0j[j] / (xl * xl) -
-                        epsi / xa + epsi / bx;
-    const double dg = (V.p0j[j] + pl) / (ux * ux * ux) + (V.q0j[j] + ql) / (xl * xl * xl);
-    const double diagx = 2.0 * dg + V.xsi[j] / xa + V.eta[j] / bx;
-    V.delx[j] = delx;
-    V.diagx[j] = diagx;
-    const double r = delx / diagx, inv = 1.0 / diagx;
-#pragma unroll
-    for (int i = 0; i < M; ++i) {
-      acc[M + i] = acc[M + i] + GG[i] * r;
-#pragma unroll
-      for (int k = 0; k < M; ++k)
-        acc[2 * M + i * M + k] = acc[2 * M + i * M + k] + GG[i] * inv * GG[k];
-    }
-  }
-  block_out<2 * M + M * M>(acc, 0u, part);
+// Variable of pass step k of this thread: upwards, or the same ones in the
+// opposite order.
+__device__ __forceinline__ int64_t pass_var(int64_t n, int64_t k, bool down) {
+  const int64_t j = k + (int64_t)blockIdx.x * kMB + threadIdx.x;
+  return down ? n - 1 - j : j;
 }
 
-// Search direction for x, xsi, eta; saves the line-search origin.
-// Value: the largest step-length bound (max).
-template <int M>
+// Residual and Newton system pieces at (x, xsi, eta) and lam; with STEP at
+// the trial point x + steg dx etc. (the direction of lam, dlam there), which
+// it stores, and lam + steg dlam.  bound (may be null): the direction pass's
+// result, from which steg is taken as the host takes it (steg then holds the
+// bound of the host's own unknowns); so the first trial is queued behind the
+// direction pass without a host read between them.
+// Values: [sum of rex^2+rexsi^2+reeta^2, max |.|, g_i (M), bb_i (M),
+// AA_ik (M*M)].
+template <int M, bool STEP>
 __global__ void __launch_bounds__(kMB)
-    dir_k(MmaVec V, Lam dlam, double epsi, double* __restrict__ part) {
-  double acc[1] = {1.0};
-  for (int64_t j = (int64_t)blockIdx.x * kMB + threadIdx.x; j < V.n;
-       j += (int64_t)gridDim.x * kMB) {
-    const double x = V.x[j], ux = V.upp[j] - x, xl = x - V.low[j];
-    const double xa = x - V.alpha[j], bx = V.beta[j] - x;
-    const double xsi = V.xsi[j], eta = V.eta[j], diagx = V.diagx[j];
-    double gl = 0.0;
+    eval_k(MmaVec V, Lam lam, Lam dlam, double epsi, double steg,
+           const double* __restrict__ bound, bool down, MmaOut out) {
+  constexpr int K = 2 + 2 * M + M * M;
+  Lam laml = lam;
+  if constexpr (STEP) {
+    if (bound != nullptr) steg = 1.0 / fmax(*bound, steg);
 #pragma unroll
     for (int i = 0; i < M; ++i)
-      gl += (V.pij[(int64_t)i * V.n + j] / (ux * ux) -
-             V.qij[(int64_t)i * V.n + j] / (xl * xl)) * dlam.v[i];
-    const double dx = -V.delx[j] / diagx - gl / diagx;
-    const double dxsi = -xsi + (epsi - dx * xsi) / xa;
-    const double deta = -eta + (epsi + dx * eta) / bx;
-    V.dx[j] = dx;
-    V.dxsi[j] = dxsi;
-    V.deta[j] = deta;
-    V.xold[j] = x;
-    V.xsiold[j] = xsi;
-    V.etaold[j] = eta;
-    double b = fmax(-(MMA_F1_01 * dxsi / xsi), -(MMA_F1_01 * deta / eta));
-    b = fmax(b, -(MMA_F1_01 * dx / xa));
-    b = fmax(b, MMA_F1_01 * dx / bx);
+      laml.v[i] = __dadd_rn(lam.v[i], __dmul_rn(steg, dlam.v[i]));
+  }
+  double acc[K];
+#pragma unroll
+  for (int q = 0; q < K; ++q) acc[q] = 0.0;
+  for (int64_t k = 0; k < V.n; k += (int64_t)gridDim.x * kMB) {
+    const int64_t j = pass_var(V.n, k, down);
+    if (j < 0 || j >= V.n) break;
+    const MmaVar<M> v(V, j);
+    double x = v.x, xsi = v.xsi, eta = v.eta;
+    if constexpr (STEP) {
+      const MmaNewton<M> o(v, x, xsi, eta, lam, epsi);
+      double dx, dxsi, deta;
+      mma_dir<M>(o, xsi, eta, dlam, epsi, dx, dxsi, deta);
+      x = x + steg * dx;
+      xsi = xsi + steg * dxsi;
+      eta = eta + steg * deta;
+      V.xt[j] = x;
+      V.xsit[j] = xsi;
+      V.etat[j] = eta;
+    }
+    const MmaNewton<M> w(v, x, xsi, eta, laml, epsi);
+    const double rex = w.dpsi - xsi + eta;
+    const double rexsi = xsi * w.xa - epsi;
+    const double reeta = eta * w.bx - epsi;
+    acc[0] += rex * rex + rexsi * rexsi + reeta * reeta;
+    acc[1] = fmax(acc[1], fmax(fabs(rex), fmax(fabs(rexsi), fabs(reeta))));
+    const double r = w.delx * w.inv;
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      acc[2 + i] += v.p[i] * w.iu + v.q[i] * w.il;
+      acc[2 + M + i] += w.GG[i] * r;
+#pragma unroll
+      for (int q = 0; q < M; ++q)
+        acc[2 + 2 * M + i * M + q] += w.GG[i] * w.inv * w.GG[q];
+    }
+  }
+  grid_out<K>(acc, 2u, out);
+}
+
+// Value: the search direction's largest step-length bound (max).
+template <int M>
+__global__ void __launch_bounds__(kMB)
+    dir_k(MmaVec V, Lam lam, Lam dlam, double epsi, bool down, MmaOut out) {
+  double acc[1] = {1.0};
+  for (int64_t k = 0; k < V.n; k += (int64_t)gridDim.x * kMB) {
+    const int64_t j = pass_var(V.n, k, down);
+    if (j < 0 || j >= V.n) break;
+    const MmaVar<M> v(V, j);
+    const MmaNewton<M> w(v, v.x, v.xsi, v.eta, lam, epsi);
+    double dx, dxsi, deta;
+    mma_dir<M>(w, v.xsi, v.eta, dlam, epsi, dx, dxsi, deta);
+    double b = fmax(-(MMA_F1_01 * dxsi / v.xsi), -(MMA_F1_01 * deta / v.eta));
+    b = fmax(b, -(MMA_F1_01 * dx * w.ia));
+    b = fmax(b, MMA_F1_01 * dx * w.ib);
     acc[0] = fmax(acc[0], b);
   }
-  block_out<1>(acc, 1u, part);
+  grid_out<1>(acc, 1u, out);
 }
 
 // KKT pieces at the design x.  Values: [sum of squares, max |.|].
@@ -303,7 +373,7 @@ template <int M>
 __global__ void __launch_bounds__(kMB)
     kkt_k(MmaVec V, Lam lam, const double* __restrict__ xd,
           const double* __restrict__ df0dx, const double* __restrict__ dfdx,
-          double* __restrict__ part) {
+          MmaOut out) {
   double acc[2] = {0.0, 0.0};
   for (int64_t j = (int64_t)blockIdx.x * kMB + threadIdx.x; j < V.n;
        j += (int64_t)gridDim.x * kMB) {
@@ -317,24 +387,32 @@ __global__ void __launch_bounds__(kMB)
     acc[0] += rex * rex + rexsi * rexsi + reeta * reeta;
     acc[1] = fmax(acc[1], fmax(fabs(rex), fmax(fabs(rexsi), fabs(reeta))));
   }
-  block_out<2>(acc, 2u, part);
+  grid_out<2>(acc, 2u, out);
 }
 
 // ---- host side -------------------------------------------------------------
 static int mma_grid(int64_t n) { return nk_grid(n, kMB, kMG); }
 
-static int finish(MmaState* S, int nvals, int grid, unsigned ismax,
-                  double* out) {
+static MmaOut mma_out(MmaState* S) {
+  return {S->part, S->count, S->hres, nullptr};
+}
+
+// The results of the pass just launched.
+static int finish(MmaState* S, int nvals, double* out) {
   NK_LAUNCHED();
-  hipLaunchKernelGGL(mma_fin_k, dim3(nvals), dim3(kFinBlock), 0, stream(),
-                     S->part, grid, ismax, S->part + kMaxVals * kMG);
-  NK_LAUNCHED();
-  NK_HIP(hipMemcpyAsync(S->hres, S->part + kMaxVals * kMG,
-                        sizeof(double) * nvals, hipMemcpyDeviceToHost,
-                        stream()));
   NK_HIP(hipStreamSynchronize(stream()));
   std::memcpy(out, S->hres, sizeof(double) * nvals);
   return kOk;
+}
+
+template <int M, bool STEP>
+static int evaluate(MmaState* S, int grid, const Lam& lam, const Lam& dlam,
+                    double epsi, double steg, const double* bound,
+                    double* out) {
+  hipLaunchKernelGGL((eval_k<M, STEP>), dim3(grid), dim3(kMB), 0, stream(),
+                     S->v, lam, dlam, epsi, steg, bound, S->down, mma_out(S));
+  S->down = !S->down;
+  return finish(S, 2 + 2 * M + M * M, out);
 }
 
 // Gaussian elimination with row partial pivoting (DGESV semantics),
@@ -404,8 +482,8 @@ static int mma_update_t(MmaState* S, int iter, double* xd, const double* df0dx,
   // ---- gensub
   hipLaunchKernelGGL((gensub_k<M>), dim3(grid), dim3(kMB), 0, stream(), V, xd,
                      df0dx, dfdx, iter < 3 ? 1 : 0, S->asyinit, S->asyincr,
-                     S->asydecr, S->part);
-  int rc = finish(S, M, grid, 0u, out);
+                     S->asydecr, mma_out(S));
+  int rc = finish(S, M, out);
   if (rc) return rc;
   for (int i = 0; i < M; ++i) S->bi[i] = out[i] - fval[i];
   // ---- subsolve
@@ -423,9 +501,7 @@ static int mma_update_t(MmaState* S, int iter, double* xd, const double* df0dx,
   while (epsi > MMA_F0_9 * S->epsimin) {
     Lam L{};
     for (int i = 0; i < M; ++i) L.v[i] = lam[i];
-    hipLaunchKernelGGL((resid_k<M, false>), dim3(grid), dim3(kMB), 0, stream(),
-                       V, L, epsi, 0.0, S->part);
-    rc = finish(S, 2 + M, grid, 2u, out);
+    rc = evaluate<M, false>(S, grid, L, L, epsi, 0.0, nullptr, out);
     if (rc) return rc;
     Small sm = small_resid(S, out + 2, y, z, lam, mu, zeta, s, epsi);
     double residumax = std::fmax(out[1], sm.max);
@@ -434,13 +510,10 @@ static int mma_update_t(MmaState* S, int iter, double* xd, const double* df0dx,
       if (residumax < epsi) break;
       ++S->newton_iters;
       for (int i = 0; i < M; ++i) L.v[i] = lam[i];
-      hipLaunchKernelGGL((newton_k<M>), dim3(grid), dim3(kMB), 0, stream(), V,
-                         L, epsi, S->part);
-      rc = finish(S, 2 * M + M * M, grid, 0u, out);
-      if (rc) return rc;
-      const double* g = out;
-      const double* bbs = out + M;
-      const double* AAs = out + 2 * M;
+      // the pieces of the last evaluation, which was at this point
+      const double* g = out + 2;
+      const double* bbs = out + 2 + M;
+      const double* AAs = out + 2 + 2 * M;
       double la = 0.0;
       for (int i = 0; i < M; ++i) la += lam[i] * S->a[i];
       const double delz = S->a0 - la - epsi / z;
@@ -476,11 +549,14 @@ static int mma_update_t(MmaState* S, int iter, double* xd, const double* df0dx,
       const double dzeta = -zeta + (epsi - zeta * dz) / z;
       Lam DL{};
       for (int i = 0; i < M; ++i) DL.v[i] = dlam[i];
-      hipLaunchKernelGGL((dir_k<M>), dim3(grid), dim3(kMB), 0, stream(), V, DL,
-                         epsi, S->part);
-      rc = finish(S, 1, grid, 1u, out);
-      if (rc) return rc;
-      double steg = out[0];
+      MmaOut dout = mma_out(S);
+      dout.host = S->hres + kMaxVals;
+      dout.dev = S->bound;
+      hipLaunchKernelGGL((dir_k<M>), dim3(grid), dim3(kMB), 0, stream(), V, L,
+                         DL, epsi, S->down, dout);
+      S->down = !S->down;
+      NK_LAUNCHED();
+      double steg = 1.0;
       for (int i = 0; i < M; ++i) {
         steg = std::fmax(steg, -(MMA_F1_01 * dy[i] / y[i]));
         steg = std::fmax(steg, -(MMA_F1_01 * dlam[i] / lam[i]));
@@ -489,7 +565,6 @@ static int mma_update_t(MmaState* S, int iter, double* xd, const double* df0dx,
       }
       steg = std::fmax(steg, -(MMA_F1_01 * dz / z));
       steg = std::fmax(steg, -(MMA_F1_01 * dzeta / zeta));
-      steg = 1.0 / steg;
       double yo[M], lo[M], so[M], muo[M];
       std::memcpy(yo, y, sizeof(y));
       std::memcpy(lo, lam, sizeof(lam));
@@ -500,6 +575,10 @@ static int mma_update_t(MmaState* S, int iter, double* xd, const double* df0dx,
       int itto = 0;
       while (newresidu > residunorm && itto < 50) {
         ++itto;
+        rc = evaluate<M, true>(S, grid, L, DL, epsi, steg,
+                               itto == 1 ? S->bound : nullptr, out);
+        if (rc) return rc;
+        if (itto == 1) steg = 1.0 / std::fmax(S->hres[kMaxVals], steg);
         for (int i = 0; i < M; ++i) {
           y[i] = yo[i] + steg * dy[i];
           lam[i] = lo[i] + steg * dlam[i];
@@ -508,16 +587,15 @@ static int mma_update_t(MmaState* S, int iter, double* xd, const double* df0dx,
         }
         z = zo + steg * dz;
         zeta = zetao + steg * dzeta;
-        for (int i = 0; i < M; ++i) L.v[i] = lam[i];
-        hipLaunchKernelGGL((resid_k<M, true>), dim3(grid), dim3(kMB), 0,
-                           stream(), V, L, epsi, steg, S->part);
-        rc = finish(S, 2 + M, grid, 2u, out);
-        if (rc) return rc;
         sm = small_resid(S, out + 2, y, z, lam, mu, zeta, s, epsi);
         newresidu = std::sqrt(sm.sq + out[0]);
         newmax = std::fmax(out[1], sm.max);
         steg = steg / 2.0;
       }
+      // the last trial is the new point
+      std::swap(V.x, V.xt);
+      std::swap(V.xsi, V.xsit);
+      std::swap(V.eta, V.etat);
       residunorm = newresidu;
       residumax = newmax;
     }
@@ -549,9 +627,9 @@ static int mma_kkt_t(MmaState* S, const double* xd, const double* df0dx,
   Lam L{};
   for (int i = 0; i < M; ++i) L.v[i] = S->lambda[i];
   hipLaunchKernelGGL((kkt_k<M>), dim3(grid), dim3(kMB), 0, stream(), S->v, L,
-                     xd, df0dx, dfdx, S->part);
+                     xd, df0dx, dfdx, mma_out(S));
   double out[2];
-  int rc = finish(S, 2, grid, 2u, out);
+  int rc = finish(S, 2, out);
   if (rc) return rc;
   double mx = out[1], sq = 0.0, la = 0.0;
   for (int i = 0; i < M; ++i) la += S->lambda[i] * S->a[i];
@@ -607,16 +685,21 @@ int nekoamd_mma_create(void** mma, const int* n, const int* m, const void* x,
   S->s.assign(*m, 0.0);
   S->mu.assign(*m, 0.0);
   const int64_t N = *n;
-  const size_t nvec = 21 + 2 * (size_t)*m;
+  const size_t nvec = 16 + 2 * (size_t)*m;
   hipError_t e = hipMalloc((void**)&S->mem, sizeof(double) * nvec * N);
   if (e == hipSuccess)
-    e = hipMalloc((void**)&S->part, sizeof(double) * (kMaxVals * kMG + kMaxVals));
+    e = hipMalloc((void**)&S->part, sizeof(double) * kMaxVals * kMG);
+  if (e == hipSuccess) e = hipMalloc((void**)&S->count, sizeof(int));
+  if (e == hipSuccess) e = hipMemset(S->count, 0, sizeof(int));
+  if (e == hipSuccess) e = hipMalloc((void**)&S->bound, sizeof(double));
   if (e == hipSuccess)
-    e = hipHostMalloc((void**)&S->hres, sizeof(double) * kMaxVals,
+    e = hipHostMalloc((void**)&S->hres, sizeof(double) * (kMaxVals + 1),
                       hipHostMallocDefault);
   if (e != hipSuccess) {
     if (S->mem) (void)hipFree(S->mem);
     if (S->part) (void)hipFree(S->part);
+    if (S->count) (void)hipFree(S->count);
+    if (S->bound) (void)hipFree(S->bound);
     delete S;
     return fail_hip(__func__, e);
   }
@@ -625,9 +708,8 @@ int nekoamd_mma_create(void** mma, const int* n, const int* m, const void* x,
   V.n = N;
   double** slots[] = {&V.x,     &V.xsi,   &V.eta,   &V.low,    &V.upp,
                       &V.alpha, &V.beta,  &V.xmin,  &V.xmax,   &V.p0j,
-                      &V.q0j,   &V.xold1, &V.xold2, &V.dx,     &V.dxsi,
-                      &V.deta,  &V.xold,  &V.xsiold, &V.etaold, &V.delx,
-                      &V.diagx};
+                      &V.q0j,   &V.xold1, &V.xold2, &V.xt,     &V.xsit,
+                      &V.etat};
   for (double** s : slots) {
     *s = p;
     p += N;
@@ -649,6 +731,8 @@ int nekoamd_mma_create(void** mma, const int* n, const int* m, const void* x,
   if (e != hipSuccess) {
     (void)hipFree(S->mem);
     (void)hipFree(S->part);
+    (void)hipFree(S->count);
+    (void)hipFree(S->bound);
     (void)hipHostFree(S->hres);
     delete S;
     return fail_hip(__func__, e);
@@ -663,6 +747,8 @@ int nekoamd_mma_create(void** mma, const int* n, const int* m, const void* x,
   if (rc) {
     (void)hipFree(S->mem);
     (void)hipFree(S->part);
+    (void)hipFree(S->count);
+    (void)hipFree(S->bound);
     (void)hipHostFree(S->hres);
     delete S;
     return rc;
@@ -677,6 +763,8 @@ int nekoamd_mma_free(void* mma) {
   NK_HIP(hipStreamSynchronize(stream()));
   if (S->mem) NK_HIP(hipFree(S->mem));
   if (S->part) NK_HIP(hipFree(S->part));
+  if (S->count) NK_HIP(hipFree(S->count));
+  if (S->bound) NK_HIP(hipFree(S->bound));
   if (S->hres) NK_HIP(hipHostFree(S->hres));
   delete S;
   return kOk;

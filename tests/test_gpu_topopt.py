@@ -172,3 +172,30 @@ def test_mma_large_n_parity(env, n):
         print(f"mma n={n} it={it}: max |x_gpu - x_oracle| = {err:.2e}, newton iters "
               f"{opt.residuals()[2]:.0f}")
         assert err < 1e-9
+
+
+@pytest.mark.parametrize("n,m", [(1, 1), (511, 2), (513, 3), (262145, 4)])
+def test_mma_pass_edges(env, n, m):
+    """One variable, one short of and one past a block of the passes, one
+    past a full grid; one to four constraints (the first active).  The same
+    bar as the large problems above: the sub-solves end at the same residual."""
+    device, sem, T, g, o = env
+    rng = np.random.default_rng(n)
+    t = np.linspace(0, 1, n)
+    x = 0.4 + 0.1 * np.sin(7 * t)
+    target = 0.5 + 0.4 * np.cos(5 * t)
+    args = (m, 0.0, [0.0] * m, [100.0] * m, [0.0] * m)
+    xd = device.DeviceArray.from_host(x)
+    opt = T.MMA(xd, *args, device.DeviceArray.from_host(np.zeros(n)),
+                device.DeviceArray.from_host(np.ones(n)))
+    ref = oracle.MMA(x, *args, np.zeros(n), np.ones(n))
+    xr = x.copy()
+    dfdx = np.vstack([np.full(n, 100.0 / n)] + [rng.uniform(0.5, 1.5, n) / n] * (m - 1))
+    for it in range(1, 4):
+        df0 = 2 * (x - target) / n
+        fval = np.array([100 * (np.mean(x) - 0.4)] + [-1.0] * (m - 1))
+        opt.update(it, xd, device.DeviceArray.from_host(df0), fval,
+                   device.DeviceArray.from_host(np.asfortranarray(dfdx).ravel(order="F")))
+        xr = ref.update(it, xr, df0, fval, dfdx)
+        x = xd.get()
+        assert np.abs(x - xr).max() < 1e-9
