@@ -305,7 +305,10 @@ int nekoamd_cg_free(void* cg);
  * indices mask[0..nmask)), preconditioned by the Jacobi diagonal d
  * (nekoamd_jacobi_update).  f must be continuous (gs-assembled) and zero on
  * the mask, as the reference's callers guarantee (adjoint_pnpn.f90:725-726).
- * Blocks until the solve is done; fills mon. */
+ * Blocks until the solve is done; fills mon.  Small meshes (lx in [4, 8], up
+ * to 256 workgroups of one to eight elements) are solved in FP64 whatever the
+ * state's precision; a mixed state's solve still ends on the recomputed
+ * residual f - A x only. */
 int nekoamd_cg_solve(void* cg, void* x, const void* f, const void* d,
                      const void* mult, const double* volume,
                      const double* abstol, const int* max_iter,
@@ -343,8 +346,8 @@ int nekoamd_fcg_solve(void* st, void* x, const void* f, const void* d,
  * diagonal, kept in the first state) and one driver (their iterations go in
  * the same batches, one host read per batch for the three); each component
  * keeps its own scalars, stopping test and reliable updates (mon[0..2]).
- * FP64 states (or lx outside [4, 10]) run the three solves one after the
- * other. */
+ * FP64 states, lx outside [4, 10] and meshes small enough for a solve to be
+ * one kernel run the three solves one after the other. */
 int nekoamd_cg_solve3(void* const* cg, void* const* x, const void* const* f,
                       const void* d, const void* mult, const double* volume,
                       const double* abstol, const int* max_iter,

@@ -8,8 +8,8 @@
 // (krylov_solver_factory at adjoint_scheme.f90:1046-1055; solves at
 // adjoint_pnpn.f90:734-736 and, per component, :784-786).
 //
-// One iteration k is four kernels (plus the gs buckets) on the library
-// stream:
+// A small mesh's solve is one kernel in FP64 (cg_grid_k, below).  Else one
+// iteration k is four kernels (plus the gs buckets) on the library stream:
 //   ax_cg  : z = d r;  p_k = z + beta p_{k-1};  x += alpha_{k-1} p_{k-1};
 //            w = A_L p_k;  per-element partials of w.p_k
 //   gs     : w = QQ^T w                                         (gs.hip)
@@ -751,6 +751,51 @@ __global__ void __launch_bounds__(kRedBlock)
   }
 }
 
+// The FP64 solve of a mixed state (cg_grid_k): r = mask(f - w) with w = QQ^T
+// A x; partials of r.r.mult and r.(d r).mult.
+__global__ void __launch_bounds__(kRedBlock)
+    cg_true_r_k(int64_t n, double* __restrict__ r, const double* __restrict__ f,
+                const double* __restrict__ w, const double* __restrict__ dm,
+                const double* __restrict__ mult, double* __restrict__ part) {
+  __shared__ double sh[kRedBlock / 64];
+  double a = 0.0, b = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * kRedBlock + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * kRedBlock) {
+    const double di = dm[i];
+    const double ri = di == 0.0 ? 0.0 : f[i] - w[i];
+    r[i] = ri;
+    const double rm = ri * mult[i];
+    a += rm * ri;
+    b += rm * (ri * di);
+  }
+  a = block_sum<kRedBlock>(a, sh);
+  b = block_sum<kRedBlock>(b, sh);
+  if (threadIdx.x == 0) {
+    part[blockIdx.x] = a;
+    part[kRedGrid + blockIdx.x] = b;
+  }
+}
+
+__global__ void __launch_bounds__(kFinBlock)
+    cg_true_fin_k(CgScal* __restrict__ sc, const double* __restrict__ part,
+                  int np) {
+  if (sc->iter == 0) return;  // done at its start
+  __shared__ double sh[kFinBlock / 64];
+  const double rtr = sum_partials<kFinBlock>(part, np, sh);
+  const double rtz = sum_partials<kFinBlock>(part + kRedGrid, np, sh);
+  if (threadIdx.x == 0) {
+    const double rn = sqrt(rtr) * sc->norm_fac;
+    sc->rtr = rtr;
+    sc->rnorm = rn;
+    sc->beta = rtz / sc->rtz2;
+    sc->rtz1 = rtz;
+    sc->nupdate = sc->nupdate + 1;
+    sc->done =
+        (rn < sc->abstol || sc->iter >= sc->max_iter || !isfinite(rn)) ? 1 : 0;
+    sc->halt = sc->done;
+  }
+}
+
 __global__ void __launch_bounds__(kFinBlock)
     cg_rel_fin_k(CgScal* __restrict__ sc, const double* __restrict__ part,
                  int np) {
@@ -787,7 +832,7 @@ __global__ void __launch_bounds__(kFinBlock)
 }
 
 // ---------------------------------------------------------------------------
-// The FP64 iteration of small meshes as one kernel: workgroup b keeps the
+// The iteration of small meshes as one kernel, in FP64: workgroup b keeps the
 // vectors and operator data of EPB elements in registers over all iterations
 // (x, r, p, d_m, mult, G, h1, h2 B: 28 to 34 VGPRs), and an iteration is two
 // exchanges over the grid (gridsum.h) -- the shared points' w and the element
@@ -800,7 +845,9 @@ __global__ void __launch_bounds__(kFinBlock)
 // L2s); the five launches it replaces take 17 us however small the mesh is.
 // FP64 pressure solve, us per solve by launches -> here: 8x4x4 order 5
 // (336 iterations) 6170 -> 2380, 8x8x4 order 7 12550 -> 6290, 12x10x8 order
-// 3 6330 -> 3470, 10x8x6 order 5 10240 -> 5260.
+// 3 6330 -> 3470, 10x8x6 order 5 10240 -> 5260; solves of mixed states
+// likewise (10x8x6 order 5 11670 -> 5460, three velocity components on 8x8x4
+// order 7 583 -> 389).
 //
 // Up to kGridWg workgroups, one per CU.  Two per CU lose: the registers then
 // spill and a reader has twice the slots to wait for (10x8x6 order 7, 480
@@ -1346,18 +1393,30 @@ static int cg_grid_pick(const CgGrid& a, bool h2, bool* ran) {
             : cg_grid_launch<LX, EL, false>(a, ran);
 }
 
-// The started FP64 solve of s by cg_grid_k; *ran = false if the mesh is not
-// one of its (more than kGridWg workgroups, lx outside 4..8, points shared
-// by more than 8 elements), or if it got stuck (another process holding the
-// device): the caller then starts the solve over with the launches.  The
-// smaller orders take the fewest elements that make 256 threads while that
-// fits, else as many as 512 threads hold.
+// Whether the mesh of s may be one of cg_grid_k's: at most kGridWg
+// workgroups, lx in 4..8.  The smaller orders take the fewest elements that
+// make 256 threads while that fits, else as many as 512 threads hold.
+static bool cg_grid_fits(const CgState* s, const CgOp& op) {
+  return !s->grid_off && s->nelv > 0 && op.lx >= 4 && op.lx <= 8 &&
+         s->nelv <= kGridWg * (op.lx == 4 ? 8 : op.lx == 5 ? 4 : op.lx == 6 ? 2 : 1);
+}
+
+// The FP64 iteration vectors of a mixed state.
+static int grid_vectors(CgState* s) {
+  for (double** v : {&s->r, &s->p, &s->dm})
+    if (!*v) NK_HIP(hipMalloc((void**)v, sizeof(double) * s->n));
+  return kOk;
+}
+
+// The started solve of s by cg_grid_k; *ran = false if points are shared by
+// more than 8 elements, if the device has no room for all its workgroups, or
+// if it got stuck (another process holding the device): the caller then
+// starts the solve over with the launches.  A mixed state's solve ends, as
+// its launches' do, on the true residual f - A x only: it is recomputed
+// whenever the iterated one meets the tolerance.
 static int cg_grid(CgState* s, const CgOp& op, double* x, const double* mult,
-                   bool* ran) {
+                   const double* f, bool* ran) {
   *ran = false;
-  if (s->grid_off || s->nelv == 0 || op.lx < 4 || op.lx > 8) return kOk;
-  if (s->nelv > kGridWg * (op.lx == 4 ? 8 : op.lx == 5 ? 4 : op.lx == 6 ? 2 : 1))
-    return kOk;
   CgGrid a{};
   bool ok = false;
   int rc = gs_point_refs(op.gs, 8, &a.ref, &a.idx, &ok);
@@ -1397,6 +1456,20 @@ static int cg_grid(CgState* s, const CgOp& op, double* x, const double* mult,
       default: rc = cg_grid_pick<8, 1, 1>(a, op.ifh2, ran);
     }
     if (rc || !*ran) return rc;
+    if (s->prec == NEKOAMD_CG_MIXED) {
+      rc = ax_helm_launch<double, double>(s->w, x, op.dx, op.h1, op.h2, op.g11,
+                                          op.g12, op.g13, op.g22, op.g23,
+                                          op.g33, op.B, op.lx, s->nelv,
+                                          op.ifh2, nullptr);
+      if (!rc) rc = gs_launch<double>(op.gs, s->w, NEKOAMD_GS_ADD, nullptr);
+      if (rc) return rc;
+      hipLaunchKernelGGL(cg_true_r_k, dim3(s->grid), dim3(kRedBlock), 0,
+                         stream(), s->n, s->r, f, s->w, s->dm, mult, s->part);
+      NK_LAUNCHED();
+      hipLaunchKernelGGL(cg_true_fin_k, dim3(1), dim3(kFinBlock), 0, stream(),
+                         s->sc, s->part, s->grid);
+      NK_LAUNCHED();
+    }
     rc = to_host(&s->host[0], s->sc, sizeof(CgScal));
     if (rc) return rc;
     NK_HIP(hipStreamSynchronize(stream()));
@@ -1679,7 +1752,8 @@ int nekoamd_cg_solve(void* cg, void* x, const void* f, const void* d,
           *ifh2 != 0};
   const double* F = (const double*)f;
   int status = kOk;
-  if (s->prec == NEKOAMD_CG_FP64) {
+  // x = 0, r = f and the scalars of an FP64 iteration
+  const auto start64 = [&]() -> int {
     if (n > 0)
       NK_HIP(hipMemcpyAsync(s->dm, d, sizeof(double) * n,
                             hipMemcpyDeviceToDevice, stream()));
@@ -1688,29 +1762,34 @@ int nekoamd_cg_solve(void* cg, void* x, const void* f, const void* d,
                          s->dm, op.mask, *nmask);
       NK_LAUNCHED();
     }
-    double* X = (double*)x;
-    const auto start = [&]() -> int {
-      hipLaunchKernelGGL(cg_start_k<double>, dim3(s->grid), dim3(kRedBlock), 0,
-                         stream(), n, X, s->r, F, s->dm, (const double*)mult,
-                         nullptr, s->part);
-      NK_LAUNCHED();
-      hipLaunchKernelGGL(cg_start_fin_k, dim3(1), dim3(kFinBlock), 0, stream(),
-                         s->sc, s->part, s->grid, *volume, *abstol, *max_iter,
-                         0);
-      NK_LAUNCHED();
-      return kOk;
-    };
-    if ((status = start())) return status;
-    const bool was_off = s->grid_off;
+    hipLaunchKernelGGL(cg_start_k<double>, dim3(s->grid), dim3(kRedBlock), 0,
+                       stream(), n, (double*)x, s->r, F, s->dm,
+                       (const double*)mult, nullptr, s->part);
+    NK_LAUNCHED();
+    hipLaunchKernelGGL(cg_start_fin_k, dim3(1), dim3(kFinBlock), 0, stream(),
+                       s->sc, s->part, s->grid, *volume, *abstol, *max_iter,
+                       0);
+    NK_LAUNCHED();
+    return kOk;
+  };
+  const bool small = cg_grid_fits(s, op);
+  if (small) {
+    // a small mesh: both precisions in FP64 (nothing is bound by the bytes
+    // that FP32 vectors save)
+    if ((status = grid_vectors(s))) return status;
+    if ((status = start64())) return status;
     bool ran = false;
-    status = cg_grid(s, op, X, (const double*)mult, &ran);
-    if (status) return status;
+    if ((status = cg_grid(s, op, (double*)x, (const double*)mult, F, &ran)))
+      return status;
     if (ran) {
       fill_monitor(s->host[0], mon);
       s->last_iter = mon->iter;
       return kOk;
     }
-    if (s->grid_off != was_off && (status = start())) return status;
+  }
+  if (s->prec == NEKOAMD_CG_FP64) {
+    if ((status = start64())) return status;
+    double* X = (double*)x;
     status = cg_drive(s, *max_iter, batch, [&](int nb) {
       for (int q = 0; q < nb; ++q) {
         int rc = cg_iteration<double>(s, op, geo64(op), X, s->r, s->p, s->w, s->dm,
@@ -1772,9 +1851,14 @@ int nekoamd_cg_solve3(void* const* cg, void* const* x, const void* const* f,
                "the three CG states differ in size or precision");
   NK_REQUIRE(lx && volume && abstol && max_iter && poll && nmask && ifh2,
              "null argument");
-  // FP64 states, or an element size without the three-direction kernel:
-  // three solves one after the other
-  if (s[0]->prec != NEKOAMD_CG_MIXED || *lx < 4 || *lx > 10) {
+  // FP64 states, an element size without the three-direction kernel, or a
+  // mesh small enough for one kernel a solve: three solves one after the
+  // other
+  const CgOp shape{gs, nullptr, 0, nullptr, nullptr, nullptr, nullptr, nullptr,
+                   nullptr, nullptr, nullptr, nullptr, nullptr, *lx, *ifh2 != 0};
+  const bool small = cg_grid_fits(s[0], shape) && cg_grid_fits(s[1], shape) &&
+                     cg_grid_fits(s[2], shape);
+  if (s[0]->prec != NEKOAMD_CG_MIXED || *lx < 4 || *lx > 10 || small) {
     for (int c = 0; c < 3; ++c) {
       const int rc = nekoamd_cg_solve(
           cg[c], x[c], f[c], d, mult, volume, abstol, max_iter, poll, gs, mask,
