@@ -90,6 +90,9 @@ __device__ __forceinline__ double lane_moved(double v) {
   return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
 }
 __device__ __forceinline__ double wave_total(double v) {
+  // rounded here: a product must not be contracted into the first addition
+  // in one kernel and not in another
+  asm volatile("" : "+v"(v));
   v += lane_moved<0xB1, 0xf>(v);   // quad_perm [1,0,3,2]
   v += lane_moved<0x4E, 0xf>(v);   // quad_perm [2,3,0,1]
   v += lane_moved<0x141, 0xf>(v);  // row_half_mirror
@@ -112,20 +115,38 @@ __device__ __forceinline__ void grid_publish(uint64_t* slots, int wg,
     grid_put(slots + ((int64_t)wg * NV + j) * 2, tag, v[j]);
 }
 
+// block_sum (reduce.h) with wave_total's order.
+template <int BS>
+__device__ __forceinline__ double block_total(double v, double* sh) {
+  v = wave_total(v);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double s = 0.0;
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int q = 0; q < BS / 64; ++q) s += sh[q];
+  }
+  __syncthreads();
+  return s;
+}
+
 // Every thread of a workgroup: the sums over the nwg slots of this tag, the
 // same value in every thread of every workgroup (blockDim.x, a multiple of
-// 64, must be the same in all).  sh: NV doubles per wave of the workgroup;
+// 64, must be the same in all).  Slots t, t + NT, .. are added by thread t <
+// NT (0: blockDim.x), then as block_total adds.  sh: NV doubles per wave of the workgroup;
 // *fail: a shared int that is 0, set if a wait was given up.  Returns false
 // (in every thread) in that case.  sh may be written again after the next
 // workgroup barrier.
-template <int NV>
+template <int NV, int NT = 0>
 __device__ __forceinline__ bool grid_sum(const uint64_t* slots, int nwg,
                                          uint32_t tag, double* sh, int* fail,
                                          double (&out)[NV]) {
   double v[NV];
 #pragma unroll
   for (int j = 0; j < NV; ++j) v[j] = 0.0;
-  for (int q = threadIdx.x; q < nwg; q += blockDim.x) {
+  const int step = NT ? NT : (int)blockDim.x;
+  for (int q = NT && (int)threadIdx.x >= NT ? nwg : (int)threadIdx.x; q < nwg;
+       q += step) {
     const uint64_t* s[NV];
     double p[NV];
 #pragma unroll

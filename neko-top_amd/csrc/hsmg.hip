@@ -53,6 +53,7 @@
 
 #include <cstdlib>
 
+#include "gridsum.h"
 #include "internal.h"
 #include "nekoamd.h"
 #include "uniform.h"
@@ -92,6 +93,10 @@ struct Hsmg {
   int crs_G = 0;
   double *S27 = nullptr, *dl = nullptr, *xl = nullptr, *rl = nullptr,
          *zl = nullptr, *wl = nullptr, *pl[2] = {}, *cpart = nullptr;
+  // crs_grid_k (null: not used): its stuck flag, then the words its
+  // workgroups exchange; the next unused tag
+  uint64_t* cwords = nullptr;
+  uint32_t ctag = 1;
   // the coarse solve (fixed kernels on fixed buffers), recorded as a graph on
   // the first application and replayed (NEKOAMD_HIP_GRAPHS=1)
   hipGraphExec_t crs_graph = nullptr;
@@ -1066,7 +1071,9 @@ void level_free(Level& L) {
 // order in every block).  sh: kHB / 64 + 1 doubles.
 __device__ __forceinline__ double crs_all_sum(const double* __restrict__ part,
                                               int n, double* sh) {
-  const double s = sum_partials<kHB>(part, n, sh);
+  double s = 0.0;
+  for (int q = threadIdx.x; q < n; q += kHB) s += part[q];
+  s = block_total<kHB>(s, sh);
   if (threadIdx.x == 0) sh[kHB / 64] = s;
   __syncthreads();
   const double t = sh[kHB / 64];
@@ -1117,7 +1124,7 @@ __global__ void __launch_bounds__(kHB)
     zl[v] = z;
     s += r * z;
   }
-  s = block_sum<kHB>(s, sh);
+  s = block_total<kHB>(s, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
@@ -1161,7 +1168,7 @@ __global__ void __launch_bounds__(kHB)
     wl[v] = acc;
     s += acc * pv;
   }
-  s = block_sum<kHB>(s, sh);
+  s = block_total<kHB>(s, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
@@ -1209,16 +1216,253 @@ __global__ void __launch_bounds__(kHB)
     }
   }
   if constexpr (!LAST) {
-    s = block_sum<kHB>(s, sh);
+    s = block_total<kHB>(s, sh);
     if (threadIdx.x == 0) part[blockIdx.x] = s;
   }
 }
 
+// The element-local copies of vertex (a, b, c): get = their sum in element
+// order, put = x at each.
+__device__ __forceinline__ double lattice_get(const double* __restrict__ r1,
+                                              int nx, int ny, int nz, int a,
+                                              int b, int c) {
+  double r = 0.0;
+  for (int ez = max(c - 1, 0); ez <= min(c, nz - 1); ++ez)
+    for (int ey = max(b - 1, 0); ey <= min(b, ny - 1); ++ey)
+      for (int ex = max(a - 1, 0); ex <= min(a, nx - 1); ++ex) {
+        const int64_t e = ex + (int64_t)nx * (ey + (int64_t)ny * ez);
+        r += r1[e * 8 + (a - ex) + 2 * ((b - ey) + 2 * (c - ez))];
+      }
+  return r;
+}
+__device__ __forceinline__ void lattice_put(double* __restrict__ e1, int nx,
+                                            int ny, int nz, int a, int b, int c,
+                                            double x) {
+  for (int ez = max(c - 1, 0); ez <= min(c, nz - 1); ++ez)
+    for (int ey = max(b - 1, 0); ey <= min(b, ny - 1); ++ey)
+      for (int ex = max(a - 1, 0); ex <= min(a, nx - 1); ++ex) {
+        const int64_t e = ex + (int64_t)nx * (ey + (int64_t)ny * ez);
+        e1[e * 8 + (a - ex) + 2 * ((b - ey) + 2 * (c - ez))] = x;
+      }
+}
+
+struct CrsGrid {
+  int nx, ny, nz, faces, iters, halo;
+  uint32_t tag;
+  const double *r1, *dl, *S;
+  double* e1;
+  uint64_t *slots, *zw;  // partial sums (4 words per kHB vertices), z (2 per vertex)
+  int* stuck;
+  double *xl, *rl, *zl, *wl, *pl;  // crs_one_k only
+};
+
+// The coarse PCG of a small mesh as one kernel: workgroup b keeps kCB
+// vertices' x, r, z and 27 coefficients in registers and p on its vertices
+// and `halo` to either side (a vertex's row reaches nxl nyl + nxl + 1 away)
+// in LDS; an iteration is two exchanges over the grid (gridsum.h): z and
+// <r, z>, from which every workgroup forms p = z + beta p on its range, and
+// <w, p>.  The arithmetic and the order of every sum are the kernel-by-kernel
+// form's (two of its blocks' partials per workgroup), so the result is the
+// same bit for bit.  Bound by the exchanges, 2 us each, where a launch of the
+// kernel-by-kernel form takes about 5, 21 of them.  GMRES + HSMG solves by
+// launches -> here: 8x4x4 order 5 3300 -> 2190 us, 16x8x8 order 7 5850 ->
+// 4060, 16x16x16 order 7 8820 -> 6830, 32x16x16 order 7 21800 -> 19200.
+constexpr int kCB = 2 * kHB;
+
+// The sum of the four waves from wave wv as that block's partial (nblk
+// blocks; the last workgroup may have one).
+__device__ __forceinline__ void crs_publish(uint64_t* slots, uint32_t tag,
+                                            const double* sw, int wv, int nblk) {
+  const int blk = 2 * blockIdx.x + wv / (kHB / 64);
+  if (blk >= nblk) return;
+  double s[1] = {0.0};
+#pragma unroll
+  for (int k = 0; k < kHB / 64; ++k) s[0] += sw[wv + k];
+  grid_publish<1>(slots, blk, tag, s);
+}
+
+__global__ void __launch_bounds__(kCB) crs_grid_k(CrsGrid g) {
+  extern __shared__ double p[];  // kCB + 2 halo
+  __shared__ double s1[kCB / 64], s2[kCB / 64], s3[kCB / 64], s4[kCB / 64];
+  __shared__ int fail;
+  const int tid = threadIdx.x, wv = tid >> 6;
+  const int nxl = g.nx + 1, nyl = g.ny + 1, nxy = nxl * nyl;
+  const int nl = nxy * (g.nz + 1);
+  const int v0 = blockIdx.x * kCB, v = v0 + tid;
+  const bool live = v < nl;
+  const int a = v % nxl, b = (v / nxl) % nyl, c = v / nxy;
+  const int range = kCB + 2 * g.halo, nblk = (nl + kHB - 1) / kHB;
+  if (tid == 0) fail = 0;
+  for (int i = tid; i < range; i += kCB) p[i] = 0.0;
+  double S[27], x = 0.0, r = 0.0, d = 0.0;
+  // a term whose vertex lies outside the lattice reads the vertex itself and
+  // is dropped
+  uint32_t in = 0;
+#pragma unroll
+  for (int q = 0; q < 27; ++q) {
+    const int di = q % 3 - 1, dj = (q / 3) % 3 - 1, dk = q / 9 - 1;
+    const bool ok = live && a + di >= 0 && a + di < nxl && b + dj >= 0 &&
+                    b + dj < nyl && c + dk >= 0 && c + dk <= g.nz;
+    in |= ok ? 1u << q : 0u;
+    S[q] = live ? g.S[(int64_t)q * nl + v] : 0.0;
+  }
+  if (live) {
+    d = g.dl[v];
+    if (!lattice_masked(g.faces, g.nx, g.ny, g.nz, a, b, c))
+      r = lattice_get(g.r1, g.nx, g.ny, g.nz, a, b, c);
+  }
+  double z = r * d, rz[1] = {0.0}, prev = 0.0, pap[1];
+  uint64_t* slot_r = g.slots;
+  uint64_t* slot_p = g.slots + 2 * nblk;
+  __syncthreads();
+  bool ok = true;
+  for (int q = 0; q < g.iters; ++q) {
+    const uint32_t tag = g.tag + 2u * (uint32_t)q;
+    if (live) grid_put(g.zw + 2 * (int64_t)v, tag, z);
+    const double t1 = wave_total(r * z);
+    if ((tid & 63) == 0) s1[wv] = t1;
+    __syncthreads();
+    if ((tid & (kHB - 1)) == 0) crs_publish(slot_r, tag, s1, wv, nblk);
+    prev = rz[0];
+    if (!(ok = (grid_sum<1, kHB>(slot_r, nblk, tag, s2, &fail, rz)))) break;
+    const double beta = q > 0 && prev != 0.0 ? rz[0] / prev : 0.0;
+    // p on the halo from the other workgroups' z, on the own range from z
+    for (int i = tid; i < 2 * g.halo; i += kCB) {
+      const int j = i < g.halo ? i : i + kCB;
+      const int u = v0 - g.halo + j;
+      if (u < 0 || u >= nl) continue;
+      const uint64_t* src[1] = {g.zw + 2 * (int64_t)u};
+      double zu[1];
+      grid_get<1>(src, 1, tag, &fail, zu);
+      p[j] = zu[0] + beta * p[j];
+    }
+    const double pv = z + beta * p[g.halo + tid];
+    p[g.halo + tid] = pv;
+    __syncthreads();
+    double w = 0.0;
+#pragma unroll
+    for (int k = 0; k < 27; ++k) {
+      const int di = k % 3 - 1, dj = (k / 3) % 3 - 1, dk = k / 9 - 1;
+      const bool ok = (in >> k) & 1u;
+      const double pm = p[g.halo + tid + (ok ? di + nxl * dj + nxy * dk : 0)];
+      const double t = S[k] * pm;
+      w += ok ? t : 0.0;
+    }
+    const double t2 = wave_total(live ? w * pv : 0.0);
+    if ((tid & 63) == 0) s3[wv] = t2;
+    __syncthreads();
+    if ((tid & (kHB - 1)) == 0) crs_publish(slot_p, tag + 1u, s3, wv, nblk);
+    // past this every workgroup has read z, so the next may overwrite it
+    if (!(ok = (grid_sum<1, kHB>(slot_p, nblk, tag + 1u, s4, &fail, pap)))) break;
+    const double alpha = pap[0] != 0.0 ? rz[0] / pap[0] : 0.0;
+    x += alpha * pv;
+    r -= alpha * w;
+    z = r * d;
+  }
+  if (!ok) {
+    if (tid == 0) dev_store(g.stuck, 1);
+    return;
+  }
+  if (live) lattice_put(g.e1, g.nx, g.ny, g.nz, a, b, c, x);
+}
+
+// The same solve by one workgroup if crs_grid_k got stuck (another process
+// holding the device); else nothing.
+__global__ void __launch_bounds__(1024) crs_one_k(CrsGrid g) {
+  __shared__ double sh[1024 / 64 + 1];
+  if (*g.stuck == 0) return;
+  const int nxl = g.nx + 1, nyl = g.ny + 1, nxy = nxl * nyl;
+  const int nl = nxy * (g.nz + 1);
+  auto all_sum = [&](double s) {
+    s = block_sum<1024>(s, sh);
+    if (threadIdx.x == 0) sh[1024 / 64] = s;
+    __syncthreads();
+    s = sh[1024 / 64];
+    __syncthreads();
+    return s;
+  };
+  for (int v = threadIdx.x; v < nl; v += 1024) {
+    const int a = v % nxl, b = (v / nxl) % nyl, c = v / nxy;
+    const double r = lattice_masked(g.faces, g.nx, g.ny, g.nz, a, b, c)
+                         ? 0.0
+                         : lattice_get(g.r1, g.nx, g.ny, g.nz, a, b, c);
+    g.xl[v] = 0.0;
+    g.pl[v] = 0.0;
+    g.rl[v] = r;
+    g.zl[v] = r * g.dl[v];
+  }
+  double prev = 0.0;
+  for (int q = 0; q < g.iters; ++q) {
+    double s = 0.0;
+    for (int v = threadIdx.x; v < nl; v += 1024) s += g.rl[v] * g.zl[v];
+    const double rz = all_sum(s);
+    const double beta = q > 0 && prev != 0.0 ? rz / prev : 0.0;
+    prev = rz;
+    for (int v = threadIdx.x; v < nl; v += 1024)
+      g.pl[v] = g.zl[v] + beta * g.pl[v];
+    __threadfence_block();
+    __syncthreads();
+    s = 0.0;
+    for (int v = threadIdx.x; v < nl; v += 1024) {
+      const int a = v % nxl, b = (v / nxl) % nyl, c = v / nxy;
+      double w = 0.0;
+      for (int k = 0; k < 27; ++k) {
+        const int di = k % 3 - 1, dj = (k / 3) % 3 - 1, dk = k / 9 - 1;
+        if (a + di < 0 || a + di >= nxl || b + dj < 0 || b + dj >= nyl ||
+            c + dk < 0 || c + dk > g.nz)
+          continue;
+        w += g.S[(int64_t)k * nl + v] * g.pl[v + di + nxl * dj + nxy * dk];
+      }
+      g.wl[v] = w;
+      s += w * g.pl[v];
+    }
+    const double pap = all_sum(s);
+    const double alpha = pap != 0.0 ? rz / pap : 0.0;
+    for (int v = threadIdx.x; v < nl; v += 1024) {
+      g.xl[v] += alpha * g.pl[v];
+      const double r = g.rl[v] - alpha * g.wl[v];
+      g.rl[v] = r;
+      g.zl[v] = r * g.dl[v];
+    }
+  }
+  for (int v = threadIdx.x; v < nl; v += 1024)
+    lattice_put(g.e1, g.nx, g.ny, g.nz, v % nxl, (v / nxl) % nyl, v / nxy,
+                g.xl[v]);
+  __syncthreads();
+  if (threadIdx.x == 0) *g.stuck = 0;
+}
+
+// Halo of crs_grid_k's ranges, or 0 if the lattice is not one of its: the
+// ranges must fit 64 KB of LDS (lattice planes of up to 56 x 56 or so) and
+// 256 workgroups (131072 vertices), which are also the block partials of the
+// other form.  Its workgroups find room beside the Schwarz kernels of the
+// library stream as those' workgroups retire.
+int crs_grid_halo(const Hsmg* h) {
+  const int64_t halo = (int64_t)(h->nx + 1) * (h->ny + 1) + h->nx + 2;
+  const bool fits = !h->graphs &&
+                    (kCB + 2 * halo) * (int64_t)sizeof(double) <= 60 * 1024 &&
+                    h->nl <= 256 * (int64_t)kCB;
+  return fits ? (int)halo : 0;
+}
+
 // e1 = crs_iter PCG iterations from r1 (element-local, before its gs), the
-// result masked and element-local: 1 + 2 crs_iter launches on the library
-// stream (or recorded as kernel nodes).
+// result masked and element-local: crs_grid_k, or 1 + 2 crs_iter launches, on
+// the launch stream (or the latter recorded as kernel nodes).
 int coarse_pcg(Hsmg* h) {
   const int G = h->crs_G, it = h->crs_iter;
+  if (h->cwords) {
+    const int halo = crs_grid_halo(h), wg = (int)((h->nl + kCB - 1) / kCB);
+    CrsGrid g{h->nx, h->ny, h->nz, h->faces, it, halo, h->ctag, h->r1, h->dl,
+              h->S27, h->e1, h->cwords + 1, h->cwords + 1 + 8 * wg,
+              (int*)h->cwords, h->xl, h->rl, h->zl, h->wl, h->pl[0]};
+    h->ctag += 2u * (uint32_t)it;
+    nk_launch(crs_grid_k, dim3(wg), dim3(kCB),
+              (unsigned)((kCB + 2 * halo) * sizeof(double)), g);
+    NK_LAUNCHED();
+    nk_launch(crs_one_k, dim3(1), dim3(1024), 0, g);
+    NK_LAUNCHED();
+    return kOk;
+  }
   double* rtz = h->cpart;           // [it][G]: <r, z> before iteration q
   double* pap = h->cpart + (int64_t)it * G;  // [it][G]: <w, p> of iteration q
   nk_launch(crs_init_k, dim3(G), dim3(kHB), 0, h->nx, h->ny, h->nz, h->faces,
@@ -1258,7 +1502,7 @@ void hsmg_destroy(Hsmg* h) {
                   (void*)h->r1, (void*)h->e1, h->rf, h->zf, (void*)h->S27,
                   (void*)h->dl, (void*)h->xl, (void*)h->rl, (void*)h->zl,
                   (void*)h->wl, (void*)h->pl[0], (void*)h->pl[1],
-                  (void*)h->cpart})
+                  (void*)h->cpart, (void*)h->cwords})
     if (p) (void)hipFree(p);
   if (h->crs_graph) (void)hipGraphExecDestroy(h->crs_graph);
   if (h->side) {
@@ -1399,6 +1643,12 @@ int coarse_lattice_setup(Hsmg* h) {
     if (e == hipSuccess) e = hipMalloc(p, vb);
   if (e == hipSuccess)
     e = hipMalloc(&h->cpart, sizeof(double) * 2 * (size_t)h->crs_iter * h->crs_G);
+  if (e == hipSuccess && crs_grid_halo(h) > 0) {
+    const size_t wb = sizeof(uint64_t) *
+                      (1 + 8 * (size_t)((nl + kCB - 1) / kCB) + 2 * (size_t)nl);
+    e = hipMalloc(&h->cwords, wb);
+    if (e == hipSuccess) e = hipMemset(h->cwords, 0, wb);
+  }
   if (e == hipSuccess) e = hipMemcpy(h->S27, S.data(), 27 * vb, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(h->dl, dl.data(), vb, hipMemcpyHostToDevice);
   if (e != hipSuccess) return fail_hip("nekoamd_hsmg_create", e);

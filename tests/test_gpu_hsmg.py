@@ -145,3 +145,26 @@ def test_fp32_hsmg_inside_fp64_gmres(pair):
     assert m32.done == 1 and m32.res_final < 1e-9
     assert m32.iter <= m64.iter + 2
     assert err < 1e-6
+
+
+@pytest.mark.parametrize("box", [(1, 1, 1), (9, 7, 5), (12, 9, 7), (58, 58, 1), (61, 61, 1)])
+def test_coarse_kernel_equals_launches(box, monkeypatch):
+    """The coarse solve as one kernel against its launches (the ones a HIP
+    graph records), bit for bit: one element, two blocks of vertices in one
+    workgroup, a last workgroup with one block, the largest plane whose range
+    fits the kernel and one past it (launches on both sides)."""
+    from nekoamd import device, sem
+    device.init(0)
+    g = sem.BoxCase(*box, 4, jitter=0.05, seed=1234)
+    M = sem.HSMG(g)
+    monkeypatch.setenv("NEKOAMD_HIP_GRAPHS", "1")
+    Mg = sem.HSMG(g)
+    rng = np.random.default_rng(5)
+    z, zg = g.field(), g.field()
+    for _ in range(3):
+        r = g.field(rng.standard_normal(g.n))
+        g.gs.op(r)
+        M.apply(z, r)
+        Mg.apply(zg, r)
+        assert np.array_equal(z.get(), zg.get()) and np.isfinite(z.get()).all()
+        assert z.get().any()
