@@ -926,7 +926,7 @@ __global__ void __launch_bounds__((LX * LX * LX * EPB + 63) / 64 * 64)
     const double w = ax_point<LX, double, H2>(p, op, su + o, sr + o, ss + o,
                                               st + o, sD, t);
     if (m > 0) grid_put(a.w + 2 * g, tag, w);
-    const double d = wave_total(live ? w * p : 0.0);
+    const double d = wave_sum(live ? w * p : 0.0);
     if ((tid & 63) == 0) s1[tid >> 6] = d;
     __syncthreads();
     if (tid == 0) {
@@ -952,7 +952,7 @@ __global__ void __launch_bounds__((LX * LX * LX * EPB + 63) / 64 * 64)
     x += alpha * p;
     r = dm == 0.0 ? 0.0 : r - alpha * ws;
     const double rm = r * mult;
-    const double c0 = wave_total(rm * r), c1 = wave_total(rm * (r * dm));
+    const double c0 = wave_sum(rm * r), c1 = wave_sum(rm * (r * dm));
     if ((tid & 63) == 0) {
       s3[tid >> 6] = c0;
       s3[NW + (tid >> 6)] = c1;

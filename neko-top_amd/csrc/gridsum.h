@@ -78,33 +78,6 @@ __device__ __forceinline__ void grid_get(const uint64_t* const (&s)[N], int n,
   }
 }
 
-// The wave's sum of v in every lane (all 64 active), by lane moves of the
-// vector unit: within a row of 16 by quad permutes and mirrors, then row 0
-// into 1 and 2 into 3, then 1 into 3; a fixed order, about a fifth of
-// wave_sum's latency, which counts where nothing else runs meanwhile.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double lane_moved(double v) {
-  const uint64_t b = (uint64_t)__double_as_longlong(v);
-  const uint32_t lo = __builtin_amdgcn_update_dpp(0, (uint32_t)b, CTRL, ROWS, 0xf, false);
-  const uint32_t hi = __builtin_amdgcn_update_dpp(0, (uint32_t)(b >> 32), CTRL, ROWS, 0xf, false);
-  return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
-}
-__device__ __forceinline__ double wave_total(double v) {
-  // rounded here: a product must not be contracted into the first addition
-  // in one kernel and not in another
-  asm volatile("" : "+v"(v));
-  v += lane_moved<0xB1, 0xf>(v);   // quad_perm [1,0,3,2]
-  v += lane_moved<0x4E, 0xf>(v);   // quad_perm [2,3,0,1]
-  v += lane_moved<0x141, 0xf>(v);  // row_half_mirror
-  v += lane_moved<0x140, 0xf>(v);  // row_mirror
-  v += lane_moved<0x142, 0xa>(v);  // row_bcast15 into rows 1 and 3
-  v += lane_moved<0x143, 0xc>(v);  // row_bcast31 into rows 2 and 3
-  const uint64_t b = (uint64_t)__double_as_longlong(v);
-  const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)b, 63);
-  const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(b >> 32), 63);
-  return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
-}
-
 // One thread of a workgroup: its NV partial sums into slots[wg].
 template <int NV>
 __device__ __forceinline__ void grid_publish(uint64_t* slots, int wg,
@@ -115,25 +88,10 @@ __device__ __forceinline__ void grid_publish(uint64_t* slots, int wg,
     grid_put(slots + ((int64_t)wg * NV + j) * 2, tag, v[j]);
 }
 
-// block_sum (reduce.h) with wave_total's order.
-template <int BS>
-__device__ __forceinline__ double block_total(double v, double* sh) {
-  v = wave_total(v);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
-  __syncthreads();
-  double s = 0.0;
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int q = 0; q < BS / 64; ++q) s += sh[q];
-  }
-  __syncthreads();
-  return s;
-}
-
 // Every thread of a workgroup: the sums over the nwg slots of this tag, the
 // same value in every thread of every workgroup (blockDim.x, a multiple of
 // 64, must be the same in all).  Slots t, t + NT, .. are added by thread t <
-// NT (0: blockDim.x), then as block_total adds.  sh: NV doubles per wave of the workgroup;
+// NT (0: blockDim.x), then as block_sum (reduce.h) adds.  sh: NV doubles per wave of the workgroup;
 // *fail: a shared int that is 0, set if a wait was given up.  Returns false
 // (in every thread) in that case.  sh may be written again after the next
 // workgroup barrier.
@@ -158,7 +116,7 @@ __device__ __forceinline__ bool grid_sum(const uint64_t* slots, int nwg,
   const int wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
-    v[j] = wave_total(v[j]);
+    v[j] = wave_sum(v[j]);
     if ((threadIdx.x & 63) == 0) sh[wv * NV + j] = v[j];
   }
   __syncthreads();

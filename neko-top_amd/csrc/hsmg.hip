@@ -1071,9 +1071,7 @@ void level_free(Level& L) {
 // order in every block).  sh: kHB / 64 + 1 doubles.
 __device__ __forceinline__ double crs_all_sum(const double* __restrict__ part,
                                               int n, double* sh) {
-  double s = 0.0;
-  for (int q = threadIdx.x; q < n; q += kHB) s += part[q];
-  s = block_total<kHB>(s, sh);
+  const double s = sum_partials<kHB>(part, n, sh);
   if (threadIdx.x == 0) sh[kHB / 64] = s;
   __syncthreads();
   const double t = sh[kHB / 64];
@@ -1124,7 +1122,7 @@ __global__ void __launch_bounds__(kHB)
     zl[v] = z;
     s += r * z;
   }
-  s = block_total<kHB>(s, sh);
+  s = block_sum<kHB>(s, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
@@ -1168,7 +1166,7 @@ __global__ void __launch_bounds__(kHB)
     wl[v] = acc;
     s += acc * pv;
   }
-  s = block_total<kHB>(s, sh);
+  s = block_sum<kHB>(s, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
@@ -1216,7 +1214,7 @@ __global__ void __launch_bounds__(kHB)
     }
   }
   if constexpr (!LAST) {
-    s = block_total<kHB>(s, sh);
+    s = block_sum<kHB>(s, sh);
     if (threadIdx.x == 0) part[blockIdx.x] = s;
   }
 }
@@ -1319,7 +1317,7 @@ __global__ void __launch_bounds__(kCB) crs_grid_k(CrsGrid g) {
   for (int q = 0; q < g.iters; ++q) {
     const uint32_t tag = g.tag + 2u * (uint32_t)q;
     if (live) grid_put(g.zw + 2 * (int64_t)v, tag, z);
-    const double t1 = wave_total(r * z);
+    const double t1 = wave_sum(r * z);
     if ((tid & 63) == 0) s1[wv] = t1;
     __syncthreads();
     if ((tid & (kHB - 1)) == 0) crs_publish(slot_r, tag, s1, wv, nblk);
@@ -1348,7 +1346,7 @@ __global__ void __launch_bounds__(kCB) crs_grid_k(CrsGrid g) {
       const double t = S[k] * pm;
       w += ok ? t : 0.0;
     }
-    const double t2 = wave_total(live ? w * pv : 0.0);
+    const double t2 = wave_sum(live ? w * pv : 0.0);
     if ((tid & 63) == 0) s3[wv] = t2;
     __syncthreads();
     if ((tid & (kHB - 1)) == 0) crs_publish(slot_p, tag + 1u, s3, wv, nblk);

@@ -65,7 +65,7 @@ __device__ __forceinline__ double2 ld_nt2(const double* p) {
 }
 
 // Block partials of KM sums (the first m meaningful) to part[i * G + blk]:
-// a butterfly over each wavefront, then the 4 wavefronts in order.
+// a sum over each wavefront, then the 4 wavefronts in order.
 template <int KM>
 __device__ __forceinline__ void block_partials(const double (&s)[KM], int m,
                                                double (*sh)[4],

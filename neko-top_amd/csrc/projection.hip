@@ -72,6 +72,9 @@ namespace nekoamd {
 
 constexpr double kProjTol = 1e-7;
 constexpr int kDotGrid = 512;     // partials per inner product (augment)
+// Blocks of an FP32-basis inner product: what the CUs hold at once (a block
+// reduces one value per basis vector, however few points it takes).
+constexpr int kProj32Grid = 2048;
 constexpr int kProjGrid = kMultiGrid;  // max partials per inner product (basis)
 
 struct ProjState {
@@ -127,9 +130,55 @@ __device__ __forceinline__ float2 ld_nt2f(const float* p) {
   return v;
 }
 
+// The FP32 passes take W consecutive points per thread: four (16-byte basis
+// loads) or two where n and the base addresses allow it (points_at_once),
+// else one.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <int W>
+__device__ __forceinline__ void ld_basis(const float* p, double (&v)[W]) {
+  if constexpr (W == 4) {
+    const f32x4 x = __builtin_nontemporal_load((const f32x4*)p);
+    v[0] = (double)x.x;
+    v[1] = (double)x.y;
+    v[2] = (double)x.z;
+    v[3] = (double)x.w;
+  } else if constexpr (W == 2) {
+    const float2 x = ld_nt2f(p);
+    v[0] = (double)x.x;
+    v[1] = (double)x.y;
+  } else {
+    v[0] = (double)__builtin_nontemporal_load(p);
+  }
+}
+template <int W>
+__device__ __forceinline__ void ld_points(const double* p, double (&v)[W]) {
+  if constexpr (W == 1) {
+    v[0] = p[0];
+  } else {
+#pragma unroll
+    for (int j = 0; j < W; j += 2) {
+      const double2 x = *(const double2*)(p + j);
+      v[j] = x.x;
+      v[j + 1] = x.y;
+    }
+  }
+}
+template <int W>
+__device__ __forceinline__ void st_points(double* p, const double (&v)[W]) {
+  if constexpr (W == 1) {
+    p[0] = v[0];
+  } else {
+#pragma unroll
+    for (int j = 0; j < W; j += 2)
+      *(double2*)(p + j) = make_double2(v[j], v[j + 1]);
+  }
+}
+
 // part[i * G + blk] = block blk's partial of <a, V_i>_mult, i < m, for the m
-// FP32 vectors V_i = V + i n (mdots_k with an FP32 basis).
-template <int KM, bool P2, typename TM>
+// FP32 vectors V_i = V + i n (mdots_k with an FP32 basis).  n = 4.2 M, m =
+// 12: 85 -> 64 us with four points per thread and wave sums without LDS (the
+// linear combinations 66 -> 56 and, with its write, 75 -> 59 us).
+template <int KM, int W, typename TM>
 __global__ void __launch_bounds__(256)
     mdots32_k(int64_t n, const double* __restrict__ a,
               const float* __restrict__ V, int m,
@@ -138,52 +187,41 @@ __global__ void __launch_bounds__(256)
   double s[KM];
 #pragma unroll
   for (int i = 0; i < KM; ++i) s[i] = 0.0;
-  if constexpr (P2) {
-    const int64_t n2 = n / 2;
-    const double2* a2 = (const double2*)a;
-    for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < n2;
-         q += (int64_t)gridDim.x * 256) {
-      const double2 av = a2[q], mv = mult_pair(mult, q);
-      const double w0 = mv.x * av.x, w1 = mv.y * av.y;
+  const int64_t nq = n / W;
+  for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < nq;
+       q += (int64_t)gridDim.x * 256) {
+    double w[W];
+    ld_points<W>(a + W * q, w);
 #pragma unroll
-      for (int c = 0; c < KM; c += 8) {
-        if (c < m) {
+    for (int j = 0; j < W; ++j) w[j] *= mult_at(mult, W * q + j);
 #pragma unroll
-          for (int i = c; i < c + 8; ++i)
-            if (i < m) {
-              const float2 v = ld_nt2f(V + (int64_t)i * n + 2 * q);
-              s[i] += w0 * (double)v.x + w1 * (double)v.y;
-            }
-          asm volatile("" ::: "memory");
-        }
-      }
-    }
-  } else {
-    for (int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x; p < n;
-         p += (int64_t)gridDim.x * 256) {
-      const double w = mult_at(mult, p) * a[p];
+    for (int c = 0; c < KM; c += 8) {
+      if (c < m) {
 #pragma unroll
-      for (int c = 0; c < KM; c += 8) {
-        if (c < m) {
+        for (int i = c; i < c + 8; ++i)
+          if (i < m) {
+            double v[W], d = 0.0;
+            ld_basis<W>(V + (int64_t)i * n + W * q, v);
 #pragma unroll
-          for (int i = c; i < c + 8; ++i)
-            if (i < m)
-              s[i] += w * (double)__builtin_nontemporal_load(V + (int64_t)i * n + p);
-          asm volatile("" ::: "memory");
-        }
+            for (int j = 0; j < W; ++j) d += w[j] * v[j];
+            s[i] += d;
+          }
+        asm volatile("" ::: "memory");
       }
     }
   }
   block_partials<KM>(s, m, sh, part);
 }
 
-// s += sum_{i<k} c[i] V_i (FP32 vectors) at the pair (2q, 2q + 1) (P2) or
-// the point q (in s.x); c in LDS.
-template <int KM, bool P2>
-__device__ __forceinline__ void comb_point32(const double* c,
-                                             const float* __restrict__ V,
-                                             int64_t n, int k, int64_t q,
-                                             double2& s) {
+// s = sum_{i<k} c[i] V_i (FP32 vectors) at the points W q, .., W q + W - 1;
+// c in LDS.
+template <int KM, int W>
+__device__ __forceinline__ void comb_points32(const double* c,
+                                              const float* __restrict__ V,
+                                              int64_t n, int k, int64_t q,
+                                              double (&s)[W]) {
+#pragma unroll
+  for (int j = 0; j < W; ++j) s[j] = 0.0;
 #pragma unroll
   for (int c0 = 0; c0 < KM; c0 += 8) {
     if (c0 < k) {
@@ -191,13 +229,10 @@ __device__ __forceinline__ void comb_point32(const double* c,
       for (int i = c0; i < c0 + 8; ++i)
         if (i < k) {
           const double ci = c[i];
-          if constexpr (P2) {
-            const float2 v = ld_nt2f(V + (int64_t)i * n + 2 * q);
-            s.x += ci * (double)v.x;
-            s.y += ci * (double)v.y;
-          } else {
-            s.x += ci * (double)__builtin_nontemporal_load(V + (int64_t)i * n + q);
-          }
+          double v[W];
+          ld_basis<W>(V + (int64_t)i * n + W * q, v);
+#pragma unroll
+          for (int j = 0; j < W; ++j) s[j] += ci * v[j];
         }
       asm volatile("" ::: "memory");
     }
@@ -205,28 +240,24 @@ __device__ __forceinline__ void comb_point32(const double* c,
 }
 
 // xout = sum_{i<m} alpha_i u_i over the FP32 basis.
-template <int KM, bool P2>
+template <int KM, int W>
 __global__ void __launch_bounds__(256)
     proj_lincomb32_k(int64_t n, int m, const double* __restrict__ alpha,
                      const float* __restrict__ xx, double* __restrict__ xout) {
   __shared__ double sa[NEKOAMD_PROJ_MAX_L];
   if (threadIdx.x < m) sa[threadIdx.x] = alpha[threadIdx.x];
   __syncthreads();
-  const int64_t nq = P2 ? n / 2 : n;
-  for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < nq;
+  for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < n / W;
        q += (int64_t)gridDim.x * 256) {
-    double2 sx = make_double2(0.0, 0.0);
-    comb_point32<KM, P2>(sa, xx, n, m, q, sx);
-    if constexpr (P2)
-      ((double2*)xout)[q] = sx;
-    else
-      xout[q] = sx.x;
+    double sx[W];
+    comb_points32<KM, W>(sa, xx, n, m, q, sx);
+    st_points<W>(xout + W * q, sx);
   }
 }
 
 // One Gram-Schmidt pass of xk against the first k FP32 basis vectors with
 // coefficients c: xk -= sum c_i u_i (FP64), and its FP32 copy to uk.
-template <int KM, bool P2>
+template <int KM, int W>
 __global__ void __launch_bounds__(256)
     proj_cgs32_k(int64_t n, int k, const double* __restrict__ c,
                  const float* __restrict__ xx, double* __restrict__ xk,
@@ -234,22 +265,21 @@ __global__ void __launch_bounds__(256)
   __shared__ double sc[KM];
   if ((int)threadIdx.x < k) sc[threadIdx.x] = c[threadIdx.x];
   __syncthreads();
-  const int64_t nq = P2 ? n / 2 : n;
-  for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < nq;
+  for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < n / W;
        q += (int64_t)gridDim.x * 256) {
-    double2 sx = make_double2(0.0, 0.0);
-    comb_point32<KM, P2>(sc, xx, n, k, q, sx);
-    if constexpr (P2) {
-      double2* x2 = (double2*)xk + q;
-      const double2 xo = *x2;
-      const double2 xn = make_double2(xo.x - sx.x, xo.y - sx.y);
-      *x2 = xn;
-      ((float2*)uk)[q] = make_float2((float)xn.x, (float)xn.y);
-    } else {
-      const double xn = xk[q] - sx.x;
-      xk[q] = xn;
-      uk[q] = (float)xn;
-    }
+    double sx[W], x[W];
+    ld_points<W>(xk + W * q, x);
+    comb_points32<KM, W>(sc, xx, n, k, q, sx);
+#pragma unroll
+    for (int j = 0; j < W; ++j) x[j] -= sx[j];
+    st_points<W>(xk + W * q, x);
+    if constexpr (W == 4)
+      *(f32x4*)(uk + W * q) =
+          f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
+    else if constexpr (W == 2)
+      *(float2*)(uk + W * q) = make_float2((float)x[0], (float)x[1]);
+    else
+      uk[q] = (float)x[0];
   }
 }
 
@@ -584,44 +614,54 @@ static int cgs(ProjState* s, int k, const double* c, double* xk, double* bk,
 }
 
 // ---- FP32 basis --------------------------------------------------------
+// Points per thread of an FP32-basis pass over n points: all vectors of the
+// basis at f, f + n, .. and FP64 arrays p0, p1.
+static int points_at_once(int64_t n, const float* f, const void* p0,
+                          const void* p1 = nullptr) {
+  if (!pairs_ok(n, p0, p1) || ((uintptr_t)f & 7) != 0) return 1;
+  return n % 4 == 0 && ((uintptr_t)f & 15) == 0 ? 4 : 2;
+}
+
 template <int KM, typename TM>
 static void mdots32_launch_km(ProjState* s, const double* a, int m,
-                              const TM* mult, int G, bool p2) {
+                              const TM* mult, int G, int w) {
   const dim3 g(G), b(256);
-  if (p2)
-    hipLaunchKernelGGL((mdots32_k<KM, true, TM>), g, b, 0, stream(), s->n, a,
+  if (w == 4)
+    hipLaunchKernelGGL((mdots32_k<KM, 4, TM>), g, b, 0, stream(), s->n, a,
+                       s->xx32, m, mult, s->part);
+  else if (w == 2)
+    hipLaunchKernelGGL((mdots32_k<KM, 2, TM>), g, b, 0, stream(), s->n, a,
                        s->xx32, m, mult, s->part);
   else
-    hipLaunchKernelGGL((mdots32_k<KM, false, TM>), g, b, 0, stream(), s->n, a,
+    hipLaunchKernelGGL((mdots32_k<KM, 1, TM>), g, b, 0, stream(), s->n, a,
                        s->xx32, m, mult, s->part);
 }
 
 template <typename TM>
 static void mdots32_launch(ProjState* s, const double* a, int m, const TM* mult,
-                           int G, bool p2) {
+                           int G, int w) {
   if (m <= 8)
-    mdots32_launch_km<8>(s, a, m, mult, G, p2);
+    mdots32_launch_km<8>(s, a, m, mult, G, w);
   else if (m <= 16)
-    mdots32_launch_km<16>(s, a, m, mult, G, p2);
+    mdots32_launch_km<16>(s, a, m, mult, G, w);
   else if (m <= 24)
-    mdots32_launch_km<24>(s, a, m, mult, G, p2);
+    mdots32_launch_km<24>(s, a, m, mult, G, w);
   else if (m <= 32)
-    mdots32_launch_km<32>(s, a, m, mult, G, p2);
+    mdots32_launch_km<32>(s, a, m, mult, G, w);
   else
-    mdots32_launch_km<64>(s, a, m, mult, G, p2);
+    mdots32_launch_km<64>(s, a, m, mult, G, w);
 }
 
 // out[0..m) = <a, u_i>_mult / nu_i^2 for the first m FP32 basis vectors.
 static int dots32(ProjState* s, const double* a, int m, const double* mult,
                   double* out) {
   if (m <= 0) return kOk;
-  const int G = nk_grid(s->n, 256, kProjGrid);
-  if (s->cnt_ok && mult == s->cnt_key) {
-    const bool p2 = pairs_ok(s->n, a, s->xx32) && ((uintptr_t)s->cnt8 & 1) == 0;
-    mdots32_launch(s, a, m, (const uint8_t*)s->cnt8, G, p2);
-  } else {
-    mdots32_launch(s, a, m, mult, G, pairs_ok(s->n, a, mult, s->xx32));
-  }
+  const int w = points_at_once(s->n, s->xx32, a);
+  const int G = nk_grid(s->n / w, 256, kProj32Grid);
+  if (s->cnt_ok && mult == s->cnt_key)
+    mdots32_launch(s, a, m, (const uint8_t*)s->cnt8, G, w);
+  else
+    mdots32_launch(s, a, m, mult, G, w);
   NK_LAUNCHED();
   hipLaunchKernelGGL(proj_fin_k, dim3(m), dim3(kFinBlock), 0, stream(),
                      s->part, G, s->inv2, m, out);
@@ -631,54 +671,61 @@ static int dots32(ProjState* s, const double* a, int m, const double* mult,
 
 template <int KM>
 static void lincomb32_launch(ProjState* s, int m, const double* alpha,
-                             double* xout, bool p2) {
-  const dim3 g(kMultiGrid), bl(256);
-  if (p2)
-    hipLaunchKernelGGL((proj_lincomb32_k<KM, true>), g, bl, 0, stream(), s->n,
-                       m, alpha, s->xx32, xout);
+                             double* xout, int w) {
+  const dim3 g(nk_grid(s->n / w, 256, kMultiGrid)), bl(256);
+  if (w == 4)
+    hipLaunchKernelGGL((proj_lincomb32_k<KM, 4>), g, bl, 0, stream(), s->n, m,
+                       alpha, s->xx32, xout);
+  else if (w == 2)
+    hipLaunchKernelGGL((proj_lincomb32_k<KM, 2>), g, bl, 0, stream(), s->n, m,
+                       alpha, s->xx32, xout);
   else
-    hipLaunchKernelGGL((proj_lincomb32_k<KM, false>), g, bl, 0, stream(),
-                       s->n, m, alpha, s->xx32, xout);
+    hipLaunchKernelGGL((proj_lincomb32_k<KM, 1>), g, bl, 0, stream(), s->n, m,
+                       alpha, s->xx32, xout);
 }
 
 // xout = sum_{i<m} alpha_i u_i over the FP32 basis.
 static int lincomb32(ProjState* s, int m, const double* alpha, double* xout) {
-  const bool p2 = pairs_ok(s->n, xout, s->xx32);
+  const int w = points_at_once(s->n, s->xx32, xout);
   if (m <= 8)
-    lincomb32_launch<8>(s, m, alpha, xout, p2);
+    lincomb32_launch<8>(s, m, alpha, xout, w);
   else if (m <= 16)
-    lincomb32_launch<16>(s, m, alpha, xout, p2);
+    lincomb32_launch<16>(s, m, alpha, xout, w);
   else if (m <= 32)
-    lincomb32_launch<32>(s, m, alpha, xout, p2);
+    lincomb32_launch<32>(s, m, alpha, xout, w);
   else
-    lincomb32_launch<64>(s, m, alpha, xout, p2);
+    lincomb32_launch<64>(s, m, alpha, xout, w);
   NK_LAUNCHED();
   return kOk;
 }
 
 template <int KM>
 static void cgs32_launch(ProjState* s, int k, const double* c, double* xk,
-                         float* uk, bool p2) {
-  const dim3 g(kMultiGrid), bl(256);
-  if (p2)
-    hipLaunchKernelGGL((proj_cgs32_k<KM, true>), g, bl, 0, stream(), s->n, k,
-                       c, s->xx32, xk, uk);
+                         float* uk, int w) {
+  const dim3 g(nk_grid(s->n / w, 256, kMultiGrid)), bl(256);
+  if (w == 4)
+    hipLaunchKernelGGL((proj_cgs32_k<KM, 4>), g, bl, 0, stream(), s->n, k, c,
+                       s->xx32, xk, uk);
+  else if (w == 2)
+    hipLaunchKernelGGL((proj_cgs32_k<KM, 2>), g, bl, 0, stream(), s->n, k, c,
+                       s->xx32, xk, uk);
   else
-    hipLaunchKernelGGL((proj_cgs32_k<KM, false>), g, bl, 0, stream(), s->n, k,
-                       c, s->xx32, xk, uk);
+    hipLaunchKernelGGL((proj_cgs32_k<KM, 1>), g, bl, 0, stream(), s->n, k, c,
+                       s->xx32, xk, uk);
 }
 
 // xk -= sum_{i<k} c_i u_i (k may be 0) and uk = (float) xk.
 static int cgs32(ProjState* s, int k, const double* c, double* xk, float* uk) {
-  const bool p2 = pairs_ok(s->n, xk, uk, s->xx32);
+  // uk is a vector of the basis
+  const int w = points_at_once(s->n, s->xx32, xk);
   if (k <= 8)
-    cgs32_launch<8>(s, k, c, xk, uk, p2);
+    cgs32_launch<8>(s, k, c, xk, uk, w);
   else if (k <= 16)
-    cgs32_launch<16>(s, k, c, xk, uk, p2);
+    cgs32_launch<16>(s, k, c, xk, uk, w);
   else if (k <= 32)
-    cgs32_launch<32>(s, k, c, xk, uk, p2);
+    cgs32_launch<32>(s, k, c, xk, uk, w);
   else
-    cgs32_launch<64>(s, k, c, xk, uk, p2);
+    cgs32_launch<64>(s, k, c, xk, uk, w);
   NK_LAUNCHED();
   return kOk;
 }

@@ -1,6 +1,6 @@
 // reduce.h -- deterministic reductions for gfx950 (64-wide wavefronts).
 //
-// Every sum is taken with a fixed tree: a butterfly over the 64 lanes, then
+// Every sum is taken with a fixed tree: one over the 64 lanes, then
 // the wavefront partials of a block in order, then (in a one-block finalise
 // kernel) the block partials in a fixed strided order.  For a given problem
 // size the result is the same bit pattern on every run.
@@ -9,10 +9,32 @@
 
 namespace nekoamd {
 
+// The wave's sum of v in every lane (all 64 active), by lane moves of the
+// vector unit: within a row of 16 by quad permutes and mirrors, then row 0
+// into 1 and 2 into 3, then 1 into 3.  A butterfly of shuffles goes through
+// LDS twelve times; where a workgroup reduces a value per basis vector that
+// was as much work as the pass itself (mdot.h).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double lane_moved(double v) {
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, (uint32_t)b, CTRL, ROWS, 0xf, false);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, (uint32_t)(b >> 32), CTRL, ROWS, 0xf, false);
+  return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  // rounded here: a product must not be contracted into the first addition
+  // in one kernel and not in another
+  asm volatile("" : "+v"(v));
+  v += lane_moved<0xB1, 0xf>(v);   // quad_perm [1,0,3,2]
+  v += lane_moved<0x4E, 0xf>(v);   // quad_perm [2,3,0,1]
+  v += lane_moved<0x141, 0xf>(v);  // row_half_mirror
+  v += lane_moved<0x140, 0xf>(v);  // row_mirror
+  v += lane_moved<0x142, 0xa>(v);  // row_bcast15 into rows 1 and 3
+  v += lane_moved<0x143, 0xc>(v);  // row_bcast31 into rows 2 and 3
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)b, 63);
+  const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(b >> 32), 63);
+  return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
 }
 
 // Sum over a block of BS threads (BS a multiple of 64).  sh: BS/64 doubles of

@@ -140,6 +140,15 @@ def test_fp32_basis_projection(sem, dims, lx, kind, keep):
     assert P.m < L
 
 
+@pytest.mark.parametrize("dims,lx", [((3, 2, 1), 5), ((1, 1, 1), 5), ((2, 1, 1), 6),
+                                     ((9, 8, 6), 7)])
+def test_fp32_basis_points_at_once(sem, dims, lx):
+    """Point counts of two (750), one (125) and four points per thread, the
+    last in more than one workgroup with a remainder; the bars of the FP32
+    basis above."""
+    test_fp32_basis_projection(sem, dims, lx, "pressure", 2)
+
+
 def test_augment_is_galerkin_scaled(sem):
     """gamma = <q,b>/<q,Aq>: b' is orthogonal to q, and a q with a
     non-positive <q,Aq> is ignored."""
