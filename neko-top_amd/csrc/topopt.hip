@@ -92,7 +92,14 @@ __device__ __forceinline__ Cof cofactors(const double xr[3], const double xs[3],
 }
 
 // Element-local gradient of NF fields (and, when OBJ, the objective
-// partials).  One workgroup per element, thread per (i,j) column.
+// partials).  One workgroup per element, thread per (i,j) column, which the
+// thread keeps in registers: the t-derivative needs no LDS, and only the
+// plane at hand is in LDS for the other two (two buffers, one barrier per
+// plane).  Bound by HBM (3 + NF fields in, and chi, B or 3 NF gradients)
+// with the LDS reads close behind: 16 per point and field here, 24 with
+// whole fields in LDS, where 25 KB per wave also left six waves on a CU.
+// Objective at 32x16x16, lx = 8: 96 -> 69 us (3.9 TB/s); 87 us with the nine
+// divisions by J per point that sum of squares / J^2 makes one.
 template <int LX, int NF, bool OBJ>
 __global__ void __launch_bounds__(LX * LX)
     grad_k(const double* __restrict__ xc, const double* __restrict__ yc,
@@ -102,28 +109,39 @@ __global__ void __launch_bounds__(LX * LX)
            double* __restrict__ gy, double* __restrict__ gz,
            const double* __restrict__ chi, const double* __restrict__ bm,
            double* __restrict__ part) {
-  constexpr int NS = LX * LX, NP = NS * LX;
-  __shared__ double s[3 + NF][NP];
+  constexpr int NS = LX * LX, NP = NS * LX, NA = 3 + NF;
+  __shared__ double s[2][NA][NS];
   const int e = blockIdx.x, t = threadIdx.x, i = t % LX, j = t / LX;
   const int64_t eb = (int64_t)e * NP + t;
   const double* src[6] = {xc, yc, zc, f0, f1, f2};
+  double col[NA][LX], Di[LX], Dj[LX];
 #pragma unroll
-  for (int a = 0; a < 3 + NF; ++a)
+  for (int k = 0; k < LX; ++k)
 #pragma unroll
-    for (int k = 0; k < LX; ++k) s[a][k * NS + t] = src[a][eb + k * NS];
-  __syncthreads();
+    for (int a = 0; a < NA; ++a) col[a][k] = src[a][eb + k * NS];
+#pragma unroll
+  for (int m = 0; m < LX; ++m) {
+    Di[m] = dx[i * LX + m];
+    Dj[m] = dx[j * LX + m];
+  }
   double diss = 0.0, lube = 0.0;
 #pragma unroll
   for (int k = 0; k < LX; ++k) {
-    double dr[3 + NF], ds[3 + NF], dt[3 + NF];
+    double(*sk)[NS] = s[k & 1];
 #pragma unroll
-    for (int a = 0; a < 3 + NF; ++a) {
+    for (int a = 0; a < NA; ++a) sk[a][t] = col[a][k];
+    // the other buffer's readers passed this barrier's predecessor only
+    // after their reads of the plane before it
+    __syncthreads();
+    double dr[NA], ds[NA], dt[NA];
+#pragma unroll
+    for (int a = 0; a < NA; ++a) {
       double r = 0.0, q = 0.0, w = 0.0;
 #pragma unroll
       for (int m = 0; m < LX; ++m) {
-        r += dx[i * LX + m] * s[a][k * NS + j * LX + m];
-        q += dx[j * LX + m] * s[a][k * NS + m * LX + i];
-        w += dx[k * LX + m] * s[a][m * NS + t];
+        r += Di[m] * sk[a][j * LX + m];
+        q += Dj[m] * sk[a][m * LX + i];
+        w += dx[k * LX + m] * col[a][m];
       }
       dr[a] = r;
       ds[a] = q;
@@ -137,39 +155,47 @@ __global__ void __launch_bounds__(LX * LX)
     double sq = 0.0;
 #pragma unroll
     for (int a = 0; a < NF; ++a) {
-      const double u0 = (c.r[0] * dr[3 + a] + c.s[0] * ds[3 + a] + c.t[0] * dt[3 + a]) / c.J;
-      const double u1 = (c.r[1] * dr[3 + a] + c.s[1] * ds[3 + a] + c.t[1] * dt[3 + a]) / c.J;
-      const double u2 = (c.r[2] * dr[3 + a] + c.s[2] * ds[3 + a] + c.t[2] * dt[3 + a]) / c.J;
+      const double n0 = c.r[0] * dr[3 + a] + c.s[0] * ds[3 + a] + c.t[0] * dt[3 + a];
+      const double n1 = c.r[1] * dr[3 + a] + c.s[1] * ds[3 + a] + c.t[1] * dt[3 + a];
+      const double n2 = c.r[2] * dr[3 + a] + c.s[2] * ds[3 + a] + c.t[2] * dt[3 + a];
       if constexpr (!OBJ) {
-        gx[g] = u0;
-        gy[g] = u1;
-        gz[g] = u2;
+        gx[g] = n0 / c.J;
+        gy[g] = n1 / c.J;
+        gz[g] = n2 / c.J;
       } else {
-        sq += u0 * u0 + u1 * u1 + u2 * u2;
+        sq += n0 * n0 + n1 * n1 + n2 * n2;
       }
     }
+    if constexpr (OBJ) sq = sq / (c.J * c.J);
     if constexpr (OBJ) {
       const double b = bm[g];
       diss += sq * b;
-      double su = s[3][k * NS + t];
-      if constexpr (NF > 1) su += s[4][k * NS + t];
-      if constexpr (NF > 2) su += s[5][k * NS + t];
+      double su = col[3][k];
+      if constexpr (NF > 1) su += col[4][k];
+      if constexpr (NF > 2) su += col[5][k];
       lube += chi[g] * su * b;
     }
   }
   if constexpr (OBJ) {
-    __shared__ double sd[2][NS];
-    sd[0][t] = diss;
-    sd[1][t] = lube;
-    __syncthreads();
-    if (t == 0) {
-      double a = 0.0, b = 0.0;
-      for (int q = 0; q < NS; ++q) {
-        a += sd[0][q];
-        b += sd[1][q];
+    if constexpr (NS == 64) {
+      diss = wave_sum(diss);
+      lube = wave_sum(lube);
+    } else {
+      __shared__ double sd[2][NS];
+      sd[0][t] = diss;
+      sd[1][t] = lube;
+      __syncthreads();
+      if (t == 0) {
+        diss = lube = 0.0;
+        for (int q = 0; q < NS; ++q) {
+          diss += sd[0][q];
+          lube += sd[1][q];
+        }
       }
-      part[e] = a;
-      part[(int64_t)gridDim.x + e] = b;
+    }
+    if (t == 0) {
+      part[e] = diss;
+      part[(int64_t)gridDim.x + e] = lube;
     }
   }
 }
@@ -214,10 +240,11 @@ static int grad_dispatch(int lx, int nelv, const double* x, const double* y,
 }
 
 // The objective's two sums (dissipation, lube) into host memory hres: the
-// gradient pass writes 2 nelv partials into part, fin2_k sums them into
-// part[2 nelv], part[2 nelv + 1], which are copied back on the library
-// stream.  part holds 2 nelv + 2 doubles.
-static int objective_sums(double* hres, double* part, const void* u,
+// gradient pass writes 2 nelv partials into part; fin2_k sums them into hres
+// itself where that is pinned, else into part[2 nelv], part[2 nelv + 1],
+// which are copied back on the library stream.  part holds 2 nelv + 2
+// doubles.
+static int objective_sums(double* hres, bool pinned, double* part, const void* u,
                           const void* v, const void* w, const void* chi,
                           const void* B, const void* x, const void* y,
                           const void* z, const void* dx, int lx, int ne) {
@@ -228,10 +255,11 @@ static int objective_sums(double* hres, double* part, const void* u,
                                   (const double*)chi, (const double*)B, part);
   if (rc) return rc;
   hipLaunchKernelGGL(fin2_k, dim3(1), dim3(kFinBlock), 0, stream(), part,
-                     (int64_t)ne, part + 2 * (size_t)ne);
+                     (int64_t)ne, pinned ? hres : part + 2 * (size_t)ne);
   NK_LAUNCHED();
-  NK_HIP(hipMemcpyAsync(hres, part + 2 * (size_t)ne, 2 * sizeof(double),
-                        hipMemcpyDeviceToHost, stream()));
+  if (!pinned)
+    NK_HIP(hipMemcpyAsync(hres, part + 2 * (size_t)ne, 2 * sizeof(double),
+                          hipMemcpyDeviceToHost, stream()));
   NK_HIP(hipStreamSynchronize(stream()));
   return kOk;
 }
@@ -450,7 +478,7 @@ int nekoamd_dissipation_objective(double* out, const void* u, const void* v,
                                hipHostMallocDefault);
   int rc = e == hipSuccess ? kOk : fail_hip(__func__, e);
   if (rc == kOk)
-    rc = objective_sums(hres, part, u, v, w, chi, B, x, y, z, dx, *lx, ne);
+    rc = objective_sums(hres, true, part, u, v, w, chi, B, x, y, z, dx, *lx, ne);
   if (rc == kOk) objective_finish(out, hres, *K, *obj_scale, *if_lube);
   if (hres) (void)hipHostFree(hres);
   (void)hipFree(part);
@@ -484,7 +512,7 @@ int nekoamd_dissipation_objective_noalloc(
   }
   double hres[2] = {0.0, 0.0};
   const int rc =
-      objective_sums(hres, part, u, v, w, chi, B, x, y, z, dx, *lx, ne);
+      objective_sums(hres, false, part, u, v, w, chi, B, x, y, z, dx, *lx, ne);
   if (rc == kOk) objective_finish(out, hres, *K, *obj_scale, *if_lube);
   return rc;
 }
