@@ -1365,21 +1365,22 @@ __global__ void __launch_bounds__(kCB) crs_grid_k(CrsGrid g) {
 }
 
 // The same solve by one workgroup if crs_grid_k got stuck (another process
-// holding the device); else nothing.
-__global__ void __launch_bounds__(1024) crs_one_k(CrsGrid g) {
-  __shared__ double sh[1024 / 64 + 1];
+// holding the device); else nothing.  kHB threads: an empty launch of 1024
+// waited 25 us for a CU with room beside the Schwarz kernels.
+__global__ void __launch_bounds__(kHB) crs_one_k(CrsGrid g) {
+  __shared__ double sh[kHB / 64 + 1];
   if (*g.stuck == 0) return;
   const int nxl = g.nx + 1, nyl = g.ny + 1, nxy = nxl * nyl;
   const int nl = nxy * (g.nz + 1);
   auto all_sum = [&](double s) {
-    s = block_sum<1024>(s, sh);
-    if (threadIdx.x == 0) sh[1024 / 64] = s;
+    s = block_sum<kHB>(s, sh);
+    if (threadIdx.x == 0) sh[kHB / 64] = s;
     __syncthreads();
-    s = sh[1024 / 64];
+    s = sh[kHB / 64];
     __syncthreads();
     return s;
   };
-  for (int v = threadIdx.x; v < nl; v += 1024) {
+  for (int v = threadIdx.x; v < nl; v += kHB) {
     const int a = v % nxl, b = (v / nxl) % nyl, c = v / nxy;
     const double r = lattice_masked(g.faces, g.nx, g.ny, g.nz, a, b, c)
                          ? 0.0
@@ -1392,16 +1393,16 @@ __global__ void __launch_bounds__(1024) crs_one_k(CrsGrid g) {
   double prev = 0.0;
   for (int q = 0; q < g.iters; ++q) {
     double s = 0.0;
-    for (int v = threadIdx.x; v < nl; v += 1024) s += g.rl[v] * g.zl[v];
+    for (int v = threadIdx.x; v < nl; v += kHB) s += g.rl[v] * g.zl[v];
     const double rz = all_sum(s);
     const double beta = q > 0 && prev != 0.0 ? rz / prev : 0.0;
     prev = rz;
-    for (int v = threadIdx.x; v < nl; v += 1024)
+    for (int v = threadIdx.x; v < nl; v += kHB)
       g.pl[v] = g.zl[v] + beta * g.pl[v];
     __threadfence_block();
     __syncthreads();
     s = 0.0;
-    for (int v = threadIdx.x; v < nl; v += 1024) {
+    for (int v = threadIdx.x; v < nl; v += kHB) {
       const int a = v % nxl, b = (v / nxl) % nyl, c = v / nxy;
       double w = 0.0;
       for (int k = 0; k < 27; ++k) {
@@ -1416,14 +1417,14 @@ __global__ void __launch_bounds__(1024) crs_one_k(CrsGrid g) {
     }
     const double pap = all_sum(s);
     const double alpha = pap != 0.0 ? rz / pap : 0.0;
-    for (int v = threadIdx.x; v < nl; v += 1024) {
+    for (int v = threadIdx.x; v < nl; v += kHB) {
       g.xl[v] += alpha * g.pl[v];
       const double r = g.rl[v] - alpha * g.wl[v];
       g.rl[v] = r;
       g.zl[v] = r * g.dl[v];
     }
   }
-  for (int v = threadIdx.x; v < nl; v += 1024)
+  for (int v = threadIdx.x; v < nl; v += kHB)
     lattice_put(g.e1, g.nx, g.ny, g.nz, v % nxl, (v / nxl) % nyl, v / nxy,
                 g.xl[v]);
   __syncthreads();
@@ -1457,7 +1458,7 @@ int coarse_pcg(Hsmg* h) {
     nk_launch(crs_grid_k, dim3(wg), dim3(kCB),
               (unsigned)((kCB + 2 * halo) * sizeof(double)), g);
     NK_LAUNCHED();
-    nk_launch(crs_one_k, dim3(1), dim3(1024), 0, g);
+    nk_launch(crs_one_k, dim3(1), dim3(kHB), 0, g);
     NK_LAUNCHED();
     return kOk;
   }
