@@ -27,7 +27,7 @@
 //
 // Measured at 32^3 p=7, before (two LDS reads per FMA) and now (one line per
 // thread, see dealias_k): forward 4.03 -> 1.24 ms, linearised 7.24 -> 2.24,
-// adjoint 6.98 -> 1.76; 13x11x9 p=5 forward 47.8 -> 23.2 us.
+// adjoint 6.98 -> 1.76; 13x11x9 p=5 forward 43.2 -> 22.3 us.
 #include <cmath>
 #include <vector>
 
