@@ -592,10 +592,13 @@ static int mma_update_t(MmaState* S, int iter, double* xd, const double* df0dx,
         newmax = std::fmax(out[1], sm.max);
         steg = steg / 2.0;
       }
-      // the last trial is the new point
-      std::swap(V.x, V.xt);
-      std::swap(V.xsi, V.xsit);
-      std::swap(V.eta, V.etat);
+      // the last trial is the new point; there is none if the residual to
+      // improve on is not finite
+      if (itto > 0) {
+        std::swap(V.x, V.xt);
+        std::swap(V.xsi, V.xsit);
+        std::swap(V.eta, V.etat);
+      }
       residunorm = newresidu;
       residumax = newmax;
     }

@@ -199,3 +199,39 @@ def test_mma_pass_edges(env, n, m):
         xr = ref.update(it, xr, df0, fval, dfdx)
         x = xd.get()
         assert np.abs(x - xr).max() < 1e-9
+
+
+@pytest.mark.parametrize("entry", ["value", "gradient", "fixed"])
+@pytest.mark.parametrize("max_iter", [1, 2])
+def test_mma_non_finite_residual_keeps_the_iterate(env, entry, max_iter):
+    """A constraint value that is NaN, an infinite gradient entry, or a variable
+    with xmin = xmax (0/0 in the asymptotes' terms): no trial of the line
+    search can lower the residual, so none is evaluated and the design is the
+    sub-problem's starting point (alpha + beta) / 2, whatever the number of
+    Newton steps.  One level of the interior-point loop (epsimin = 0.5)."""
+    device, sem, T, g, o = env
+    n = 1000
+    rng = np.random.default_rng(11)
+    x = rng.uniform(0.2, 0.8, n)
+    lo, hi = np.zeros(n), np.ones(n)
+    df0 = rng.uniform(-1.0, 1.0, n)
+    if entry == "fixed":
+        lo[17] = hi[17] = x[17]
+    elif entry == "gradient":
+        df0[17] = np.inf
+    fval = [np.nan if entry == "value" else 0.1]
+    # first update: asymptotes at x -+ w / 2, alpha and beta from them
+    w = hi - lo
+    low, upp = x - 0.5 * w, x + 0.5 * w
+    f01 = np.float64(np.float32(0.1))
+    alpha = np.maximum(np.maximum(lo, low + 0.1 * (x - low)), x - 0.5 * w)
+    beta = np.minimum(np.minimum(hi, upp - f01 * (upp - x)), x + 0.5 * w)
+    want = 0.5 * (alpha + beta)
+    xd = device.DeviceArray.from_host(x)
+    opt = T.MMA(xd, 1, 0.0, [0.0], [100.0], [0.0], device.DeviceArray.from_host(lo),
+                device.DeviceArray.from_host(hi), max_iter=max_iter, epsimin=0.5)
+    opt.update(1, xd, device.DeviceArray.from_host(df0), fval,
+               device.DeviceArray.from_host(np.full(n, 1.0 / n)))
+    # a few roundings of values in [0, 1]
+    assert np.abs(xd.get() - want).max() <= 1e-15
+    assert opt.residuals()[2] == max_iter
