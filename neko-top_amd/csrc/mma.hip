@@ -68,7 +68,7 @@ struct MmaState {
   double* mem = nullptr;   // one device block for all vectors
   double* part = nullptr;  // kMaxVals * kMG partials
   int* count = nullptr;    // workgroups of the running pass that are done
-  bool down = false;       // direction of the next pass over the variables
+  bool down = false;       // direction of the update's next pass
   double* bound = nullptr; // the direction pass's result
   // pinned: the last evaluation's results, then the direction pass's
   double* hres = nullptr;
@@ -479,6 +479,8 @@ static int mma_update_t(MmaState* S, int iter, double* xd, const double* df0dx,
   MmaVec& V = S->v;
   const int grid = mma_grid(V.n);
   double out[kMaxVals];
+  // the order of an update's sums must not depend on the updates before it
+  S->down = false;
   // ---- gensub
   hipLaunchKernelGGL((gensub_k<M>), dim3(grid), dim3(kMB), 0, stream(), V, xd,
                      df0dx, dfdx, iter < 3 ? 1 : 0, S->asyinit, S->asyincr,

@@ -235,3 +235,28 @@ def test_mma_non_finite_residual_keeps_the_iterate(env, entry, max_iter):
     # a few roundings of values in [0, 1]
     assert np.abs(xd.get() - want).max() <= 1e-15
     assert opt.residuals()[2] == max_iter
+
+
+def test_mma_update_does_not_depend_on_earlier_ones(env):
+    """A first update (its asymptotes come from x alone) of the same inputs
+    gives the same bits on a fresh state and on one that has made other
+    updates, with odd and even numbers of passes among them."""
+    device, sem, T, g, o = env
+    n = 200001
+    rng = np.random.default_rng(3)
+    x = rng.uniform(0.2, 0.8, n)
+    lo, hi = (device.DeviceArray.from_host(np.full(n, v)) for v in (0.0, 1.0))
+    dfdx = device.DeviceArray.from_host(rng.uniform(0.5, 1.5, n) * 100.0 / n)
+    df0 = rng.uniform(-1.0, 0.2, n) / n
+
+    def state():
+        return T.MMA(device.DeviceArray.from_host(x), 1, 1.0, [0.0], [100.0], [0.0], lo, hi)
+
+    def update(opt, scale):
+        xd = device.DeviceArray.from_host(x)
+        opt.update(1, xd, device.DeviceArray.from_host(scale * df0), [1.0], dfdx)
+        return xd.get()
+
+    used = state()
+    for scale in (1.0, 0.1, 3.0, 0.01, 30.0, 0.5):
+        assert np.array_equal(update(used, scale), update(state(), scale)), scale
