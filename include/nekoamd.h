@@ -301,6 +301,17 @@ typedef struct {
 int nekoamd_cg_create(void** cg, const int64_t* n, const int* nelv,
                       const int* precision);
 int nekoamd_cg_free(void* cg);
+/* The workgroups of a small mesh's solve (below) wait for one another at most
+ * us microseconds (default 1e6; 0: every wait is given up at once).  A solve
+ * that gives one up, because another process holds the device, starts over
+ * with launches, and this state's later solves take them from the start,
+ * until this is called again. */
+int nekoamd_cg_set_wait(void* cg, const int64_t* us);
+/* How the state's last solve ran. */
+#define NEKOAMD_BY_LAUNCHES 0   /* a handful of launches per iteration */
+#define NEKOAMD_ONE_KERNEL 1    /* one kernel that keeps the vectors */
+#define NEKOAMD_COUPLED 2       /* nekoamd_cg_solve3's coupled launches */
+int nekoamd_cg_path(void* cg, int* path);
 /* x = A^-1 f for A = QQ^T (h1 A_L + h2 B) with the Dirichlet mask (0-based
  * indices mask[0..nmask)), preconditioned by the Jacobi diagonal d
  * (nekoamd_jacobi_update).  f must be continuous (gs-assembled) and zero on

@@ -116,11 +116,13 @@ struct CgState {
   float* geo32 = nullptr;
   const void* geo_key[9] = {};
   // cg_grid_k: the words its workgroups exchange (per workgroup 2 of pap, 4
-  // of rtr and rtz; then 2 of w per point), the next unused tag, and whether
-  // a solve of this state got stuck in it
+  // of rtr and rtz; then 2 of w per point), the next unused tag, the longest
+  // wait, and whether a solve of this state got stuck in it
   uint64_t* slots = nullptr;
   uint32_t tag = 1;
+  unsigned long long wait = kGridWait;
   bool grid_off = false;
+  int path = NEKOAMD_BY_LAUNCHES;  // of the last solve
 };
 
 // ---------------------------------------------------------------------------
@@ -865,6 +867,7 @@ struct CgGrid {
   const int32_t* idx;
   CgScal* sc;
   uint64_t* slots;
+  unsigned long long wait;
   uint32_t tag;
   int nelv;
 };
@@ -941,13 +944,13 @@ __global__ void __launch_bounds__((LX * LX * LX * EPB + 63) / 64 * 64)
       double v[8];
 #pragma unroll
       for (int k = 0; k < 8; ++k) src[k] = a.w + 2 * (int64_t)idx[k];
-      grid_get<8>(src, m, tag, &fail, v);
+      grid_get<8>(src, m, tag, a.wait, &fail, v);
       ws = v[0];
 #pragma unroll
       for (int k = 1; k < 8; ++k)
         if (k < m) ws += v[k];
     }
-    if (!(ok = grid_sum<1>(slot_p, nwg, tag, s2, &fail, pap))) break;
+    if (!(ok = grid_sum<1>(slot_p, nwg, tag, a.wait, s2, &fail, pap))) break;
     alpha = rtz1 / pap[0];
     x += alpha * p;
     r = dm == 0.0 ? 0.0 : r - alpha * ws;
@@ -969,7 +972,7 @@ __global__ void __launch_bounds__((LX * LX * LX * EPB + 63) / 64 * 64)
     }
     // every workgroup has read its copies' w before it publishes here, so
     // the next iteration may overwrite them
-    if (!(ok = grid_sum<2>(slot_r, nwg, tag + 1u, s4, &fail, rr))) break;
+    if (!(ok = grid_sum<2>(slot_r, nwg, tag + 1u, a.wait, s4, &fail, rr))) break;
     ++it;
     rn = sqrt(rr[0]) * norm_fac;
     beta = rr[1] / rtz1;
@@ -1444,6 +1447,7 @@ static int cg_grid(CgState* s, const CgOp& op, double* x, const double* mult,
   a.bm = op.B;
   a.sc = s->sc;
   a.slots = s->slots;
+  a.wait = s->wait;
   a.nelv = s->nelv;
   for (;;) {
     a.tag = s->tag;
@@ -1708,6 +1712,22 @@ int nekoamd_cg_status(void* cg, nekoamd_cg_monitor_t* mon) {
   return kOk;
 }
 
+int nekoamd_cg_set_wait(void* cg, const int64_t* us) {
+  CgState* s = as_cg(cg);
+  NK_REQUIRE(s && us, "null argument");
+  NK_REQUIRE(*us >= 0 && *us <= 1000000000, "wait outside [0, 1e9] us");
+  s->wait = (unsigned long long)*us * kGridTicks;
+  s->grid_off = false;
+  return kOk;
+}
+
+int nekoamd_cg_path(void* cg, int* path) {
+  CgState* s = as_cg(cg);
+  NK_REQUIRE(s && path, "null argument");
+  *path = s->path;
+  return kOk;
+}
+
 int nekoamd_cg_solve(void* cg, void* x, const void* f, const void* d,
                      const void* mult, const double* volume,
                      const double* abstol, const int* max_iter,
@@ -1784,9 +1804,11 @@ int nekoamd_cg_solve(void* cg, void* x, const void* f, const void* d,
     if (ran) {
       fill_monitor(s->host[0], mon);
       s->last_iter = mon->iter;
+      s->path = NEKOAMD_ONE_KERNEL;
       return kOk;
     }
   }
+  s->path = NEKOAMD_BY_LAUNCHES;
   if (s->prec == NEKOAMD_CG_FP64) {
     if ((status = start64())) return status;
     double* X = (double*)x;
@@ -1935,6 +1957,7 @@ int nekoamd_cg_solve3(void* const* cg, void* const* x, const void* const* f,
     rc = nekoamd_cg_status(cg[c], &mon[c]);
     if (rc) return rc;
     s[c]->last_iter = mon[c].iter;
+    s[c]->path = NEKOAMD_COUPLED;
   }
   return kOk;
 }

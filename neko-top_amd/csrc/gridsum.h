@@ -15,7 +15,8 @@
 // every workgroup is past reading it.
 //
 // All workgroups must be resident at once: the launcher bounds the grid by
-// the occupancy of an empty device.  A wait lasts at most kGridWait; a
+// the occupancy of an empty device.  A wait lasts at most `wait` ticks of the
+// 100 MHz clock (0: it is given up before the words are looked at); a
 // workgroup that gives up leaves, and so the others do.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -24,7 +25,8 @@
 
 namespace nekoamd {
 
-constexpr unsigned long long kGridWait = 100000000ull;  // 1 s at 100 MHz
+constexpr unsigned long long kGridTicks = 100;  // of the clock, per us
+constexpr unsigned long long kGridWait = 1000000 * kGridTicks;  // default, 1 s
 
 template <typename T>
 __device__ __forceinline__ T dev_load(const T* p) {
@@ -50,12 +52,12 @@ __device__ __forceinline__ void grid_put(uint64_t* s, uint32_t tag, double v) {
 // the first n of them count.  *fail = 1 if the wait was given up.
 template <int N>
 __device__ __forceinline__ void grid_get(const uint64_t* const (&s)[N], int n,
-                                         uint32_t tag, int* fail,
-                                         double (&out)[N]) {
+                                         uint32_t tag, unsigned long long wait,
+                                         int* fail, double (&out)[N]) {
   const unsigned long long t0 = wall_clock64();
   for (;;) {
     uint64_t w[2 * N];
-    bool here = true;
+    bool here = wait != 0;
 #pragma unroll
     for (int j = 0; j < N; ++j)
       if (j < n) {
@@ -71,7 +73,7 @@ __device__ __forceinline__ void grid_get(const uint64_t* const (&s)[N], int n,
             (long long)((w[2 * j] & 0xFFFFFFFFull) | (w[2 * j + 1] << 32)));
       }
     if (here) return;
-    if (wall_clock64() - t0 > kGridWait) {
+    if (wall_clock64() - t0 >= wait) {
       *fail = 1;
       return;
     }
@@ -91,13 +93,14 @@ __device__ __forceinline__ void grid_publish(uint64_t* slots, int wg,
 // Every thread of a workgroup: the sums over the nwg slots of this tag, the
 // same value in every thread of every workgroup (blockDim.x, a multiple of
 // 64, must be the same in all).  Slots t, t + NT, .. are added by thread t <
-// NT (0: blockDim.x), then as block_sum (reduce.h) adds.  sh: NV doubles per wave of the workgroup;
-// *fail: a shared int that is 0, set if a wait was given up.  Returns false
+// NT (0: blockDim.x), then as block_sum (reduce.h) adds.  sh: NV doubles per
+// wave of the workgroup; *fail: a shared int that is 0, set if a wait was given up.  Returns false
 // (in every thread) in that case.  sh may be written again after the next
 // workgroup barrier.
 template <int NV, int NT = 0>
 __device__ __forceinline__ bool grid_sum(const uint64_t* slots, int nwg,
-                                         uint32_t tag, double* sh, int* fail,
+                                         uint32_t tag, unsigned long long wait,
+                                         double* sh, int* fail,
                                          double (&out)[NV]) {
   double v[NV];
 #pragma unroll
@@ -109,7 +112,7 @@ __device__ __forceinline__ bool grid_sum(const uint64_t* slots, int nwg,
     double p[NV];
 #pragma unroll
     for (int j = 0; j < NV; ++j) s[j] = slots + ((int64_t)q * NV + j) * 2;
-    grid_get<NV>(s, NV, tag, fail, p);
+    grid_get<NV>(s, NV, tag, wait, fail, p);
 #pragma unroll
     for (int j = 0; j < NV; ++j) v[j] += p[j];
   }

@@ -1322,7 +1322,8 @@ __global__ void __launch_bounds__(kCB) crs_grid_k(CrsGrid g) {
     __syncthreads();
     if ((tid & (kHB - 1)) == 0) crs_publish(slot_r, tag, s1, wv, nblk);
     prev = rz[0];
-    if (!(ok = (grid_sum<1, kHB>(slot_r, nblk, tag, s2, &fail, rz)))) break;
+    if (!(ok = (grid_sum<1, kHB>(slot_r, nblk, tag, kGridWait, s2, &fail, rz))))
+      break;
     const double beta = q > 0 && prev != 0.0 ? rz[0] / prev : 0.0;
     // p on the halo from the other workgroups' z, on the own range from z
     for (int i = tid; i < 2 * g.halo; i += kCB) {
@@ -1331,7 +1332,7 @@ __global__ void __launch_bounds__(kCB) crs_grid_k(CrsGrid g) {
       if (u < 0 || u >= nl) continue;
       const uint64_t* src[1] = {g.zw + 2 * (int64_t)u};
       double zu[1];
-      grid_get<1>(src, 1, tag, &fail, zu);
+      grid_get<1>(src, 1, tag, kGridWait, &fail, zu);
       p[j] = zu[0] + beta * p[j];
     }
     const double pv = z + beta * p[g.halo + tid];
@@ -1351,7 +1352,8 @@ __global__ void __launch_bounds__(kCB) crs_grid_k(CrsGrid g) {
     __syncthreads();
     if ((tid & (kHB - 1)) == 0) crs_publish(slot_p, tag + 1u, s3, wv, nblk);
     // past this every workgroup has read z, so the next may overwrite it
-    if (!(ok = (grid_sum<1, kHB>(slot_p, nblk, tag + 1u, s4, &fail, pap)))) break;
+    if (!(ok = (grid_sum<1, kHB>(slot_p, nblk, tag + 1u, kGridWait, s4, &fail, pap))))
+      break;
     const double alpha = pap[0] != 0.0 ? rz[0] / pap[0] : 0.0;
     x += alpha * pv;
     r -= alpha * w;

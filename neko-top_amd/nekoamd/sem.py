@@ -251,6 +251,20 @@ class CG:
             ri(1 if ifh2 else 0), C.byref(mon)), "cg_solve")
         return mon
 
+    BY_LAUNCHES, ONE_KERNEL, COUPLED = 0, 1, 2
+
+    @property
+    def path(self):
+        """How the last solve ran: BY_LAUNCHES, ONE_KERNEL or COUPLED."""
+        p = C.c_int(-1)
+        check(lib().nekoamd_cg_path(C.c_void_p(self.h), C.byref(p)), "cg_path")
+        return p.value
+
+    def set_wait(self, us):
+        """The longest wait of the one-kernel solve's workgroups
+        (nekoamd_cg_set_wait)."""
+        check(lib().nekoamd_cg_set_wait(C.c_void_p(self.h), ri64(us)), "cg_set_wait")
+
     @staticmethod
     def solve3(cgs, xs, fs, d, mask, h1, h2=None, ifh2=False, abstol=1e-8, max_iter=800,
                poll=8):

@@ -536,6 +536,7 @@ def test_cg_small_meshes(box, mixed, ifh2, sem):
         ref, it, r0, r1 = o.cg(f, mask, h1, h2, ifh2, abstol=abstol, max_iter=max_iter)
         mon = cg.solve(x, g.field(f), d, g.mask(faces), h1d, h2d, ifh2, abstol=abstol,
                        max_iter=max_iter)
+        assert cg.path == cg.ONE_KERNEL
         assert abs(mon.res_start - r0) <= 1e-12 * r0
         if abstol == 0.0:
             # four iterations: sums of up to 1e5 terms, each of eps relative
@@ -566,3 +567,35 @@ def test_cg_small_mesh_over_many_iterations(sem):
     ref = o.cg(f, mask, abstol=1e-12, max_iter=2000)[0]
     assert mon.iter == 2100
     assert np.abs(x.get() - ref).max() <= 1e-9 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("box", [(1, 1, 1, 4), (5, 4, 3, 6), (8, 8, 4, 8)])
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("wait", [0, 2])
+def test_cg_small_mesh_with_waits_given_up(box, mixed, wait, sem):
+    """The one-kernel solve with waits of at most 0 us (all given up: it
+    starts over with launches, and so does the next solve from its start) and
+    2 us (about one exchange: either way): the solution is the oracle's.  A
+    new wait lets the state try the kernel again."""
+    g = sem.BoxCase(*box, jitter=0.05, seed=1234)
+    o = oracle.build_case(*box, jitter=0.05, seed=1234)
+    mask = oracle.face_mask(*box, sem.PRS_DIRICHLET)
+    f = o.gs(o.B * np.random.default_rng(3).uniform(-1, 1, o.n))
+    f[mask] = 0.0
+    ref, it, r0, _ = o.cg(f, mask, np.ones(o.n), None, False, abstol=1e-9, max_iter=3000)
+    h1, d, x = g.field(np.ones(g.n)), g.field(), g.field()
+    g.jacobi(d, h1)
+    cg = sem.CG(g, mixed=mixed)
+    cg.set_wait(wait)
+    for us, path in ((None, cg.BY_LAUNCHES), (None, cg.BY_LAUNCHES), (10**6, cg.ONE_KERNEL)):
+        if us is not None:
+            cg.set_wait(us)
+        x.upload(np.full(g.n, 7.0))
+        mon = cg.solve(x, g.field(f), d, g.mask(sem.PRS_DIRICHLET), h1, abstol=1e-9,
+                       max_iter=3000)
+        assert cg.path == path or (wait == 2 and us is None and cg.path == cg.ONE_KERNEL)
+        assert mon.done == 1 and mon.res_final < 1e-9
+        assert abs(mon.res_start - r0) <= 1e-6 * r0  # FP32 start in mixed launches
+        # FP32 iterations need more of them
+        assert abs(mon.iter - it) <= (1 if not mixed or cg.path == cg.ONE_KERNEL else it + 20)
+        assert np.abs(x.get() - ref).max() <= 1e-5 * np.abs(ref).max()
