@@ -311,6 +311,7 @@ int nekoamd_cg_set_wait(void* cg, const int64_t* us);
 #define NEKOAMD_BY_LAUNCHES 0   /* a handful of launches per iteration */
 #define NEKOAMD_ONE_KERNEL 1    /* one kernel that keeps the vectors */
 #define NEKOAMD_COUPLED 2       /* nekoamd_cg_solve3's coupled launches */
+#define NEKOAMD_ONE_WORKGROUP 3 /* nekoamd_hsmg_path only */
 int nekoamd_cg_path(void* cg, int* path);
 /* x = A^-1 f for A = QQ^T (h1 A_L + h2 B) with the Dirichlet mask (0-based
  * indices mask[0..nmask)), preconditioned by the Jacobi diagonal d
@@ -415,6 +416,15 @@ int nekoamd_hsmg_create(void** st, const int* nx, const int* ny, const int* nz,
                         const int* dirichlet_faces, const int* crs_iter,
                         const int* precision);
 int nekoamd_hsmg_free(void* st);
+/* The coarse solve of a lattice that fits the device is one kernel whose
+ * workgroups wait for one another at most us microseconds (default 1e6; 0:
+ * every wait is given up at once).  The application that gives one up, and
+ * those already queued, are finished by one workgroup; later ones take
+ * launches, until this is called again (it synchronises).  path: how the last
+ * application's coarse solve ran (NEKOAMD_BY_LAUNCHES, also before the first,
+ * NEKOAMD_ONE_KERNEL or NEKOAMD_ONE_WORKGROUP; it synchronises). */
+int nekoamd_hsmg_set_wait(void* st, const int64_t* us);
+int nekoamd_hsmg_path(void* st, int* path);
 int nekoamd_hsmg_apply(void* st, void* z, const void* r);
 
 

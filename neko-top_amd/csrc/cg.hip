@@ -1358,31 +1358,17 @@ static int cg_drive(CgState* s, int max_iter, int batch, F&& queue_batch) {
   return status;
 }
 
-// Workgroups of cg_grid_k on this device at once (0: it does not fit).
-template <int LX, int EPB, bool H2>
-static int cg_grid_room(int nelv, int* wg) {
-  constexpr int BS = (LX * LX * LX * EPB + 63) / 64 * 64;
-  *wg = (nelv + EPB - 1) / EPB;
-  if (*wg > kGridWg) return 0;
-  int dev = 0, cus = 0, per = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
-                            dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &per, (const void*)cg_grid_k<LX, EPB, H2>, BS, 0) != hipSuccess)
-    return 0;
-  return cus * per;
-}
-
 // One launch of up to kGridCap iterations; *ran = false where the mesh does
 // not fit.
 template <int LX, int EPB, bool H2>
 static int cg_grid_launch(const CgGrid& a, bool* ran) {
-  int wg = 0;
-  *ran = cg_grid_room<LX, EPB, H2>(a.nelv, &wg) >= wg;
+  constexpr int BS = (LX * LX * LX * EPB + 63) / 64 * 64;
+  const int wg = (a.nelv + EPB - 1) / EPB;
+  *ran = wg <= kGridWg &&
+         grid_room((const void*)cg_grid_k<LX, EPB, H2>, BS, 0) >= wg;
   if (!*ran) return kOk;
-  hipLaunchKernelGGL((cg_grid_k<LX, EPB, H2>), dim3(wg),
-                     dim3((LX * LX * LX * EPB + 63) / 64 * 64), 0, stream(), a);
+  hipLaunchKernelGGL((cg_grid_k<LX, EPB, H2>), dim3(wg), dim3(BS), 0, stream(),
+                     a);
   NK_LAUNCHED();
   return kOk;
 }

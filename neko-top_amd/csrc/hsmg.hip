@@ -94,9 +94,15 @@ struct Hsmg {
   double *S27 = nullptr, *dl = nullptr, *xl = nullptr, *rl = nullptr,
          *zl = nullptr, *wl = nullptr, *pl[2] = {}, *cpart = nullptr;
   // crs_grid_k (null: not used): its stuck flag, then the words its
-  // workgroups exchange; the next unused tag
+  // workgroups exchange; the next unused tag; the longest wait; in pinned
+  // memory, whether crs_one_k has taken over; whether the last application
+  // took the launches
   uint64_t* cwords = nullptr;
+  int halo = 0;
   uint32_t ctag = 1;
+  unsigned long long wait = kGridWait;
+  int* took_over = nullptr;
+  bool by_launches = true;
   // the coarse solve (fixed kernels on fixed buffers), recorded as a graph on
   // the first application and replayed (NEKOAMD_HIP_GRAPHS=1)
   hipGraphExec_t crs_graph = nullptr;
@@ -1250,7 +1256,8 @@ struct CrsGrid {
   const double *r1, *dl, *S;
   double* e1;
   uint64_t *slots, *zw;  // partial sums (4 words per kHB vertices), z (2 per vertex)
-  int* stuck;
+  unsigned long long wait;
+  int *stuck, *took_over;
   double *xl, *rl, *zl, *wl, *pl;  // crs_one_k only
 };
 
@@ -1284,6 +1291,9 @@ __global__ void __launch_bounds__(kCB) crs_grid_k(CrsGrid g) {
   __shared__ double s1[kCB / 64], s2[kCB / 64], s3[kCB / 64], s4[kCB / 64];
   __shared__ int fail;
   const int tid = threadIdx.x, wv = tid >> 6;
+  // no wait after one that an earlier application gave up
+  const unsigned long long wait =
+      __builtin_amdgcn_readfirstlane(*g.stuck) != 0 ? 0 : g.wait;
   const int nxl = g.nx + 1, nyl = g.ny + 1, nxy = nxl * nyl;
   const int nl = nxy * (g.nz + 1);
   const int v0 = blockIdx.x * kCB, v = v0 + tid;
@@ -1322,7 +1332,7 @@ __global__ void __launch_bounds__(kCB) crs_grid_k(CrsGrid g) {
     __syncthreads();
     if ((tid & (kHB - 1)) == 0) crs_publish(slot_r, tag, s1, wv, nblk);
     prev = rz[0];
-    if (!(ok = (grid_sum<1, kHB>(slot_r, nblk, tag, kGridWait, s2, &fail, rz))))
+    if (!(ok = (grid_sum<1, kHB>(slot_r, nblk, tag, wait, s2, &fail, rz))))
       break;
     const double beta = q > 0 && prev != 0.0 ? rz[0] / prev : 0.0;
     // p on the halo from the other workgroups' z, on the own range from z
@@ -1332,7 +1342,7 @@ __global__ void __launch_bounds__(kCB) crs_grid_k(CrsGrid g) {
       if (u < 0 || u >= nl) continue;
       const uint64_t* src[1] = {g.zw + 2 * (int64_t)u};
       double zu[1];
-      grid_get<1>(src, 1, tag, kGridWait, &fail, zu);
+      grid_get<1>(src, 1, tag, wait, &fail, zu);
       p[j] = zu[0] + beta * p[j];
     }
     const double pv = z + beta * p[g.halo + tid];
@@ -1352,7 +1362,7 @@ __global__ void __launch_bounds__(kCB) crs_grid_k(CrsGrid g) {
     __syncthreads();
     if ((tid & (kHB - 1)) == 0) crs_publish(slot_p, tag + 1u, s3, wv, nblk);
     // past this every workgroup has read z, so the next may overwrite it
-    if (!(ok = (grid_sum<1, kHB>(slot_p, nblk, tag + 1u, kGridWait, s4, &fail, pap))))
+    if (!(ok = (grid_sum<1, kHB>(slot_p, nblk, tag + 1u, wait, s4, &fail, pap))))
       break;
     const double alpha = pap[0] != 0.0 ? rz[0] / pap[0] : 0.0;
     x += alpha * pv;
@@ -1366,9 +1376,12 @@ __global__ void __launch_bounds__(kCB) crs_grid_k(CrsGrid g) {
   if (live) lattice_put(g.e1, g.nx, g.ny, g.nz, a, b, c, x);
 }
 
-// The same solve by one workgroup if crs_grid_k got stuck (another process
-// holding the device); else nothing.  kHB threads: an empty launch of 1024
-// waited 25 us for a CU with room beside the Schwarz kernels.
+// The same solve by one workgroup (its sums in another order) if crs_grid_k
+// got stuck, now or before (another process holding the device); else
+// nothing.  The flag stays set, so what is already queued neither waits again
+// nor goes without its result, and the host turns to the launches when it
+// sees took_over.  kHB threads: an empty launch of 1024 waited 25 us for a CU
+// with room beside the Schwarz kernels.
 __global__ void __launch_bounds__(kHB) crs_one_k(CrsGrid g) {
   __shared__ double sh[kHB / 64 + 1];
   if (*g.stuck == 0) return;
@@ -1429,20 +1442,27 @@ __global__ void __launch_bounds__(kHB) crs_one_k(CrsGrid g) {
   for (int v = threadIdx.x; v < nl; v += kHB)
     lattice_put(g.e1, g.nx, g.ny, g.nz, v % nxl, (v / nxl) % nyl, v / nxy,
                 g.xl[v]);
-  __syncthreads();
-  if (threadIdx.x == 0) *g.stuck = 0;
+  if (threadIdx.x == 0) *g.took_over = 1;
 }
 
+unsigned crs_grid_lds(int halo) {
+  return (unsigned)((kCB + 2 * halo) * sizeof(double));
+}
+int crs_grid_wgs(const Hsmg* h) { return (int)((h->nl + kCB - 1) / kCB); }
+
 // Halo of crs_grid_k's ranges, or 0 if the lattice is not one of its: the
-// ranges must fit 64 KB of LDS (lattice planes of up to 56 x 56 or so) and
+// ranges must fit 60 KB of LDS (lattice planes of up to 58 x 58 elements) and
 // 256 workgroups (131072 vertices), which are also the block partials of the
-// other form.  Its workgroups find room beside the Schwarz kernels of the
-// library stream as those' workgroups retire.
+// other form, and an empty device must hold them all at once.  They find room
+// beside the Schwarz kernels of the library stream as those' workgroups
+// retire.
 int crs_grid_halo(const Hsmg* h) {
   const int64_t halo = (int64_t)(h->nx + 1) * (h->ny + 1) + h->nx + 2;
   const bool fits = !h->graphs &&
                     (kCB + 2 * halo) * (int64_t)sizeof(double) <= 60 * 1024 &&
-                    h->nl <= 256 * (int64_t)kCB;
+                    h->nl <= 256 * (int64_t)kCB &&
+                    grid_room((const void*)crs_grid_k, kCB,
+                              crs_grid_lds((int)halo)) >= crs_grid_wgs(h);
   return fits ? (int)halo : 0;
 }
 
@@ -1451,14 +1471,17 @@ int crs_grid_halo(const Hsmg* h) {
 // the launch stream (or the latter recorded as kernel nodes).
 int coarse_pcg(Hsmg* h) {
   const int G = h->crs_G, it = h->crs_iter;
-  if (h->cwords) {
-    const int halo = crs_grid_halo(h), wg = (int)((h->nl + kCB - 1) / kCB);
-    CrsGrid g{h->nx, h->ny, h->nz, h->faces, it, halo, h->ctag, h->r1, h->dl,
-              h->S27, h->e1, h->cwords + 1, h->cwords + 1 + 8 * wg,
-              (int*)h->cwords, h->xl, h->rl, h->zl, h->wl, h->pl[0]};
+  // took_over: written by a kernel that may still be running, read at any
+  // time from then on
+  h->by_launches = !h->cwords || *(volatile int*)h->took_over;
+  if (!h->by_launches) {
+    const int wg = crs_grid_wgs(h);
+    CrsGrid g{h->nx, h->ny, h->nz, h->faces, it, h->halo, h->ctag, h->r1, h->dl,
+              h->S27, h->e1, h->cwords + 1, h->cwords + 1 + 8 * wg, h->wait,
+              (int*)h->cwords, h->took_over, h->xl, h->rl, h->zl, h->wl,
+              h->pl[0]};
     h->ctag += 2u * (uint32_t)it;
-    nk_launch(crs_grid_k, dim3(wg), dim3(kCB),
-              (unsigned)((kCB + 2 * halo) * sizeof(double)), g);
+    nk_launch(crs_grid_k, dim3(wg), dim3(kCB), crs_grid_lds(h->halo), g);
     NK_LAUNCHED();
     nk_launch(crs_one_k, dim3(1), dim3(kHB), 0, g);
     NK_LAUNCHED();
@@ -1505,6 +1528,7 @@ void hsmg_destroy(Hsmg* h) {
                   (void*)h->wl, (void*)h->pl[0], (void*)h->pl[1],
                   (void*)h->cpart, (void*)h->cwords})
     if (p) (void)hipFree(p);
+  if (h->took_over) (void)hipHostFree(h->took_over);
   if (h->crs_graph) (void)hipGraphExecDestroy(h->crs_graph);
   if (h->side) {
     (void)hipStreamSynchronize(h->side);
@@ -1528,8 +1552,8 @@ static bool graphs_requested() {
 // stream (default priority) once r1 is ready, so that they run under the
 // fine and mid Schwarz steps; ev_crs is recorded when they are done and the
 // library stream waits on it before reading e1 (coarse_join).  Without
-// graphs the 1 + 2 crs_iter kernels are queued on the side stream; with
-// graphs they are one graph launch there, the graph built on the first call
+// graphs coarse_pcg's kernels are queued on the side stream; with graphs its
+// 1 + 2 crs_iter launches are one graph launch there, built on the first call
 // by recording coarse_pcg's launches as kernel nodes (LaunchRecorder), not
 // by stream capture: nothing is queued on any stream while it is built.
 int coarse_solve(Hsmg* h) {
@@ -1644,11 +1668,15 @@ int coarse_lattice_setup(Hsmg* h) {
     if (e == hipSuccess) e = hipMalloc(p, vb);
   if (e == hipSuccess)
     e = hipMalloc(&h->cpart, sizeof(double) * 2 * (size_t)h->crs_iter * h->crs_G);
-  if (e == hipSuccess && crs_grid_halo(h) > 0) {
-    const size_t wb = sizeof(uint64_t) *
-                      (1 + 8 * (size_t)((nl + kCB - 1) / kCB) + 2 * (size_t)nl);
+  h->halo = crs_grid_halo(h);
+  if (e == hipSuccess && h->halo > 0) {
+    const size_t wb =
+        sizeof(uint64_t) * (1 + 8 * (size_t)crs_grid_wgs(h) + 2 * (size_t)nl);
     e = hipMalloc(&h->cwords, wb);
     if (e == hipSuccess) e = hipMemset(h->cwords, 0, wb);
+    if (e == hipSuccess)
+      e = hipHostMalloc((void**)&h->took_over, sizeof(int), hipHostMallocDefault);
+    if (e == hipSuccess) *h->took_over = 0;
   }
   if (e == hipSuccess) e = hipMemcpy(h->S27, S.data(), 27 * vb, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(h->dl, dl.data(), vb, hipMemcpyHostToDevice);
@@ -1850,6 +1878,29 @@ int nekoamd_hsmg_free(void* st) {
   if (!st) return kOk;
   NK_HIP(hipStreamSynchronize(stream()));
   hsmg_destroy(static_cast<Hsmg*>(st));
+  return kOk;
+}
+
+int nekoamd_hsmg_set_wait(void* st, const int64_t* us) {
+  NK_INIT();
+  auto* h = static_cast<Hsmg*>(st);
+  NK_REQUIRE(h && us, "null argument");
+  NK_REQUIRE(*us >= 0 && *us <= 1000000000, "wait outside [0, 1e9] us");
+  h->wait = (unsigned long long)*us * kGridTicks;
+  if (!h->cwords) return kOk;
+  NK_HIP(hipStreamSynchronize(stream()));
+  NK_HIP(hipMemset(h->cwords, 0, sizeof(uint64_t)));
+  *h->took_over = 0;
+  return kOk;
+}
+
+int nekoamd_hsmg_path(void* st, int* path) {
+  NK_INIT();
+  auto* h = static_cast<Hsmg*>(st);
+  NK_REQUIRE(h && path, "null argument");
+  NK_HIP(hipStreamSynchronize(stream()));
+  *path = h->by_launches ? NEKOAMD_BY_LAUNCHES
+          : *(volatile int*)h->took_over ? NEKOAMD_ONE_WORKGROUP : NEKOAMD_ONE_KERNEL;
   return kOk;
 }
 

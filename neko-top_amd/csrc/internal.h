@@ -176,6 +176,10 @@ template <typename T>
 int gs_launch3(void* gs, T* const* u, int op, const int* const* skip,
                const bool* active);
 
+// Workgroups of a kernel (threads, LDS bytes beyond its static ones) that an
+// empty device holds at once; 0 if that cannot be told.
+int grid_room(const void* kernel, int threads, size_t lds);
+
 // The gs map seen from its points: (*ref)[l] = {offset into *idx of the tuple
 // point l is in, its multiplicity}, {0, 0} for a point in none.  Made on the
 // first call and kept with the map; *ok = false (and nothing made) if a

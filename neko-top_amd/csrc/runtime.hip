@@ -31,6 +31,17 @@ int fail_arg(const char* where, const char* what) {
 }
 
 hipStream_t stream() { return g_stream; }
+
+int grid_room(const void* kernel, int threads, size_t lds) {
+  int dev = 0, cus = 0, per = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
+                            dev) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads,
+                                                   lds) != hipSuccess)
+    return 0;
+  return cus * per;
+}
 LaunchRecorder*& launch_recorder() {
   static thread_local LaunchRecorder* rec = nullptr;
   return rec;

@@ -381,6 +381,21 @@ class HSMG:
     def apply(self, z, r):
         check(lib().nekoamd_hsmg_apply(C.c_void_p(self.h), ptr(z), ptr(r)), "hsmg_apply")
 
+    BY_LAUNCHES, ONE_KERNEL, ONE_WORKGROUP = 0, 1, 3
+
+    @property
+    def path(self):
+        """How the last application's coarse solve ran: BY_LAUNCHES,
+        ONE_KERNEL or ONE_WORKGROUP."""
+        p = C.c_int(-1)
+        check(lib().nekoamd_hsmg_path(C.c_void_p(self.h), C.byref(p)), "hsmg_path")
+        return p.value
+
+    def set_wait(self, us):
+        """The longest wait of the coarse kernel's workgroups
+        (nekoamd_hsmg_set_wait)."""
+        check(lib().nekoamd_hsmg_set_wait(C.c_void_p(self.h), ri64(us)), "hsmg_set_wait")
+
     def __del__(self):
         try:
             lib().nekoamd_hsmg_free(C.c_void_p(self.h))

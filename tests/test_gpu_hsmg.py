@@ -51,8 +51,8 @@ def test_repeated_applies_match_oracle(pair, graphs, monkeypatch):
     and host reads) between them, each within the bar.  With
     NEKOAMD_HIP_GRAPHS=1 when the multigrid is created, its coarse solve is a
     HIP graph recorded from kernel nodes on the first application and replayed
-    on a side stream after: every replay equals the kernel-by-kernel result
-    bit for bit (the same kernels in the same order)."""
+    on a side stream after: every replay equals the one-kernel result bit for
+    bit (the same sums in the same order)."""
     from nekoamd import sem
     g, M, Mo = pair
     Mg = None
@@ -168,3 +168,48 @@ def test_coarse_kernel_equals_launches(box, monkeypatch):
         Mg.apply(zg, r)
         assert np.array_equal(z.get(), zg.get()) and np.isfinite(z.get()).all()
         assert z.get().any()
+        assert Mg.path == Mg.BY_LAUNCHES
+        assert M.path == (M.BY_LAUNCHES if box[0] > 58 else M.ONE_KERNEL)
+
+
+@pytest.mark.parametrize("box", [(1, 1, 1), (12, 9, 7), (16, 16, 16)])
+def test_coarse_kernel_with_waits_given_up(box, monkeypatch):
+    """All waits of the coarse kernel given up at once: the application is
+    finished by one workgroup (its sums in another order: the rounding of ten
+    iterations of a preconditioner, 1e-12), the next ones take the launches
+    (bit for bit) and a new wait the kernel again.  Three applications queued
+    without a host wait between them are right whichever of the two ways
+    each takes."""
+    from nekoamd import device, sem
+    device.init(0)
+    g = sem.BoxCase(*box, 4, jitter=0.05, seed=1234)
+    M = sem.HSMG(g)
+    monkeypatch.setenv("NEKOAMD_HIP_GRAPHS", "1")
+    Mg = sem.HSMG(g)
+    rng = np.random.default_rng(6)
+    rs = [g.field(rng.standard_normal(g.n)) for _ in range(3)]
+    zs = [g.field() for _ in rs]
+    want = []
+    for r, z in zip(rs, zs):
+        g.gs.op(r)
+        Mg.apply(z, r)
+        want.append(z.get())
+
+    def close(z, w):
+        return np.abs(z.get() - w).max() <= 1e-12 * np.abs(w).max()
+
+    z = zs[0]
+    M.set_wait(0)
+    M.apply(z, rs[0])
+    assert M.path == M.ONE_WORKGROUP and close(z, want[0])
+    for k in (1, 2):
+        M.apply(z, rs[k])
+        assert M.path == M.BY_LAUNCHES and np.array_equal(z.get(), want[k])
+    M.set_wait(10**6)
+    M.apply(z, rs[0])
+    assert M.path == M.ONE_KERNEL and np.array_equal(z.get(), want[0])
+    M.set_wait(0)
+    for r, z in zip(rs, zs):
+        M.apply(z, r)
+    device.sync()
+    assert all(close(z, w) for z, w in zip(zs, want))
