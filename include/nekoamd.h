@@ -305,7 +305,7 @@ int nekoamd_cg_free(void* cg);
  * us microseconds (default 1e6; 0: every wait is given up at once).  A solve
  * that gives one up, because another process holds the device, starts over
  * with launches, and this state's later solves take them from the start,
- * until this is called again. */
+ * until this is called again.  us < 0: launches from the first solve on. */
 int nekoamd_cg_set_wait(void* cg, const int64_t* us);
 /* How the state's last solve ran. */
 #define NEKOAMD_BY_LAUNCHES 0   /* a handful of launches per iteration */

@@ -1701,9 +1701,9 @@ int nekoamd_cg_status(void* cg, nekoamd_cg_monitor_t* mon) {
 int nekoamd_cg_set_wait(void* cg, const int64_t* us) {
   CgState* s = as_cg(cg);
   NK_REQUIRE(s && us, "null argument");
-  NK_REQUIRE(*us >= 0 && *us <= 1000000000, "wait outside [0, 1e9] us");
-  s->wait = (unsigned long long)*us * kGridTicks;
-  s->grid_off = false;
+  NK_REQUIRE(*us <= 1000000000, "wait above 1e9 us");
+  s->grid_off = *us < 0;
+  s->wait = (unsigned long long)std::max<int64_t>(*us, 0) * kGridTicks;
   return kOk;
 }
 

@@ -238,9 +238,25 @@ def test_jacobi_parity(cases, key):
     assert rel_max(d.get(), ref) < 1e-12
 
 
+# a small mesh's solve is one kernel; the launches of larger ones on it too
+WAYS = pytest.mark.parametrize("launches", [False, True], ids=["one_kernel", "launches"])
+
+
+def _cg(sem, g, launches, mixed=False):
+    cg = sem.CG(g, mixed=mixed)
+    if launches:
+        cg.set_wait(-1)
+    return cg
+
+
+def _check_way(cg, launches, by_launches=0):
+    assert cg.path == (by_launches if launches else cg.ONE_KERNEL)
+
+
 @pytest.mark.parametrize("key", ["cfg1", "p7"])
 @pytest.mark.parametrize("kind", ["pressure", "velocity"])
-def test_cg_parity(cases, key, kind, sem):
+@WAYS
+def test_cg_parity(cases, key, kind, launches, sem):
     g, o = cases[key]
     rng = np.random.default_rng(11)
     if kind == "pressure":
@@ -257,9 +273,10 @@ def test_cg_parity(cases, key, kind, sem):
     h1d = g.field(h1)
     h2d = g.field(h2) if ifh2 else None
     g.jacobi(d, h1d, h2d, ifh2)
-    cg = sem.CG(g)
+    cg = _cg(sem, g, launches)
     x = g.field()
     mon = cg.solve(x, g.field(f), d, g.mask(faces), h1d, h2d, ifh2, abstol=1e-8, max_iter=800)
+    _check_way(cg, launches)
     xg = x.get()
     print(f"cg {kind} {key}: iters gpu {mon.iter} oracle {it_ref}; "
           f"res {mon.res_final:.3e} / {r1_ref:.3e}")
@@ -279,7 +296,8 @@ def _true_residual(o, x, f, mask, h1, h2, ifh2):
 
 @pytest.mark.parametrize("key", ["cfg1", "p7"])
 @pytest.mark.parametrize("kind", ["pressure", "velocity"])
-def test_cg_mixed_reaches_fp64_tolerance(cases, key, kind, sem):
+@WAYS
+def test_cg_mixed_reaches_fp64_tolerance(cases, key, kind, launches, sem):
     """FP32 iterations with FP64 reliable updates: the FP64 residual the
     solve reports is the oracle's residual of the returned x (to 1e-2
     relative: it is ~1e-8 against an |f| of ~1), it is below 1e-8, x agrees
@@ -301,9 +319,10 @@ def test_cg_mixed_reaches_fp64_tolerance(cases, key, kind, sem):
     h1d = g.field(h1)
     h2d = g.field(h2) if ifh2 else None
     g.jacobi(d, h1d, h2d, ifh2)
-    cg = sem.CG(g, mixed=True)
+    cg = _cg(sem, g, launches, mixed=True)
     x = g.field()
     mon = cg.solve(x, g.field(f), d, g.mask(faces), h1d, h2d, ifh2, abstol=1e-8, max_iter=800)
+    _check_way(cg, launches)
     xg = x.get()
     res_true = _true_residual(o, xg, f, mask, h1, h2, ifh2)
     print(f"cg mixed {kind} {key}: iters {mon.iter} (fp64 oracle {it_ref}), "
@@ -320,12 +339,13 @@ def test_cg_mixed_reaches_fp64_tolerance(cases, key, kind, sem):
     assert np.all(xg[mask] == 0.0)
 
 
-def test_cg_mixed_max_iter_and_zero_rhs(cases, sem):
+@WAYS
+def test_cg_mixed_max_iter_and_zero_rhs(cases, launches, sem):
     g, o = cases["cfg1"]
     d = g.field()
     h1 = g.field(np.ones(g.n))
     g.jacobi(d, h1)
-    cg = sem.CG(g, mixed=True)
+    cg = _cg(sem, g, launches, mixed=True)
     x = g.field()
     f = o.gs(o.B)
     mask = oracle.face_mask(g.nx, g.ny, g.nz, g.lx, sem.PRS_DIRICHLET)
@@ -338,16 +358,18 @@ def test_cg_mixed_max_iter_and_zero_rhs(cases, sem):
     assert abs(mon.res_final - res_true) < 1e-6 * res_true
     assert abs(mon.res_final - r1_ref) < 1e-4 * r1_ref
     mon = cg.solve(x, g.field(), d, g.mask(sem.PRS_DIRICHLET), h1, abstol=1e-8, max_iter=50)
+    _check_way(cg, launches)
     assert mon.iter == 0 and mon.res_start == 0.0
     assert not x.get().any()
 
 
-def test_cg_max_iter_and_zero_rhs(cases, sem):
+@WAYS
+def test_cg_max_iter_and_zero_rhs(cases, launches, sem):
     g, o = cases["cfg1"]
     d = g.field()
     h1 = g.field(np.ones(g.n))
     g.jacobi(d, h1)
-    cg = sem.CG(g)
+    cg = _cg(sem, g, launches)
     x = g.field()
     f = o.gs(o.B)
     mask = oracle.face_mask(g.nx, g.ny, g.nz, g.lx, sem.PRS_DIRICHLET)
@@ -357,6 +379,7 @@ def test_cg_max_iter_and_zero_rhs(cases, sem):
     assert mon.iter == 5 == it_ref
     assert abs(mon.res_final - r1_ref) < 1e-10 * r1_ref
     mon = cg.solve(x, g.field(), d, g.mask(sem.PRS_DIRICHLET), h1, abstol=1e-8, max_iter=50)
+    _check_way(cg, launches)
     assert mon.iter == 0 and mon.res_start == 0.0
     assert not x.get().any()
 
@@ -458,9 +481,10 @@ def test_gs_mass_average(cases, key, sem):
 
 
 @pytest.mark.parametrize("key", ["cfg1", "p7"])
-def test_cg_solve3_matches_separate_solves(cases, key, sem):
+@WAYS
+def test_cg_solve3_matches_separate_solves(cases, key, launches, sem):
     """The coupled mixed solve (one set-up and one driver for the three
-    components) against three separate mixed solves and the FP64 oracle:
+    components; on a small mesh one kernel a component) against three separate mixed solves and the FP64 oracle:
     every component reaches an FP64 residual < 1e-8 (the oracle's residual
     of its x agrees), x within 1e-6 of the oracle's FP64 solve and within
     1e-7 of its separate solve, and iteration counts within 2 of the
@@ -484,14 +508,15 @@ def test_cg_solve3_matches_separate_solves(cases, key, sem):
     fd = [g.field(f) for f in fs]
     sep, mons = [], []
     for c in range(3):
-        cg = sem.CG(g, mixed=True)
+        cg = _cg(sem, g, launches, mixed=True)
         x = g.field()
         mons.append(cg.solve(x, fd[c], d, dmask, h1d, h2d, ifh2, abstol=1e-8, max_iter=800))
         sep.append(x.get())
-    cgs = [sem.CG(g, mixed=True) for _ in range(3)]
+    cgs = [_cg(sem, g, launches, mixed=True) for _ in range(3)]
     xs = [g.field() for _ in range(3)]
     m3 = sem.CG.solve3(cgs, xs, fd, d, dmask, h1d, h2d, ifh2, abstol=1e-8, max_iter=800)
     for c in range(3):
+        _check_way(cgs[c], launches, sem.CG.COUPLED)
         xg = xs[c].get()
         x_ref = o.cg(fs[c], mask, h1, h2, ifh2, abstol=1e-8, max_iter=800)[0]
         res_true = _true_residual(o, xg, fs[c], mask, h1, h2, ifh2)
