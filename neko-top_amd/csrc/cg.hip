@@ -122,6 +122,8 @@ struct CgState {
   uint32_t tag = 1;
   unsigned long long wait = kGridWait;
   bool grid_off = false;
+  // per ifh2: whether an empty device holds all its workgroups (-1: not asked)
+  int room[2] = {-1, -1};
   int path = NEKOAMD_BY_LAUNCHES;  // of the last solve
 };
 
@@ -1358,15 +1360,17 @@ static int cg_drive(CgState* s, int max_iter, int batch, F&& queue_batch) {
   return status;
 }
 
-// One launch of up to kGridCap iterations; *ran = false where the mesh does
-// not fit.
+// One launch of up to kGridCap iterations; with room: no launch, only
+// whether an empty device holds the workgroups.
 template <int LX, int EPB, bool H2>
-static int cg_grid_launch(const CgGrid& a, bool* ran) {
+static int cg_grid_launch(const CgGrid& a, int* room) {
   constexpr int BS = (LX * LX * LX * EPB + 63) / 64 * 64;
   const int wg = (a.nelv + EPB - 1) / EPB;
-  *ran = wg <= kGridWg &&
-         grid_room((const void*)cg_grid_k<LX, EPB, H2>, BS, 0) >= wg;
-  if (!*ran) return kOk;
+  if (room) {
+    *room = wg <= kGridWg &&
+            grid_room((const void*)cg_grid_k<LX, EPB, H2>, BS, 0) >= wg;
+    return kOk;
+  }
   hipLaunchKernelGGL((cg_grid_k<LX, EPB, H2>), dim3(wg), dim3(BS), 0, stream(),
                      a);
   NK_LAUNCHED();
@@ -1374,20 +1378,40 @@ static int cg_grid_launch(const CgGrid& a, bool* ran) {
 }
 
 template <int LX, int ES, int EL>
-static int cg_grid_pick(const CgGrid& a, bool h2, bool* ran) {
+static int cg_grid_pick(const CgGrid& a, bool h2, int* room) {
   if (a.nelv <= kGridWg * ES)
-    return h2 ? cg_grid_launch<LX, ES, true>(a, ran)
-              : cg_grid_launch<LX, ES, false>(a, ran);
-  return h2 ? cg_grid_launch<LX, EL, true>(a, ran)
-            : cg_grid_launch<LX, EL, false>(a, ran);
+    return h2 ? cg_grid_launch<LX, ES, true>(a, room)
+              : cg_grid_launch<LX, ES, false>(a, room);
+  return h2 ? cg_grid_launch<LX, EL, true>(a, room)
+            : cg_grid_launch<LX, EL, false>(a, room);
 }
 
-// Whether the mesh of s may be one of cg_grid_k's: at most kGridWg
-// workgroups, lx in 4..8.  The smaller orders take the fewest elements that
-// make 256 threads while that fits, else as many as 512 threads hold.
-static bool cg_grid_fits(const CgState* s, const CgOp& op) {
-  return !s->grid_off && s->nelv > 0 && op.lx >= 4 && op.lx <= 8 &&
-         s->nelv <= kGridWg * (op.lx == 4 ? 8 : op.lx == 5 ? 4 : op.lx == 6 ? 2 : 1);
+// The smaller orders take the fewest elements that make 256 threads while
+// those are at most kGridWg workgroups, else as many as 512 threads hold.
+static int cg_grid_any(int lx, const CgGrid& a, bool h2, int* room) {
+  switch (lx) {
+    case 4: return cg_grid_pick<4, 4, 8>(a, h2, room);
+    case 5: return cg_grid_pick<5, 2, 4>(a, h2, room);
+    case 6: return cg_grid_pick<6, 1, 2>(a, h2, room);
+    case 7: return cg_grid_pick<7, 1, 1>(a, h2, room);
+    default: return cg_grid_pick<8, 1, 1>(a, h2, room);
+  }
+}
+
+// Whether solves of s are cg_grid_k's: lx in 4..8, the workgroups all at once
+// on an empty device, points shared by at most 8 elements, and no wait given
+// up before.  Then a.ref and a.idx are set.
+static int cg_grid_fits(CgState* s, const CgOp& op, CgGrid& a, bool* fits) {
+  *fits = !s->grid_off && s->nelv > 0 && op.lx >= 4 && op.lx <= 8 &&
+          (int64_t)s->nelv * op.lx * op.lx * op.lx == s->n;
+  if (!*fits) return kOk;
+  int& room = s->room[op.ifh2];
+  if (room < 0) {
+    a.nelv = s->nelv;
+    if (const int rc = cg_grid_any(op.lx, a, op.ifh2, &room)) return rc;
+  }
+  *fits = room != 0;
+  return *fits ? gs_point_refs(op.gs, 8, &a.ref, &a.idx, fits) : kOk;
 }
 
 // The FP64 iteration vectors of a mixed state.
@@ -1397,19 +1421,15 @@ static int grid_vectors(CgState* s) {
   return kOk;
 }
 
-// The started solve of s by cg_grid_k; *ran = false if points are shared by
-// more than 8 elements, if the device has no room for all its workgroups, or
-// if it got stuck (another process holding the device): the caller then
-// starts the solve over with the launches.  A mixed state's solve ends, as
-// its launches' do, on the true residual f - A x only: it is recomputed
-// whenever the iterated one meets the tolerance.
-static int cg_grid(CgState* s, const CgOp& op, double* x, const double* mult,
-                   const double* f, bool* ran) {
+// The started solve of s by cg_grid_k (cg_grid_fits); *ran = false if it got
+// stuck (another process holding the device): the caller then starts the
+// solve over with the launches.  A mixed state's solve ends, as its launches'
+// do, on the true residual f - A x only: it is recomputed whenever the
+// iterated one meets the tolerance.
+static int cg_grid(CgState* s, const CgOp& op, CgGrid& a, double* x,
+                   const double* mult, const double* f, bool* ran) {
   *ran = false;
-  CgGrid a{};
-  bool ok = false;
-  int rc = gs_point_refs(op.gs, 8, &a.ref, &a.idx, &ok);
-  if (rc || !ok) return rc;
+  int rc = kOk;
   if (!s->slots) {
     const size_t bytes = sizeof(uint64_t) * (6 * kGridWg + 2 * (size_t)s->n);
     NK_HIP(hipMalloc((void**)&s->slots, bytes));
@@ -1438,14 +1458,8 @@ static int cg_grid(CgState* s, const CgOp& op, double* x, const double* mult,
   for (;;) {
     a.tag = s->tag;
     s->tag += 2 * kGridCap;
-    switch (op.lx) {
-      case 4: rc = cg_grid_pick<4, 4, 8>(a, op.ifh2, ran); break;
-      case 5: rc = cg_grid_pick<5, 2, 4>(a, op.ifh2, ran); break;
-      case 6: rc = cg_grid_pick<6, 1, 2>(a, op.ifh2, ran); break;
-      case 7: rc = cg_grid_pick<7, 1, 1>(a, op.ifh2, ran); break;
-      default: rc = cg_grid_pick<8, 1, 1>(a, op.ifh2, ran);
-    }
-    if (rc || !*ran) return rc;
+    rc = cg_grid_any(op.lx, a, op.ifh2, nullptr);
+    if (rc) return rc;
     if (s->prec == NEKOAMD_CG_MIXED) {
       rc = ax_helm_launch<double, double>(s->w, x, op.dx, op.h1, op.h2, op.g11,
                                           op.g12, op.g13, op.g22, op.g23,
@@ -1465,10 +1479,10 @@ static int cg_grid(CgState* s, const CgOp& op, double* x, const double* mult,
     NK_HIP(hipStreamSynchronize(stream()));
     if (s->host[0].stuck) {
       s->grid_off = true;
-      *ran = false;
       return kOk;
     }
-    if (s->host[0].done) return kOk;
+    *ran = s->host[0].done != 0;
+    if (*ran) return kOk;
   }
 }
 
@@ -1778,14 +1792,16 @@ int nekoamd_cg_solve(void* cg, void* x, const void* f, const void* d,
     NK_LAUNCHED();
     return kOk;
   };
-  const bool small = cg_grid_fits(s, op);
+  CgGrid grid{};
+  bool small = false;
+  if ((status = cg_grid_fits(s, op, grid, &small))) return status;
   if (small) {
     // a small mesh: both precisions in FP64 (nothing is bound by the bytes
     // that FP32 vectors save)
     if ((status = grid_vectors(s))) return status;
     if ((status = start64())) return status;
     bool ran = false;
-    if ((status = cg_grid(s, op, (double*)x, (const double*)mult, F, &ran)))
+    if ((status = cg_grid(s, op, grid, (double*)x, (const double*)mult, F, &ran)))
       return status;
     if (ran) {
       fill_monitor(s->host[0], mon);
@@ -1860,12 +1876,14 @@ int nekoamd_cg_solve3(void* const* cg, void* const* x, const void* const* f,
   NK_REQUIRE(lx && volume && abstol && max_iter && poll && nmask && ifh2,
              "null argument");
   // FP64 states, an element size without the three-direction kernel, or a
-  // mesh small enough for one kernel a solve: three solves one after the
-  // other
+  // mesh whose solves are one kernel each: three solves one after the other
   const CgOp shape{gs, nullptr, 0, nullptr, nullptr, nullptr, nullptr, nullptr,
                    nullptr, nullptr, nullptr, nullptr, nullptr, *lx, *ifh2 != 0};
-  const bool small = cg_grid_fits(s[0], shape) && cg_grid_fits(s[1], shape) &&
-                     cg_grid_fits(s[2], shape);
+  bool small = true;
+  for (int c = 0; c < 3 && small; ++c) {
+    CgGrid grid{};
+    if (const int rc = cg_grid_fits(s[c], shape, grid, &small)) return rc;
+  }
   if (s[0]->prec != NEKOAMD_CG_MIXED || *lx < 4 || *lx > 10 || small) {
     for (int c = 0; c < 3; ++c) {
       const int rc = nekoamd_cg_solve(

@@ -624,3 +624,55 @@ def test_cg_small_mesh_with_waits_given_up(box, mixed, wait, sem):
         # FP32 iterations need more of them
         assert abs(mon.iter - it) <= (1 if not mixed or cg.path == cg.ONE_KERNEL else it + 20)
         assert np.abs(x.get() - ref).max() <= 1e-5 * np.abs(ref).max()
+
+
+def _other_map(sem, box, gid):
+    """The case of a box with another numbering."""
+    g = sem.BoxCase(*box, jitter=0.05, seed=1234)
+    o = oracle.build_case(*box, jitter=0.05, seed=1234)
+    o.gid = gid(o.gid.copy())
+    o.gs_idx, o.gs_m, o.gs_cnt = oracle.gs_build(o.gid)
+    o.mult = 1.0 / o.gs(np.ones(o.n))
+    g.gs = sem.GatherScatter(o.gid)
+    g.mult = g.field(o.mult)
+    return g, o
+
+
+def _solve3(sem, g, o, mixed):
+    rng = np.random.default_rng(17)
+    faces = sem.VEL_DIRICHLET
+    mask = oracle.face_mask(g.nx, g.ny, g.nz, g.lx, faces)
+    h1, h2 = np.full(g.n, 0.01), np.full(g.n, 1500.0)
+    fs = []
+    for _ in range(3):
+        f = o.gs(o.B * rng.uniform(-1, 1, g.n))
+        f[mask] = 0.0
+        fs.append(f)
+    d, h1d, h2d = g.field(), g.field(h1), g.field(h2)
+    g.jacobi(d, h1d, h2d, True)
+    cgs = [sem.CG(g, mixed=mixed) for _ in range(3)]
+    xs = [g.field() for _ in range(3)]
+    for _ in range(2):
+        mons = sem.CG.solve3(cgs, xs, [g.field(f) for f in fs], d, g.mask(faces), h1d, h2d, True,
+                             abstol=1e-8, max_iter=800)
+    for c in range(3):
+        ref = o.cg(fs[c], mask, h1, h2, True, abstol=1e-8, max_iter=800)[0]
+        assert mons[c].done == 1 and mons[c].res_final < 1e-8
+        assert rel_max(xs[c].get(), ref) < 1e-6
+    return [cg.path for cg in cgs]
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+def test_cg_small_mesh_with_shared_points_beyond_the_kernel(mixed, sem):
+    """A point of 16 elements (two vertices made one), more than the one
+    kernel gathers: the launches of a larger mesh, and the coupled solve in
+    mixed precision, against the oracle on the same map."""
+    def merge(gid):
+        u, c = np.unique(gid, return_counts=True)
+        v = u[c == 8]
+        gid[gid == v[-1]] = v[0]
+        return gid
+    g, o = _other_map(sem, (5, 4, 4, 4), merge)
+    assert o.gs_m.max() == 16
+    way = sem.CG.COUPLED if mixed else sem.CG.BY_LAUNCHES
+    assert _solve3(sem, g, o, mixed) == [way] * 3
