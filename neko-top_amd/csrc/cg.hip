@@ -1411,7 +1411,7 @@ static int cg_grid_fits(CgState* s, const CgOp& op, CgGrid& a, bool* fits) {
     if (const int rc = cg_grid_any(op.lx, a, op.ifh2, &room)) return rc;
   }
   *fits = room != 0;
-  return *fits ? gs_point_refs(op.gs, 8, &a.ref, &a.idx, fits) : kOk;
+  return *fits ? gs_point_refs(op.gs, s->n, 8, &a.ref, &a.idx, fits) : kOk;
 }
 
 // The FP64 iteration vectors of a mixed state.

@@ -501,11 +501,11 @@ __global__ void __launch_bounds__(256)
     ref[idx[off + k]] = make_int2((int)(off + k / m * m), m);
 }
 
-int gs_point_refs(void* gs, int maxm, const int2** ref, const int32_t** idx,
-                  bool* ok) {
+int gs_point_refs(void* gs, int64_t n, int maxm, const int2** ref,
+                  const int32_t** idx, bool* ok) {
   GsMap* g = (GsMap*)gs;
   if (!g) return fail_arg("gs_point_refs", "null gs handle");
-  *ok = g->n > 0 && g->dev_len <= INT32_MAX;
+  *ok = g->n > 0 && g->n == n && g->dev_len <= INT32_MAX;
   for (int b = 0; b < g->nb; ++b) *ok = *ok && g->m[b] <= maxm;
   if (!*ok) return kOk;
   if (!g->ref) {

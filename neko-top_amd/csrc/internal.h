@@ -182,10 +182,11 @@ int grid_room(const void* kernel, int threads, size_t lds);
 
 // The gs map seen from its points: (*ref)[l] = {offset into *idx of the tuple
 // point l is in, its multiplicity}, {0, 0} for a point in none.  Made on the
-// first call and kept with the map; *ok = false (and nothing made) if a
-// multiplicity exceeds maxm or an offset does not fit.
-int gs_point_refs(void* gs, int maxm, const int2** ref, const int32_t** idx,
-                  bool* ok);
+// first call and kept with the map; *ok = false (and nothing made) if the map
+// is not one of n points, a multiplicity exceeds maxm or an offset does not
+// fit.
+int gs_point_refs(void* gs, int64_t n, int maxm, const int2** ref,
+                  const int32_t** idx, bool* ok);
 
 template <typename T>
 int bc_zero_launch(T* u, const int32_t* mask, int64_t nmask, const int* skip);

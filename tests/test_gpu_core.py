@@ -626,14 +626,15 @@ def test_cg_small_mesh_with_waits_given_up(box, mixed, wait, sem):
         assert np.abs(x.get() - ref).max() <= 1e-5 * np.abs(ref).max()
 
 
-def _other_map(sem, box, gid):
-    """The case of a box with another numbering."""
+def _other_map(sem, box, gid, points=None):
+    """The case of a box with another numbering (points: the device's map
+    covers only so many of them, the others being in no other element)."""
     g = sem.BoxCase(*box, jitter=0.05, seed=1234)
     o = oracle.build_case(*box, jitter=0.05, seed=1234)
     o.gid = gid(o.gid.copy())
     o.gs_idx, o.gs_m, o.gs_cnt = oracle.gs_build(o.gid)
     o.mult = 1.0 / o.gs(np.ones(o.n))
-    g.gs = sem.GatherScatter(o.gid)
+    g.gs = sem.GatherScatter(o.gid[:points])
     g.mult = g.field(o.mult)
     return g, o
 
@@ -676,3 +677,13 @@ def test_cg_small_mesh_with_shared_points_beyond_the_kernel(mixed, sem):
     assert o.gs_m.max() == 16
     way = sem.CG.COUPLED if mixed else sem.CG.BY_LAUNCHES
     assert _solve3(sem, g, o, mixed) == [way] * 3
+
+
+def test_cg_small_mesh_with_a_map_of_fewer_points(sem):
+    """A map over the first two of three elements (the third shares nothing):
+    the launches, against the oracle with the same connections."""
+    def apart(gid):
+        gid[128:] = gid.max() + 1 + np.arange(64)
+        return gid
+    g, o = _other_map(sem, (3, 1, 1, 4), apart, points=128)
+    assert _solve3(sem, g, o, False) == [sem.CG.BY_LAUNCHES] * 3
