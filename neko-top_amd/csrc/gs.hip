@@ -29,6 +29,7 @@
 // for the tuples in id order (the measured figure) and 1.61x for this layout.
 #include <algorithm>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "internal.h"
@@ -508,18 +509,26 @@ int gs_point_refs(void* gs, int64_t n, int maxm, const int2** ref,
   *ok = g->n > 0 && g->n == n && g->dev_len <= INT32_MAX;
   for (int b = 0; b < g->nb; ++b) *ok = *ok && g->m[b] <= maxm;
   if (!*ok) return kOk;
+  // solves of one mesh on several host threads share the map; the table is
+  // given to a solve once the kernels that fill it are queued before it
+  static std::mutex making;
+  std::lock_guard<std::mutex> lock(making);
   if (!g->ref) {
     int2* r = nullptr;
     NK_HIP(hipMalloc((void**)&r, sizeof(int2) * g->n));
-    g->ref = r;
-    NK_HIP(hipMemsetAsync(r, 0, sizeof(int2) * g->n, stream()));
-    for (int b = 0; b < g->nb; ++b) {
+    hipError_t e = hipMemsetAsync(r, 0, sizeof(int2) * g->n, stream());
+    for (int b = 0; b < g->nb && e == hipSuccess; ++b) {
       const int64_t nocc = g->cnt[b] * g->m[b];
       if (nocc == 0) continue;
       hipLaunchKernelGGL(gs_ref_k, dim3(nk_grid(nocc, 256)), dim3(256), 0,
                          stream(), nocc, g->m[b], g->dev_off[b], g->idx_d, r);
-      NK_LAUNCHED();
+      e = hipGetLastError();
     }
+    if (e != hipSuccess) {
+      (void)hipFree(r);
+      return fail_hip(__func__, e);
+    }
+    g->ref = r;
   }
   *ref = g->ref;
   *idx = g->idx_d;

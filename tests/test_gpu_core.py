@@ -687,3 +687,47 @@ def test_cg_small_mesh_with_a_map_of_fewer_points(sem):
         return gid
     g, o = _other_map(sem, (3, 1, 1, 4), apart, points=128)
     assert _solve3(sem, g, o, False) == [sem.CG.BY_LAUNCHES] * 3
+
+
+def test_cg_small_mesh_on_several_threads(sem):
+    """First solves on a new mesh from four host threads at once, each with
+    its own state and fields and one gather-scatter map: the solution of a
+    solve alone, bit for bit."""
+    import threading
+    box = (8, 8, 4, 8)
+    o = oracle.build_case(*box, jitter=0.05, seed=1234)
+    mask = oracle.face_mask(*box, sem.PRS_DIRICHLET)
+    rng = np.random.default_rng(3)
+    fs = [o.gs(o.B * rng.uniform(-1, 1, o.n)) for _ in range(4)]
+    for f in fs:
+        f[mask] = 0.0
+
+    def case():
+        g = sem.BoxCase(*box, jitter=0.05, seed=1234)
+        h1, d = g.field(np.ones(g.n)), g.field()
+        g.jacobi(d, h1)
+        return g, (d, g.mask(sem.PRS_DIRICHLET), h1), [
+            (sem.CG(g), g.field(), g.field(f)) for f in fs]
+
+    def solve(job, args):
+        cg, x, f = job
+        cg.solve(x, f, *args, abstol=1e-8, max_iter=3000)
+
+    g, args, jobs = case()
+    for job in jobs:
+        solve(job, args)
+    want = [x.get() for _, x, _ in jobs]
+    g2, args2, jobs2 = case()
+    start = threading.Barrier(4)
+
+    def run(job):
+        start.wait()
+        solve(job, args2)
+
+    threads = [threading.Thread(target=run, args=(job,)) for job in jobs2]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for (cg, x, _), w in zip(jobs2, want):
+        assert cg.path == cg.ONE_KERNEL and np.array_equal(x.get(), w)
