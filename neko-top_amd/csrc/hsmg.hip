@@ -1455,10 +1455,12 @@ int crs_grid_wgs(const Hsmg* h) { return (int)((h->nl + kCB - 1) / kCB); }
 // 256 workgroups (131072 vertices), which are also the block partials of the
 // other form, and an empty device must hold them all at once.  They find room
 // beside the Schwarz kernels of the library stream as those' workgroups
-// retire.
+// retire.  Two iterations at least: a caller's captured application replays
+// with the tags of its capture, and only then does no word hold the tag that
+// a replay waits for first, from the replay before.
 int crs_grid_halo(const Hsmg* h) {
   const int64_t halo = (int64_t)(h->nx + 1) * (h->ny + 1) + h->nx + 2;
-  const bool fits = !h->graphs &&
+  const bool fits = !h->graphs && h->crs_iter >= 2 &&
                     (kCB + 2 * halo) * (int64_t)sizeof(double) <= 60 * 1024 &&
                     h->nl <= 256 * (int64_t)kCB &&
                     grid_room((const void*)crs_grid_k, kCB,

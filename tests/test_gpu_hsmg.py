@@ -213,3 +213,44 @@ def test_coarse_kernel_with_waits_given_up(box, monkeypatch):
         M.apply(z, r)
     device.sync()
     assert all(close(z, w) for z, w in zip(zs, want))
+
+
+@pytest.mark.parametrize("crs_iter", [1, 2, 10])
+def test_captured_application_replays(crs_iter):
+    """An application captured from the library stream by the caller: every
+    replay, with eager applications between them, equals the eager result bit
+    for bit.  One coarse iteration takes the launches."""
+    import ctypes as C
+    from nekoamd import device, sem
+    from nekoamd._lib import lib
+    device.init(0)
+    hip = C.CDLL("libamdhip64.so")
+
+    def ok(rc):
+        assert rc == 0, rc
+    stream = C.c_void_p(lib().nekoamd_stream())
+    g = sem.BoxCase(16, 8, 8, 4, jitter=0.05, seed=1234)
+    M = sem.HSMG(g, crs_iter=crs_iter)
+    rng = np.random.default_rng(8)
+    r, z, zg = g.field(), g.field(), g.field()
+    other = g.field(rng.standard_normal(g.n))
+    M.apply(z, r)  # the side stream is made on the first application
+    assert M.path == (M.ONE_KERNEL if crs_iter > 1 else M.BY_LAUNCHES)
+    graph, run = C.c_void_p(), C.c_void_p()
+    ok(hip.hipStreamBeginCapture(stream, 2))  # relaxed
+    M.apply(zg, r)
+    ok(hip.hipStreamEndCapture(stream, C.byref(graph)))
+    ok(hip.hipGraphInstantiate(C.byref(run), graph, None, None, 0))
+    for k in range(5):
+        v = g.field(rng.standard_normal(g.n))
+        g.gs.op(v)
+        r.copy_from(v)
+        ok(hip.hipGraphLaunch(run, stream))
+        device.sync()
+        got = zg.get()
+        if k % 2:
+            M.apply(z, other)
+        M.apply(z, r)
+        assert np.array_equal(got, z.get()) and got.any()
+    ok(hip.hipGraphExecDestroy(run))
+    ok(hip.hipGraphDestroy(graph))
