@@ -122,7 +122,7 @@ __device__ __forceinline__ TA ax_point_sk(TA u, const AxPoint<TA>& a,
 }
 
 // Sum of v over the workgroup of NP = LX^3 threads; valid on thread 0.
-// sd: NP doubles of LDS.  A fixed order: wavefront butterflies, then the
+// sd: NP doubles of LDS.  A fixed order: wavefront sums, then the
 // wavefront sums in order when NP is a multiple of 64; else a serial sum.
 template <int NP>
 __device__ __forceinline__ double element_sum(double v, double* sd) {

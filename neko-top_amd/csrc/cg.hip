@@ -547,7 +547,7 @@ __global__ void __launch_bounds__(kRedBlock)
   __shared__ double s_alpha;
   if (sc->halt) return;
   if (threadIdx.x < 64) {
-    // kPapParts == 64: one value per lane, the same butterfly in every block
+    // kPapParts == 64: one value per lane, the same tree in every block
     const double pap = wave_sum(part_pap[threadIdx.x]);
     if (threadIdx.x == 0) {
       const double al = sc->rtz1 / pap;
@@ -661,7 +661,7 @@ __global__ void __launch_bounds__(kRedBlock)
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       if (!act[c]) continue;
-      // kPapParts == 64: one value per lane, the same butterfly in every block
+      // kPapParts == 64: one value per lane, the same tree in every block
       const double pap = wave_sum(v.part_pap[c][threadIdx.x]);
       if (threadIdx.x == 0) {
         const double al = v.sc[c]->rtz1 / pap;
@@ -848,10 +848,10 @@ __global__ void __launch_bounds__(kFinBlock)
 // Bound by the two exchanges, about 2 us each (a store and a load past the
 // L2s); the five launches it replaces take 17 us however small the mesh is.
 // FP64 pressure solve, us per solve by launches -> here: 8x4x4 order 5
-// (336 iterations) 6170 -> 2380, 8x8x4 order 7 12550 -> 6290, 12x10x8 order
-// 3 6330 -> 3470, 10x8x6 order 5 10240 -> 5260; solves of mixed states
-// likewise (10x8x6 order 5 11670 -> 5460, three velocity components on 8x8x4
-// order 7 583 -> 389).
+// (336 iterations) 5610 -> 2430, 8x8x4 order 7 9990 -> 6100, 12x10x8 order
+// 3 5570 -> 3440, 10x8x6 order 5 9430 -> 5380; solves of mixed states
+// likewise (10x8x6 order 5 12770 -> 5400, three velocity components on 8x8x4
+// order 7 649 coupled -> 385).
 //
 // Up to kGridWg workgroups, one per CU.  Two per CU lose: the registers then
 // spill and a reader has twice the slots to wait for (10x8x6 order 7, 480

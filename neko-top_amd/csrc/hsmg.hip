@@ -103,8 +103,8 @@ struct Hsmg {
   unsigned long long wait = kGridWait;
   int* took_over = nullptr;
   bool by_launches = true;
-  // the coarse solve (fixed kernels on fixed buffers), recorded as a graph on
-  // the first application and replayed (NEKOAMD_HIP_GRAPHS=1)
+  // the coarse solve's launches (fixed kernels on fixed buffers), recorded as
+  // a graph on the first application and replayed (NEKOAMD_HIP_GRAPHS=1)
   hipGraphExec_t crs_graph = nullptr;
   // the graph runs on a side stream (default priority), overlapping the
   // fine and mid Schwarz steps: r1 ready -> ev_r1; coarse done -> ev_crs
@@ -1270,8 +1270,9 @@ struct CrsGrid {
 // form's (two of its blocks' partials per workgroup), so the result is the
 // same bit for bit.  Bound by the exchanges, 2 us each, where a launch of the
 // kernel-by-kernel form takes about 5, 21 of them.  GMRES + HSMG solves by
-// launches -> here: 8x4x4 order 5 3300 -> 2190 us, 16x8x8 order 7 5850 ->
-// 4060, 16x16x16 order 7 8820 -> 6830, 32x16x16 order 7 21800 -> 19200.
+// launches -> here (one box, in turn): 8x4x4 order 5 3550 -> 1970 us, 16x8x8
+// order 7 5410 -> 3710, 16x16x16 order 7 8500 -> 6680, 32x16x16 order 7
+// 20600 -> 18700.
 constexpr int kCB = 2 * kHB;
 
 // The sum of the four waves from wave wv as that block's partial (nblk

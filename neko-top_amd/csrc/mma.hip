@@ -96,8 +96,12 @@ struct MmaOut {
 // value v, else sum.  Every block stores its partials past its L2 (device
 // scope) and waits for those stores before it counts itself done; the last
 // one to do so sums them all, in an order that does not depend on which
-// block that is, and writes the results to the host's memory.  (A fence in
-// their place writes back the whole L2 in every block: 75 us more a pass.)
+// block that is, and writes the results to the host's memory.  That the
+// relaxed count cannot be seen before the partials rests on gfx950, not on
+// the memory model: a device-scope store has reached memory that all XCDs see
+// when vmcnt counts it done, and the barrier keeps thread 0's count behind
+// every storing thread's wait.  (A release fence, which the model asks for,
+// writes back the whole L2 in every block: 75 us more a pass.)
 template <int K>
 __device__ __forceinline__ void grid_out(double (&acc)[K], unsigned ismax,
                                          const MmaOut& o) {
