@@ -859,6 +859,10 @@ __global__ void __launch_bounds__(kFinBlock)
 // workgroups of two elements: 16300 against 15300).
 constexpr int kGridWg = 256;    // most workgroups of cg_grid_k
 constexpr int kGridCap = 2048;  // iterations of one launch
+// words of the sums' slots, the one nobody fills too, in whole pages: an
+// element's words of w then share no line with another's where it fills them
+constexpr int kGridSlots = 2048;
+static_assert(6 * (kGridWg + 1) <= kGridSlots, "slots");
 
 struct CgGrid {
   double *x, *r, *p;
@@ -890,7 +894,7 @@ __global__ void __launch_bounds__((LX * LX * LX * EPB + 63) / 64 * 64)
   __shared__ int fail;
   CgScal* sc = a.sc;
   if (sc->halt) return;  // the same in every workgroup: set before the launch
-  const int tid = threadIdx.x, nwg = gridDim.x;
+  const int tid = threadIdx.x, nwg = gridDim.x + (a.wait == 0);
   const int el = tid / NP, t = tid % NP, o = el * NP;
   const int e = blockIdx.x * EPB + el;
   const bool live = tid < NB && e < a.nelv;
@@ -1431,14 +1435,14 @@ static int cg_grid(CgState* s, const CgOp& op, CgGrid& a, double* x,
   *ran = false;
   int rc = kOk;
   if (!s->slots) {
-    const size_t bytes = sizeof(uint64_t) * (6 * kGridWg + 2 * (size_t)s->n);
+    const size_t bytes = sizeof(uint64_t) * (kGridSlots + 2 * (size_t)s->n);
     NK_HIP(hipMalloc((void**)&s->slots, bytes));
     NK_HIP(hipMemsetAsync(s->slots, 0, bytes, stream()));
   }
   a.x = x;
   a.r = s->r;
   a.p = s->p;
-  a.w = s->slots + 6 * kGridWg;
+  a.w = s->slots + kGridSlots;
   a.dm = s->dm;
   a.mult = mult;
   a.dx = op.dx;

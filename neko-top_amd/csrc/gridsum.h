@@ -16,8 +16,10 @@
 //
 // All workgroups must be resident at once: the launcher bounds the grid by
 // the occupancy of an empty device.  A wait lasts at most `wait` ticks of the
-// 100 MHz clock (0: it is given up before the words are looked at); a
-// workgroup that gives up leaves, and so the others do.
+// 100 MHz clock; a workgroup that gives up leaves, and so the others do.  To
+// have the first wait given up at once, the launcher passes wait 0 and has
+// the sums take one slot more than there are workgroups, which nobody fills
+// (a test of the wait in the loop that polls costs 4 % of a small solve).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -57,7 +59,7 @@ __device__ __forceinline__ void grid_get(const uint64_t* const (&s)[N], int n,
   const unsigned long long t0 = wall_clock64();
   for (;;) {
     uint64_t w[2 * N];
-    bool here = wait != 0;
+    bool here = true;
 #pragma unroll
     for (int j = 0; j < N; ++j)
       if (j < n) {

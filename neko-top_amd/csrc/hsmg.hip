@@ -1293,14 +1293,17 @@ __global__ void __launch_bounds__(kCB) crs_grid_k(CrsGrid g) {
   __shared__ int fail;
   const int tid = threadIdx.x, wv = tid >> 6;
   // no wait after one that an earlier application gave up
-  const unsigned long long wait =
-      __builtin_amdgcn_readfirstlane(*g.stuck) != 0 ? 0 : g.wait;
+  const bool off =
+      __builtin_amdgcn_readfirstlane(*g.stuck) != 0 || g.wait == 0;
+  const unsigned long long wait = off ? 0 : g.wait;
   const int nxl = g.nx + 1, nyl = g.ny + 1, nxy = nxl * nyl;
   const int nl = nxy * (g.nz + 1);
   const int v0 = blockIdx.x * kCB, v = v0 + tid;
   const bool live = v < nl;
   const int a = v % nxl, b = (v / nxl) % nyl, c = v / nxy;
   const int range = kCB + 2 * g.halo, nblk = (nl + kHB - 1) / kHB;
+  // slot_r's slot nblk is slot_p's first, which holds no tag of slot_r
+  const int nslots = nblk + off;
   if (tid == 0) fail = 0;
   for (int i = tid; i < range; i += kCB) p[i] = 0.0;
   double S[27], x = 0.0, r = 0.0, d = 0.0;
@@ -1333,7 +1336,7 @@ __global__ void __launch_bounds__(kCB) crs_grid_k(CrsGrid g) {
     __syncthreads();
     if ((tid & (kHB - 1)) == 0) crs_publish(slot_r, tag, s1, wv, nblk);
     prev = rz[0];
-    if (!(ok = (grid_sum<1, kHB>(slot_r, nblk, tag, wait, s2, &fail, rz))))
+    if (!(ok = (grid_sum<1, kHB>(slot_r, nslots, tag, wait, s2, &fail, rz))))
       break;
     const double beta = q > 0 && prev != 0.0 ? rz[0] / prev : 0.0;
     // p on the halo from the other workgroups' z, on the own range from z
@@ -1363,7 +1366,7 @@ __global__ void __launch_bounds__(kCB) crs_grid_k(CrsGrid g) {
     __syncthreads();
     if ((tid & (kHB - 1)) == 0) crs_publish(slot_p, tag + 1u, s3, wv, nblk);
     // past this every workgroup has read z, so the next may overwrite it
-    if (!(ok = (grid_sum<1, kHB>(slot_p, nblk, tag + 1u, wait, s4, &fail, pap))))
+    if (!(ok = (grid_sum<1, kHB>(slot_p, nslots, tag + 1u, wait, s4, &fail, pap))))
       break;
     const double alpha = pap[0] != 0.0 ? rz[0] / pap[0] : 0.0;
     x += alpha * pv;
