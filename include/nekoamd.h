@@ -318,8 +318,9 @@ int nekoamd_cg_path(void* cg, int* path);
  * (nekoamd_jacobi_update).  f must be continuous (gs-assembled) and zero on
  * the mask, as the reference's callers guarantee (adjoint_pnpn.f90:725-726).
  * Blocks until the solve is done; fills mon.  Small meshes (lx in [4, 8], up
- * to 256 workgroups of one to eight elements) are solved in FP64 whatever the
- * state's precision; a mixed state's solve still ends on the recomputed
+ * to 256 workgroups of one to eight elements that the device holds at once, a
+ * gs map of the n points with at most 8 elements to a point) are solved by
+ * one kernel in FP64 whatever the state's precision; a mixed state's solve still ends on the recomputed
  * residual f - A x only. */
 int nekoamd_cg_solve(void* cg, void* x, const void* f, const void* d,
                      const void* mult, const double* volume,

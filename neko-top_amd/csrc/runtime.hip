@@ -38,8 +38,10 @@ int grid_room(const void* kernel, int threads, size_t lds) {
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
                             dev) != hipSuccess ||
       hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads,
-                                                   lds) != hipSuccess)
+                                                   lds) != hipSuccess) {
+    (void)hipGetLastError();  // not the next launch's
     return 0;
+  }
   return cus * per;
 }
 LaunchRecorder*& launch_recorder() {
